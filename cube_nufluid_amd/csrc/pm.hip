@@ -329,19 +329,6 @@ __device__ __forceinline__ int cell_of(const int64_t* cs, int64_t p) {
   return lo;
 }
 
-// maximum over the wavefront of non-negative floats as their bit patterns
-// (which order as the floats do), by DPP: pairs and quads, half rows, rows,
-// then rows 0-1 into row 1 and rows 0-3 into row 3; lane 63 holds it
-__device__ __forceinline__ uint32_t wave_max_bits(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false));   // quad_perm 2,3,0,1
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));  // row_half_mirror
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));  // row_mirror
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // block reduction of NV non-negative float maxima into slot fields
 // f0..f0+NV-1
 template <int NV, int W>

@@ -211,7 +211,6 @@ __global__ __launch_bounds__(PP_NT) void k_pp(Geo g, const void* __restrict__ xp
 // PB = 4 serves pp_range <= 2, PB = 2 pp_range 3..4 (window <= 20 cells).
 #define PD_NT 256
 #define PP_SLOTS 1024
-#define PF_OWN 4096  // region particles covered by the LDS owner table
 struct PPent { float x, y, z; int32_t p; };
 
 struct PPctx {  // per-call constants
@@ -220,6 +219,7 @@ struct PPctx {  // per-call constants
   const double* vdt;  // decoded velocities for c_old
   const double* venc;
   int32_t kmax, pr;
+  int32_t whole;      // pairs whose 2^-32 units sum exactly in a double
 };
 
 template <int PB>
@@ -273,21 +273,14 @@ __device__ __forceinline__ void pf_region(const Geo& g, const int64_t* cstart, i
 
 // window cell of region particle t (false if outside the window) and its
 // block-local fine coordinates (exact in FP32: at most 20 significant bits)
-// region cell of region particle t: from the owner table when given, else
-// by binary search of the offsets
 template <int PB>
 __device__ __forceinline__ bool pf_cand(const Geo& g, const void* xp, const int64_t* beg, const int32_t* off, int32_t t, int pr,
-                                        int W, int& wi, PPent& e, const uint8_t* owner = nullptr) {
+                                        int W, int& wi, PPent& e) {
   using G = PBgeo<PB>;
-  int a = 0;
-  if (owner) {
-    a = owner[t];
-  } else {
-    int b = G::NCELL;
-    while (b - a > 1) {
-      const int m = (a + b) >> 1;
-      if (off[m] <= t) a = m; else b = m;
-    }
+  int a = 0, b = G::NCELL;  // region cell: the last one starting at or before t
+  while (b - a > 1) {
+    const int m = (a + b) >> 1;
+    if (off[m] <= t) a = m; else b = m;
   }
   const int64_t p = beg[a] + (t - off[a]);
   const int rel[3] = {a % G::SPAN - 1, (a / G::SPAN) % G::SPAN - 1, a / (G::SPAN * G::SPAN) - 1};
@@ -332,6 +325,7 @@ template <>
 struct PPacc<float> {
   long long a[3] = {0, 0, 0};
   __device__ __forceinline__ void add(int e, float v) { a[e] += llrint((double)v * PP_FIX); }
+  __device__ __forceinline__ void add_whole(int e, double v) { a[e] += (long long)v; }
   __device__ __forceinline__ double get(int e) const { return (double)a[e] * (1.0 / PP_FIX); }
 };
 // FP32 pairs summed in double in a fixed candidate order (runs sorted by
@@ -391,58 +385,44 @@ __device__ __forceinline__ double pf_pair_sel(double dx, double dy, double dz, d
   return pf_pair(dx, dy, dz, mass, rsoft, rsoft2, sc) ? sc : 0.0;
 }
 
-// run-start tables: int32 entries (dense pool), or two 16-bit entries per
-// word in LDS (the binned kernel: values never exceed its candidate cap)
+// the pair term of pf_pair_sel with fewer operations: powers of R = r instead
+// of r/16, the powers of two folded into the constants (exactly), and the r > rsoft test against two FP32 bounds
+// around rsoft^2 (lo, hi; 1e-6 apart from it) with the exact test between
+// them, so both forms give the same bits
+struct PFsoft { float rsoft, lo, hi; };
+__device__ __forceinline__ float pf_pair_fast(float dx, float dy, float dz, float mass, const PFsoft& q) {
+  const float r2 = pf_r2(dx, dy, dz);
+  bool ok = r2 > q.hi;
+  if (!ok && r2 >= q.lo) {
+    const double e2 = (double)dx * (double)dx + (double)dy * (double)dy + (double)dz * (double)dz;
+    ok = sqrt(e2) > (double)q.rsoft;
+  }
+  const float r2c = ok ? r2 : 1.0f;
+  const float ri = __builtin_amdgcn_rsqf(r2c);
+  const float R = r2c * ri, R2 = R * R;
+  const float pc = fmaf(R2 * R, fmaf(0.75f / 1048576.0f, R2, -1.75f / 4096.0f), 1.0f);
+  const float sc = mass * pc * (ri * ri * ri);
+  return ok ? sc : 0.0f;
+}
+
+// run-start table of a dense block
 struct RunI32 {
   const int32_t* p;
   __device__ __forceinline__ int get(int i) const { return p[i]; }
 };
-struct RunU16 {
-  uint32_t* w;
-  __device__ __forceinline__ int get(int i) const { return (int)((w[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu); }
-  // add one to entry i, returning its previous value
-  __device__ __forceinline__ int inc(int i) const {
-    return (int)((atomicAdd(&w[i >> 1], 1u << ((i & 1) * 16)) >> ((i & 1) * 16)) & 0xFFFFu);
-  }
-};
 __host__ __device__ constexpr int pf_wc16_bytes(int W3) { return ((W3 + 3) / 2 * 4 + 15) / 16 * 16; }
 
-// exclusive scan of the 16-bit counts at entries 1..n of t in place, entry
-// n+1 = total; each thread owns whole words, so no two threads write one
-template <int NT>
-__device__ void pf_scan16(RunU16 t, int n, int32_t* wsum) {
-  const int nw = (n + 3) / 2;  // words covering entries 0..n+1
-  const int per = (nw + NT - 1) / NT;
-  const int w0 = min(nw, (int)threadIdx.x * per), w1 = min(nw, w0 + per);
-  int32_t s = 0;
-  for (int w = w0; w < w1; w++)
-    for (int h = 0; h < 2; h++) {
-      const int e = 2 * w + h;
-      if (e >= 1 && e <= n) s += t.get(e);
-    }
-  int32_t run = block_incl_scan<NT>(s, wsum) - s;
-  for (int w = w0; w < w1; w++) {
-    uint32_t word = t.w[w];
-    for (int h = 0; h < 2; h++) {
-      const int e = 2 * w + h;
-      if (e >= 1 && e <= n + 1) {
-        const uint32_t c = (word >> (16 * h)) & 0xFFFFu;
-        word = (word & ~(0xFFFFu << (16 * h))) | ((uint32_t)run << (16 * h));
-        if (e <= n) run += (int32_t)c;
-      }
-    }
-    t.w[w] = word;
-  }
-  __syncthreads();
-}
-
-// force on one target from the candidate runs (start[] exclusive offsets);
-// candidate coordinates are exact in FP32, so RT only sets the pair
-// arithmetic.  ROWSUM: candidates are in a fixed order, so each x-run is
-// summed in RT and added to the accumulator once per run.
-template <typename RT, bool ROWSUM, typename Acc, typename EntT, typename RunT>
+// force on one target from the candidate runs of a dense block (start[]
+// exclusive offsets); candidate coordinates are exact in FP32, so RT only
+// sets the pair arithmetic.  The candidates of a run are in no fixed order,
+// so every pair is rounded to 2^-32 units before it is added.
+//   FP32: a run of up to `whole` pairs sums its units as whole numbers in a
+// double, which is exact while the sum stays below 2^53 (no pair exceeds
+// mass/rsoft^2), and joins the 64-bit integer once: the pair's rounding and
+// add take 12 VALU operations instead of 33.  Longer runs add integers.
+template <typename RT, typename EntT, typename RunT>
 __device__ __forceinline__ void pf_force(const EntT* ent, const RunT start, int W, int pr, const PPent& ti, float mass_f,
-                                         float rsoft_f, Acc& acc, unsigned long long& npl) {
+                                         float rsoft_f, int whole, PPacc<RT>& acc, unsigned long long& npl) {
   const int wx = (int)floorf(ti.x) + pr, wy = (int)floorf(ti.y) + pr, wz = (int)floorf(ti.z) + pr;
   const RT mass = (RT)mass_f, rsoft = (RT)rsoft_f, rsoft2 = (RT)rsoft_f * (RT)rsoft_f, tx = (RT)ti.x, ty = (RT)ti.y,
            tz = (RT)ti.z;
@@ -451,31 +431,47 @@ __device__ __forceinline__ void pf_force(const EntT* ent, const RunT start, int 
       const int row = (kz * W + ky) * W;
       const int j0 = start.get(row + wx - pr), j1 = start.get(row + wx + pr + 1);
       npl += (unsigned long long)(j1 - j0);
-      RT sx = 0, sy = 0, sz = 0;
+      if constexpr (sizeof(RT) == 4) {
+        if (j1 - j0 <= whole) {
+          const PFsoft soft{rsoft_f, rsoft2 * (1.0f - 1e-6f), rsoft2 * (1.0f + 1e-6f)};
+          double u[3] = {0, 0, 0};
+          for (int j = j0; j < j1; j++) {
+            const PPent pj = ent[j];
+            const float dx = pj.x - tx, dy = pj.y - ty, dz = pj.z - tz;
+            const float sc = pf_pair_fast(dx, dy, dz, mass, soft);
+            u[0] += (double)rintf(sc * dx * (float)PP_FIX);
+            u[1] += (double)rintf(sc * dy * (float)PP_FIX);
+            u[2] += (double)rintf(sc * dz * (float)PP_FIX);
+          }
+          if (j1 > j0) {
+            acc.add_whole(0, u[0]);
+            acc.add_whole(1, u[1]);
+            acc.add_whole(2, u[2]);
+          }
+          continue;
+        }
+      }
       for (int j = j0; j < j1; j++) {
         const PPent pj = ent[j];
         const RT dx = (RT)pj.x - tx, dy = (RT)pj.y - ty, dz = (RT)pj.z - tz;
         RT sc;
-        if (ROWSUM) {
-          // branch-free: an excluded pair adds sc = 0 (a signed zero, which
-          // leaves the running sum unchanged)
-          sc = pf_pair_sel(dx, dy, dz, mass, rsoft, rsoft2);
-          sx = fma(sc, dx, sx);
-          sy = fma(sc, dy, sy);
-          sz = fma(sc, dz, sz);
-        } else {
-          if (!pf_pair(dx, dy, dz, mass, rsoft, rsoft2, sc)) continue;
-          acc.add(0, sc * dx);
-          acc.add(1, sc * dy);
-          acc.add(2, sc * dz);
-        }
-      }
-      if (ROWSUM && j1 > j0) {
-        acc.add(0, sx);
-        acc.add(1, sy);
-        acc.add(2, sz);
+        if (!pf_pair(dx, dy, dz, mass, rsoft, rsoft2, sc)) continue;
+        acc.add(0, sc * dx);
+        acc.add(1, sc * dy);
+        acc.add(2, sc * dz);
       }
     }
+}
+
+// x/b for a constant b whose reciprocal y is correctly rounded: the quotient
+// estimate corrected by its exact remainder is the correctly rounded x/b
+// (Markstein 1990) wherever the remainder does not underflow (|x| above
+// 1e-290; x = 0 gives 0).  Three operations instead of the general divide's
+// twenty.  An infinite x keeps its estimate.
+__device__ __forceinline__ double div_const(double x, double b, double y) {
+  const double q = x * y;
+  const double r = fma(fma(-q, b, x), y, q);
+  return r == r ? r : q;
 }
 
 // kick (ext_pp_force.f90:114-119) from prefetched codes, or probe write;
@@ -489,7 +485,8 @@ __device__ __forceinline__ float pf_apply(const Geo& g, const PPctx& c, void* vp
   } else {
     for (int e = 0; e < 3; e++) {
       double v = vdecode(c.vdt, vc[e], g.izipv);
-      v = v + f[e] * (double)c.a_mid * (double)c.dt / 6.0 / (double)PI_F;
+      const double k6 = div_const(f[e] * (double)c.a_mid * (double)c.dt, 6.0, 1.0 / 6.0);
+      v = v + div_const(k6, (double)PI_F, 1.0 / (double)PI_F);
       store_v(vp, 3 * p + e, g.izipv, vencode(c.venc, c.kmax, g.izipv, c.c_old, v));
     }
   }
@@ -528,172 +525,342 @@ __device__ void pf_reduce(float f2loc, unsigned long long npl, int32_t ninner, f
 template <int PB>
 struct PFcfg;
 template <>
-struct PFcfg<4> { static constexpr int NT = 512, K = 4, CAP = 2048; };
+struct PFcfg<4> { static constexpr int NT = 512, K = 4, CAP = 2048, OWN = 4096; };
 template <>
-struct PFcfg<2> { static constexpr int NT = 128, K = 4, CAP = 1024; };
+struct PFcfg<2> { static constexpr int NT = 128, K = 4, CAP = 1024, OWN = 2048; };
 
-__host__ __device__ constexpr int pf_wc_bytes(int W3) { return ((W3 + 2) * 4 + 15) / 16 * 16; }
-
-// LDS (dynamic): the run table, W^3+2 16-bit entries (entry 1+i: count,
-// then start, then end of run i; entry 0 = 0), then CAP entries
-template <int PB, typename RT>
-__global__ __launch_bounds__(PFcfg<PB>::NT) void k_pp_fast(Geo g, PPctx c, const void* __restrict__ xp, void* vp,
-                                                          const int64_t* __restrict__ cstart, uint32_t* f2max_bits,
-                                                          unsigned long long* npairs_out, unsigned long long* nupd_out,
-                                                          double* probe, int32_t* dense, uint32_t* ndense) {
+// One workgroup per PB^3 coarse cells.  The kernel is bound by VALU issue
+// (98% of the SIMDs' issue slots at 1024^3 particles), so it is written for
+// instruction count; the reach PR and the code width ZX are template
+// parameters.
+//   1. region particles are binned by window fine cell in LDS (16-bit counts,
+//      scanned two to a word); a particle's region cell comes from a byte
+//      table filled by a max-scan of the cells' first particles, whose cost
+//      does not depend on how crowded a cell is;
+//   2. each run is put in particle-index order, which fixes the order of the
+//      pair sums; most runs hold one particle and move nothing;
+//   3. targets are dealt to the lanes in window order.  A wavefront walks
+//      each of the (2 PR+1)^2 rows to its longest run among its lanes, and
+//      lanes in neighbouring fine cells have runs of similar length: against
+//      the order of the coarse cells the walk takes 171 steps instead of 317
+//      per wavefront on a 128^3 box at z = 0.6 (94 if no lane ever idled),
+//      77 instead of 131 at z = 1.1 and 11.7 instead of 11.3 on a nearly
+//      uniform one.
+// Against one kernel for every reach, particles ranked after a second pass over
+// their entries and targets in coarse-cell order, the whole PP pass takes 17.9
+// instead of 29.3 ms at 512^3 particles and z = 1.1 (46 pairs each), 4.8
+// instead of 8.7 ms at 256^3 and z = 0.5 (114), 0.82 instead of 1.10 ms at
+// 256^3 and z = 9 (2.4) and, with reach 2, 1.8 instead of 5.0 ms at 101^3 (84).
+// LDS (dynamic): the run table, W^3+2 16-bit entries (entry 1+i: count, then
+// start, then end of run i; entry 0 = 0), then CAP entries.  Three workgroups
+// fit a CU.
+template <int PR, int ZX, typename RT>
+__global__ __launch_bounds__(PFcfg<(PR <= 2 ? 4 : 2)>::NT) void k_pp_fast(Geo g, PPctx c, const void* __restrict__ xp, void* vp,
+                                                                        const int64_t* __restrict__ cstart, uint32_t* f2max_bits,
+                                                                        unsigned long long* npairs_out,
+                                                                        unsigned long long* nupd_out, double* probe,
+                                                                        int32_t* dense, uint32_t* ndense) {
+  constexpr int PB = PR <= 2 ? 4 : 2;
   using G = PBgeo<PB>;
-  constexpr int NT = PFcfg<PB>::NT, K = PFcfg<PB>::K, CAP = PFcfg<PB>::CAP;
+  using C = PFcfg<PB>;
+  constexpr int NT = C::NT, K = C::K, CAP = C::CAP, NW = NT / 64;
+  constexpr int W = G::FB + 2 * PR, W3 = W * W * W, NWORD = (W3 + 3) / 2;
   extern __shared__ __align__(16) uint8_t pf_dyn[];
-  __shared__ int64_t beg[G::NCELL];
+  __shared__ int2 cinfo[G::NCELL];  // first particle minus its region index; window origin, 8 bits an axis
   __shared__ int32_t off[G::NCELL + 1];
-  __shared__ int32_t ncand_s, wsum[NT / 64], redi[NT / 64];
-  __shared__ float redf[NT / 64];
-  __shared__ unsigned long long redn[NT / 64];
-  __shared__ uint8_t owner[PF_OWN];
-  __shared__ int32_t inoff[PB * PB * PB + 1];
-  __shared__ uint8_t ia[PB * PB * PB];
+  __shared__ int32_t wsum[NW];
+  __shared__ int32_t ncand_s;
+  __shared__ __align__(8) uint8_t owner[C::OWN];  // region cell of region particle t; later the target list
+  constexpr int PE = (CAP + NT - 1) / NT;
+  __shared__ int32_t tcnt[64];
+  static_assert(PE * NW <= 64, "one lane per count");
+  __shared__ uint32_t redf[NW], redn[NW];
   int c0x, c0y, c0z;
   pf_origin<PB>(g, blockIdx.x, c0x, c0y, c0z);
-  const int pr = c.pr, W = G::FB + 2 * pr, W3 = W * W * W;
-  const RunU16 wc{(uint32_t*)pf_dyn};
-  PPent* ent = (PPent*)(pf_dyn + pf_wc16_bytes(W3));
-  for (int i = threadIdx.x; i < (W3 + 3) / 2; i += NT) wc.w[i] = 0u;
-  if (threadIdx.x == 0) ncand_s = 0;
-  pf_region<PB, NT>(g, cstart, c0x, c0y, c0z, beg, off, wsum);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t* const wcw = (uint32_t*)pf_dyn;
+  const uint16_t* const wc = (const uint16_t*)pf_dyn;
+  PPent* const ent = (PPent*)(pf_dyn + pf_wc16_bytes(W3));
+  auto inc = [&](int i) -> int {  // add one to entry i, returning its previous value
+    return (int)((atomicAdd(&wcw[i >> 1], 1u << ((i & 1) * 16)) >> ((i & 1) * 16)) & 0xFFFFu);
+  };
+  for (int i = tid; i < NWORD; i += NT) wcw[i] = 0u;
+  constexpr int OW = C::OWN / NT / 8;  // 8-byte words of the owner table per thread
+  {
+    unsigned long long* o8 = (unsigned long long*)owner;
+    for (int i = tid; i < C::OWN / 8; i += NT) o8[i] = 0ull;
+  }
+  if (tid == 0) ncand_s = 0;
+  // region cells: particle ranges, scanned
+  static_assert(G::NCELL <= NT && G::NCELL <= 256, "one thread per region cell; owner entries are bytes");
+  int32_t rc0 = 0, rn = 0, rpack = 0;
+  if (tid < G::NCELL) {
+    const int rx = tid % G::SPAN, ry = (tid / G::SPAN) % G::SPAN, rz = tid / (G::SPAN * G::SPAN);
+    const int64_t r = rank_of(g, wrapc(c0x + rx - 1, g.nc), wrapc(c0y + ry - 1, g.nc), wrapc(c0z + rz - 1, g.nc));
+    const int64_t b = cstart[r];
+    rc0 = (int32_t)b;
+    rn = (int32_t)(cstart[r + 1] - b);
+    rpack = (CUBE_NCELL * rx) | ((CUBE_NCELL * ry) << 8) | ((CUBE_NCELL * rz) << 16);
+  }
+  const int32_t rincl = wave_incl_add(rn);
+  if (lane == 63) wsum[wv] = rincl;
   __syncthreads();
-  const int32_t ntot = off[G::NCELL];
-  // owner table: region cell of each of the first PF_OWN region particles
-  static_assert(G::NCELL <= 256, "owner entries are bytes");
-  const bool use_owner = ntot <= PF_OWN;
-  if (use_owner && (int)threadIdx.x < G::NCELL)
-    for (int32_t t = off[threadIdx.x]; t < off[threadIdx.x + 1]; t++) owner[t] = (uint8_t)threadIdx.x;
+  int32_t rbase = 0, ntot = 0;
+  for (int w = 0; w < NW; w++) {
+    const int32_t v = wsum[w];
+    if (w < wv) rbase += v;
+    ntot += v;
+  }
+  const int32_t roff = rbase + rincl - rn;
+  if (tid < G::NCELL) {
+    off[tid] = roff;
+    cinfo[tid] = make_int2(rc0 - roff, rpack);
+    if (rn > 0 && roff < C::OWN) owner[roff] = (uint8_t)tid;
+  }
+  if (tid == 0) off[G::NCELL] = ntot;
   __syncthreads();
-  const uint8_t* own = use_owner ? owner : nullptr;
-  // pass 1: the first K*NT region particles are kept in registers
+  const bool use_owner = ntot <= C::OWN;
+  if (use_owner) {
+    // running maximum of the first-particle marks (they increase with t)
+    unsigned long long w8[OW];
+    int32_t m = 0;
+#pragma unroll
+    for (int q = 0; q < OW; q++) {
+      w8[q] = ((unsigned long long*)owner)[tid * OW + q];
+      if (w8[q]) m = (int32_t)(w8[q] >> ((63 - __clzll((long long)w8[q])) & ~7)) & 0xFF;
+    }
+    const int32_t mi = wave_incl_max(m);
+    if (lane == 63) wsum[wv] = mi;
+    __syncthreads();
+    int32_t run = __builtin_amdgcn_update_dpp(0, mi, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    for (int w = 0; w < wv; w++) run = max(run, wsum[w]);
+#pragma unroll
+    for (int q = 0; q < OW; q++) {
+      unsigned long long o = 0;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int32_t v = (int32_t)((w8[q] >> (8 * e)) & 0xFFu);
+        run = v ? v : run;
+        o |= (unsigned long long)(uint32_t)run << (8 * e);
+      }
+      ((unsigned long long*)owner)[tid * OW + q] = o;
+    }
+    __syncthreads();
+  }
+  // window cell and block-local position of region particle t (exact in FP32:
+  // at most 20 significant bits); false outside the window
+  auto cand = [&](int32_t t, int& wi, PPent& e) -> bool {
+    int a;
+    if (use_owner) {
+      a = owner[t];
+    } else {
+      a = 0;
+      int b = G::NCELL;
+      while (b - a > 1) {
+        const int m = (a + b) >> 1;
+        if (off[m] <= t) a = m; else b = m;
+      }
+    }
+    const int2 ci = cinfo[a];
+    const uint32_t p = (uint32_t)(ci.x + t);
+    uint32_t u[3];
+    if (ZX == 1) {
+      const uint8_t* q = (const uint8_t*)xp + (size_t)p * 3;
+      u[0] = q[0]; u[1] = q[1]; u[2] = q[2];
+    } else {
+      const uint16_t* q = (const uint16_t*)xp + (size_t)p * 3;
+      u[0] = q[0]; u[1] = q[1]; u[2] = q[2];
+    }
+    constexpr int SH = ZX == 1 ? 6 : 14;                    // bits below the fine cell
+    constexpr float res = ZX == 1 ? 0.0078125f : 3.0517578125e-05f;
+    int w[3];
+    float x[3];
+    bool keep = true;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int o4 = (ci.y >> (8 * d)) & 0xFF;              // 4 * (cell - first region cell)
+      w[d] = o4 + (int)(u[d] >> SH) + (PR - CUBE_NCELL);
+      // 4*(u+0.5)/2^(8 izipx) above the cell's edge, as one whole number of half units
+      x[d] = (float)(((o4 - CUBE_NCELL) << (SH + 1)) + (int)(2 * u[d] + 1)) * res;
+      keep = keep && (uint32_t)w[d] < (uint32_t)W;
+    }
+    wi = (w[2] * W + w[1]) * W + w[0];
+    e = PPent{x[0], x[1], x[2], (int32_t)p};
+    return keep;
+  };
+  // the first K*NT region particles are kept in registers
   PPent re[K];
   int rw[K];
-  bool rk[K];
-  int32_t mine = 0;
+  int mine = 0;
 #pragma unroll
   for (int k = 0; k < K; k++) {
-    const int32_t t = threadIdx.x + k * NT;
-    rk[k] = t < ntot && pf_cand<PB>(g, xp, beg, off, t, pr, W, rw[k], re[k], own);
+    const int32_t t = tid + k * NT;
+    bool ok = false;
+    if (t < ntot) ok = cand(t, rw[k], re[k]);
+    if (!ok) rw[k] = -1;
+    mine += __popcll(__ballot(ok));
   }
 #pragma unroll
   for (int k = 0; k < K; k++)
-    if (rk[k]) {
-      wc.inc(1 + rw[k]);
-      mine++;
-    }
-  for (int32_t t = threadIdx.x + K * NT; t < ntot; t += NT) {
+    if (rw[k] >= 0) inc(1 + rw[k]);
+  for (int32_t t0 = K * NT; t0 < ntot; t0 += NT) {
+    const int32_t t = t0 + tid;
     int wi;
     PPent e;
-    if (pf_cand<PB>(g, xp, beg, off, t, pr, W, wi, e)) {
-      wc.inc(1 + wi);
-      mine++;
-    }
+    const bool ok = t < ntot && cand(t, wi, e);
+    if (ok) inc(1 + wi);
+    mine += __popcll(__ballot(ok));
   }
-  if (mine) atomicAdd(&ncand_s, mine);
+  if (lane == 0 && mine) atomicAdd(&ncand_s, mine);
   __syncthreads();
   const int32_t ncand = ncand_s;
   if (ncand > CAP) {
-    if (threadIdx.x == 0) dense[atomicAdd(ndense, 1u)] = (int32_t)blockIdx.x;
+    if (tid == 0) dense[atomicAdd(ndense, 1u)] = (int32_t)blockIdx.x;
     return;
   }
-  pf_scan16<NT>(wc, W3, wsum);
+  // exclusive scan of the counts in place, two to a word (entry 0 and the
+  // entries past W3 are zero, so whole words need no masks)
+  {
+    constexpr int PER = (NWORD + NT - 1) / NT;
+    uint32_t v[PER];
+    int32_t s = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int i = tid * PER + q;
+      v[q] = i < NWORD ? wcw[i] : 0u;
+      s += (int32_t)((v[q] & 0xFFFFu) + (v[q] >> 16));
+    }
+    const int32_t incl = wave_incl_add(s);
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    uint32_t run = (uint32_t)(incl - s);
+    for (int w = 0; w < wv; w++) run += (uint32_t)wsum[w];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int i = tid * PER + q;
+      const uint32_t lo = v[q] & 0xFFFFu;
+      if (i < NWORD) wcw[i] = run | ((run + lo) << 16);
+      run += lo + (v[q] >> 16);
+    }
+    __syncthreads();
+  }
   // scatter; afterwards entry 1+i is the end of run i, so entry i is the start of run i
 #pragma unroll
   for (int k = 0; k < K; k++)
-    if (rk[k]) ent[wc.inc(1 + rw[k])] = re[k];
-  for (int32_t t = threadIdx.x + K * NT; t < ntot; t += NT) {
+    if (rw[k] >= 0) ent[inc(1 + rw[k])] = re[k];
+  for (int32_t t = tid + K * NT; t < ntot; t += NT) {
     int wi;
     PPent e;
-    if (pf_cand<PB>(g, xp, beg, off, t, pr, W, wi, e)) ent[wc.inc(1 + wi)] = e;
+    if (cand(t, wi, e)) ent[inc(1 + wi)] = e;
   }
   __syncthreads();
-  // runs in particle-index order, so the pair sums below have a fixed
-  // order: each entry moves to its run's start plus its rank by particle
-  // index within the run (entries are held in registers across the barrier)
-  {
-    constexpr int PE = (CAP + NT - 1) / NT;
-    PPent me[PE];
-    int dst[PE];
+  // runs in particle-index order: an entry whose rank by index within its run
+  // is not its place moves there (held in registers across the barrier).
+  // Targets are the entries of the block's own fine cells; an entry's run
+  // stays where it is, so its old place tells the target's place.
+  PPent me[PE];
+  int dst[PE];
+  uint32_t inner = 0;
 #pragma unroll
-    for (int k = 0; k < PE; k++) {
-      const int m = threadIdx.x + k * NT;
-      dst[k] = -1;
-      if (m < ncand) {
-        me[k] = ent[m];
-        const int wi = (((int)floorf(me[k].z) + pr) * W + ((int)floorf(me[k].y) + pr)) * W + (int)floorf(me[k].x) + pr;
-        const int a = wc.get(wi), b = wc.get(wi + 1);
-        int rank = 0;
-        if (b - a > 1)
-          for (int j = a; j < b; j++) rank += ent[j].p < me[k].p ? 1 : 0;
-        dst[k] = a + rank;
+  for (int k = 0; k < PE; k++) {
+    const int m = tid + k * NT;
+    dst[k] = m;
+    bool in = false;
+    if (m < ncand) {
+      me[k] = ent[m];
+      const int fx = (int)floorf(me[k].x), fy = (int)floorf(me[k].y), fz = (int)floorf(me[k].z);
+      in = ((uint32_t)fx < (uint32_t)G::FB) && ((uint32_t)fy < (uint32_t)G::FB) && ((uint32_t)fz < (uint32_t)G::FB);
+      const int wi = ((fz + PR) * W + (fy + PR)) * W + fx + PR;
+      const int a = wc[wi], b = wc[wi + 1];
+      if (b - a > 1) {
+        int rank = a;
+        for (int j = a; j < b; j++) rank += ent[j].p < me[k].p ? 1 : 0;
+        dst[k] = rank;
       }
     }
-    __syncthreads();
-    // the owner table is dead now; its bytes hold tpos[t], the sorted
-    // position of region particle t < PF_OWN/2, for the target lookup below
-    uint16_t* tpos = reinterpret_cast<uint16_t*>(owner);
+    const unsigned long long bal = __ballot(in);
+    if (in) inner |= 1u << k;
+    if (lane == 0) tcnt[k * NW + wv] = __popcll(bal);
+  }
+  __syncthreads();
+  uint16_t* const tl = reinterpret_cast<uint16_t*>(owner);
+  const int32_t tv = lane < PE * NW ? tcnt[lane] : 0;
+  const int32_t ti_incl = wave_incl_add(tv);
+  const int32_t ntarget = __builtin_amdgcn_readlane(ti_incl, 63);
 #pragma unroll
-    for (int k = 0; k < PE; k++)
-      if (dst[k] >= 0) {
-        ent[dst[k]] = me[k];
-        const int rx = (int)floorf(me[k].x * 0.25f), ry = (int)floorf(me[k].y * 0.25f), rz = (int)floorf(me[k].z * 0.25f);
-        const int a = ((rz + 1) * G::SPAN + (ry + 1)) * G::SPAN + (rx + 1);
-        const int32_t t = off[a] + (int32_t)((int64_t)me[k].p - beg[a]);
-        if (t < PF_OWN / 2) tpos[t] = (uint16_t)dst[k];
-      }
+  for (int k = 0; k < PE; k++) {
+    const int m = tid + k * NT;
+    if (dst[k] != m) ent[dst[k]] = me[k];
+    const bool in = (inner >> k) & 1u;
+    const unsigned long long bal = __ballot(in);
+    const int32_t tb = __builtin_amdgcn_readlane(ti_incl - tv, k * NW + wv);
+    if (in) tl[tb + __popcll(bal & ((1ull << lane) - 1))] = (uint16_t)m;
   }
   __syncthreads();
-  // targets: the particles of the workgroup's own PB^3 coarse cells, dealt
-  // out densely to the threads (inner cell ib <-> region cell ia[ib])
-  if (threadIdx.x < 64) {
-    const int ib = threadIdx.x;
-    int32_t cnt = 0;
-    if (ib < PB * PB * PB) {
-      const int a = ((ib / (PB * PB)) + 1) * G::SPAN * G::SPAN + ((ib / PB) % PB + 1) * G::SPAN + (ib % PB) + 1;
-      ia[ib] = (uint8_t)a;
-      cnt = off[a + 1] - off[a];
-    }
-    int32_t incl = cnt;
-    for (int o = 1; o < 64; o <<= 1) {
-      const int32_t v = __shfl_up(incl, o);
-      if (ib >= o) incl += v;
-    }
-    if (ib < PB * PB * PB) inoff[ib + 1] = incl;
-    if (ib == 0) inoff[0] = 0;
-  }
-  __syncthreads();
-  const int32_t ntarget = inoff[PB * PB * PB];
   float f2loc = 0.f;
-  unsigned long long npl = 0;
-  int32_t ninner = 0;
-  for (int32_t k = threadIdx.x; k < ntarget; k += NT) {
-    int lo = 0, hi = PB * PB * PB;
-    while (hi - lo > 1) {
-      const int m = (lo + hi) >> 1;
-      if (inoff[m] <= k) lo = m; else hi = m;
-    }
-    const int a = ia[lo];
-    const int32_t t = off[a] + (k - inoff[lo]);
-    PPent ti;
-    if (t < PF_OWN / 2) {
-      ti = ent[reinterpret_cast<const uint16_t*>(owner)[t]];
-    } else {
-      int wi_unused;
-      (void)pf_cand<PB>(g, xp, beg, off, t, pr, W, wi_unused, ti);
-    }
-    ninner++;
+  uint32_t npl = 0;
+  const PFsoft soft{c.rsoft, c.rsoft * c.rsoft * (1.0f - 1e-6f), c.rsoft * c.rsoft * (1.0f + 1e-6f)};
+  for (int32_t k = tid; k < ntarget; k += NT) {
+    const PPent ti = ent[tl[k]];
     int32_t vc[3] = {0, 0, 0};
     if (!probe)
       for (int e = 0; e < 3; e++) vc[e] = load_v(vp, 3 * (int64_t)ti.p + e, g.izipv);
     typename std::conditional<sizeof(RT) == 4, PPaccOrd, PPacc<double>>::type acc;
-    pf_force<RT, true>(ent, wc, W, pr, ti, c.mass, c.rsoft, acc, npl);
+    // rows wz-PR..wz+PR, wy-PR..wy+PR; run of x cells wx-PR..wx+PR.  The
+    // next row's bounds are requested before this row is walked.
+    const uint16_t* row = wc + ((int)floorf(ti.z) * W + (int)floorf(ti.y)) * W + (int)floorf(ti.x);
+    int j0 = row[0], j1 = row[2 * PR + 1];
+#pragma unroll 1
+    for (int r = 0; r < (2 * PR + 1) * (2 * PR + 1); r++) {
+      row += (r + 1) % (2 * PR + 1) == 0 ? W * (W - 2 * PR) : W;
+      const bool more = r + 1 < (2 * PR + 1) * (2 * PR + 1);
+      const int n0 = more ? row[0] : 0, n1 = more ? row[2 * PR + 1] : 0;
+      npl += (uint32_t)(j1 - j0);
+      RT sx = 0, sy = 0, sz = 0;
+      for (int j = j0; j < j1; j++) {
+        const PPent pj = ent[j];
+        // branch-free: an excluded pair adds sc = 0 (a signed zero, which
+        // leaves the running sum unchanged)
+        RT sc;
+        const RT dx = (RT)pj.x - (RT)ti.x, dy = (RT)pj.y - (RT)ti.y, dz = (RT)pj.z - (RT)ti.z;
+        if constexpr (sizeof(RT) == 4) sc = pf_pair_fast(dx, dy, dz, c.mass, soft);
+        else sc = pf_pair_sel(dx, dy, dz, (RT)c.mass, (RT)c.rsoft, (RT)c.rsoft * (RT)c.rsoft);
+        sx = fma(sc, dx, sx);
+        sy = fma(sc, dy, sy);
+        sz = fma(sc, dz, sz);
+      }
+      if (j1 > j0) {
+        acc.add(0, sx);
+        acc.add(1, sy);
+        acc.add(2, sz);
+      }
+      j0 = n0;
+      j1 = n1;
+    }
     f2loc = fmaxf(f2loc, pf_apply(g, c, vp, probe, ti.p, vc, acc));
   }
-  pf_reduce<NT>(f2loc, npl, ninner, redf, redn, redi, f2max_bits, npairs_out, nupd_out);
+  // totals into one of PP_SLOTS slots per workgroup (max and integer sums are
+  // order-independent)
+  const uint32_t fm = wave_max_bits(__float_as_uint(f2loc));
+  const int32_t nsum = __builtin_amdgcn_readlane(wave_incl_add((int32_t)npl), 63);
+  if (lane == 0) {
+    redf[wv] = fm;
+    redn[wv] = (uint32_t)nsum;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t m = 0;
+    unsigned long long nn = 0;
+    for (int i = 0; i < NW; i++) {
+      m = max(m, redf[i]);
+      nn += redn[i];
+    }
+    const int sl = blockIdx.x & (PP_SLOTS - 1);
+    if (m) atomicMax(f2max_bits + sl, m);
+    if (nn) atomicAdd(npairs_out + sl, nn);
+    if (ntarget) atomicAdd(nupd_out + sl, (unsigned long long)ntarget);
+  }
 }
 
 // Dense blocks, step 1 (one workgroup per listed block, grid-stride): sort
@@ -832,7 +999,7 @@ __global__ __launch_bounds__(PD_NT) void k_pp_dense_pairs(Geo g, PPctx c, void* 
       if (!probe)
         for (int q = 0; q < 3; q++) vc[q] = load_v(vp, 3 * (int64_t)ti.p + q, g.izipv);
       PPacc<RT> acc;
-      pf_force<RT, false>(ent, RunI32{st}, W, pr, ti, c.mass, c.rsoft, acc, npl);
+      pf_force<RT>(ent, RunI32{st}, W, pr, ti, c.mass, c.rsoft, c.whole, acc, npl);
       f2loc = pf_apply(g, c, vp, probe, ti.p, vc, acc);
       ninner = 1;
     }
@@ -840,19 +1007,24 @@ __global__ __launch_bounds__(PD_NT) void k_pp_dense_pairs(Geo g, PPctx c, void* 
   }
 }
 
-template <int PB, typename RT>
+template <int PR, typename RT>
 static int pp_launch(cube_handle* h, const Geo& g, const PPctx& c, uint32_t* f2, unsigned long long* npr, unsigned long long* nup,
                      double* probe, int32_t* dense, uint32_t* ndense, int64_t* info, int64_t* items, uint32_t* nitems,
                      int32_t* fall, uint32_t* nfall, unsigned long long* pool_used) {
+  constexpr int PB = PR <= 2 ? 4 : 2;
   using G = PBgeo<PB>;
-  const int W = G::FB + 2 * c.pr, W3 = W * W * W;
+  constexpr int W = G::FB + 2 * PR, W3 = W * W * W;
   const int64_t nbx = h->nc / PB, nb = nbx * nbx * nbx;
-  const size_t lds_fast = pf_wc16_bytes(W3) + sizeof(PPent) * PFcfg<PB>::CAP;
+  constexpr size_t lds_fast = pf_wc16_bytes(W3) + sizeof(PPent) * PFcfg<PB>::CAP;
+  static_assert(lds_fast + 9 * 1024 <= 64 * 1024, "fits without raising the dynamic LDS limit");
   const size_t lds_tab = sizeof(int32_t) * (W3 + 1);
   const uint64_t pool_cap = h->fine.bytes_R() / sizeof(PPent);
-  HIP_TRY(h, hipFuncSetAttribute((const void*)k_pp_fast<PB, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_fast));
-  k_pp_fast<PB, RT><<<(unsigned)nb, PFcfg<PB>::NT, lds_fast, h->stream>>>(g, c, h->xp, h->vp, h->cstart, f2, npr, nup, probe, dense,
-                                                                      ndense);
+  if (h->p.izipx == 1)
+    k_pp_fast<PR, 1, RT><<<(unsigned)nb, PFcfg<PB>::NT, lds_fast, h->stream>>>(g, c, h->xp, h->vp, h->cstart, f2, npr, nup, probe,
+                                                                               dense, ndense);
+  else
+    k_pp_fast<PR, 2, RT><<<(unsigned)nb, PFcfg<PB>::NT, lds_fast, h->stream>>>(g, c, h->xp, h->vp, h->cstart, f2, npr, nup, probe,
+                                                                               dense, ndense);
   HIP_TRY(h, hipGetLastError());
   k_pp_dense_prep<PB><<<2048, PD_NT, lds_tab, h->stream>>>(g, c.pr, h->xp, h->cstart, dense, ndense, (PPent*)h->fine.W, pool_cap,
                                                             pool_used, info, items, nitems, fall, nfall);
@@ -926,11 +1098,20 @@ int pp_launch_step(cube_handle* h, float a_mid, float dt, double c_old, double* 
   int64_t* items = info + 2 * nb2;
   int32_t* dense = (int32_t*)(items + h->p.np_max / PD_NT + nb2 + 1);
   int32_t* fall = dense + nb2;
-  PPctx c{h->mass_p, h->p.rsoft, a_mid, dt, c_old, vtab_for(h, c_old), h->venc, h->vkmax, prange};
+  PPctx c{h->mass_p, h->p.rsoft, a_mid, dt, c_old, vtab_for(h, c_old), h->venc, h->vkmax, prange, 0};
+  {
+    // whole-number sums stay below 2^53 for up to 2^20 / (mass/rsoft^2) pairs, with a factor 2 to spare
+    const double most = (double)h->mass_p / ((double)h->p.rsoft * (double)h->p.rsoft);
+    c.whole = most > 0 ? (int32_t)std::min(1048576.0 / most, 1048576.0) : 0;
+  }
   int pr = prof_begin(h, PS_PP);
 #define PP_ARGS h, g, c, f2, npr, nup, probe, dense, ndense, info, items, nitems, fall, nfall, pool_used
-  if (h->prec == 4) rc = PBsel == 4 ? pp_launch<4, float>(PP_ARGS) : pp_launch<2, float>(PP_ARGS);
-  else rc = PBsel == 4 ? pp_launch<4, double>(PP_ARGS) : pp_launch<2, double>(PP_ARGS);
+  switch (prange) {
+    case 1: rc = h->prec == 4 ? pp_launch<1, float>(PP_ARGS) : pp_launch<1, double>(PP_ARGS); break;
+    case 2: rc = h->prec == 4 ? pp_launch<2, float>(PP_ARGS) : pp_launch<2, double>(PP_ARGS); break;
+    case 3: rc = h->prec == 4 ? pp_launch<3, float>(PP_ARGS) : pp_launch<3, double>(PP_ARGS); break;
+    default: rc = h->prec == 4 ? pp_launch<4, float>(PP_ARGS) : pp_launch<4, double>(PP_ARGS);
+  }
 #undef PP_ARGS
   if (rc) return rc;
   // blocks the pool could not hold: chunked kernel on their PP_BP^3 sub-blocks
