@@ -34,6 +34,9 @@
 #define HNT 256
 #define HFIX 1099511627776.0  // 2^40
 #define HMAXCELLS 2048        // search-box cells a workgroup stages in LDS
+#define HGL 8                 // refined-grid loads in flight per thread
+#define HGU 4                 // particles per thread and round of a peak's gather
+#define HSORT 4096            // search lists up to this are sorted in LDS
 #define HSPIN_LIMIT (1u << 26)
 
 int cic_halo_density(cube_handle* h, float* out);
@@ -42,6 +45,8 @@ static_assert(sizeof(cube_halo_params) == 80, "cube_halo_params layout");
 static_assert(sizeof(cube_halo_catalog) == 80, "cube_halo_catalog layout");
 
 namespace {
+
+static_assert(HSORT * sizeof(uint64_t) <= HMAXCELLS * 16, "sort keys fit the cell tables");
 
 struct HalopCfg {
   int32_t nc, nt, nnt, ncb, N, nft, nfb;
@@ -132,7 +137,7 @@ __global__ void k_halo_peaks(const float* __restrict__ rho, HalopCfg c, uint32_t
 // ------------------------------------------------------------ mesh walk
 __global__ void k_halo_walk(const float* __restrict__ rho, HalopCfg c, const int4* __restrict__ cand, int64_t ncand,
                             const uint64_t* __restrict__ tab, int64_t ntab, int32_t R, uint32_t* nvalid, int32_t* vidx,
-                            float* cden, float* cmesh, float* chpos, uint32_t* cloop) {
+                            float* cden, float* cmesh, float* chpos, uint32_t* cloop, uint32_t* nshort) {
   const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (s >= ncand) return;
   const int4 cd = cand[s];
@@ -146,6 +151,7 @@ __global__ void k_halo_walk(const float* __restrict__ rho, HalopCfg c, const int
   const int32_t lo = 1 - c.nfb, hi = c.nft + c.nfb - 1;
   int32_t dx, dy, dz, r2;
   if (ntab > 0) hoff_decode(tab[0], R, dx, dy, dz, r2);
+  bool ended = false;
   for (int64_t ii = 1; ii <= ntab; ii++) {
     int32_t nx = 0, ny = 0, nz = 0, nr2 = -1;
     if (ii < ntab) hoff_decode(tab[ii], R, nx, ny, nz, nr2);
@@ -153,10 +159,11 @@ __global__ void k_halo_walk(const float* __restrict__ rho, HalopCfg c, const int
     const bool skip = ix <= lo || ix >= hi || iy <= lo || iy >= hi || iz <= lo || iz >= hi;
     if (!skip) {
       m_mesh = m_mesh + R3(ix, iy, iz);
-      if (!(ii < ntab && nr2 == r2) && ii >= 19 && m_mesh / (float)ii < c.den_odc) break;
+      if (!(ii < ntab && nr2 == r2) && ii >= 19 && m_mesh / (float)ii < c.den_odc) { ended = true; break; }
     }
     dx = nx; dy = ny; dz = nz; r2 = nr2;
   }
+  if (!ended && nshort) atomicAdd(nshort, 1u);  // the table ends before the halo does
   if (!(m_mesh > c.mass_p * (float)c.min_np / 2.0f)) return;
   const uint32_t v = atomicAdd(nvalid, 1u);
   const float cc = R3(i0, j0, k0);
@@ -233,6 +240,31 @@ __global__ void k_halo_bin_fill(int64_t npk, const HPk* __restrict__ pk, const i
   binlist[binoff[b] + atomicAdd(binfill + b, 1u)] = (int32_t)s;
 }
 
+// largest number of particles in any peak's search box (one wavefront per
+// peak): no peak gathers more
+__global__ __launch_bounds__(HNT) void k_halo_box_count(Geo g, HalopCfg c, int64_t npk, const HPk* __restrict__ pk,
+                                                        const int64_t* __restrict__ cstart, unsigned long long* most) {
+  const int64_t s = (int64_t)blockIdx.x * (HNT / 64) + (threadIdx.x >> 6);
+  if (s >= npk) return;
+  const HPk p = pk[s];
+  const int32_t lane = threadIdx.x & 63;
+  const int32_t T[3] = {p.t % c.nnt, (p.t / c.nnt) % c.nnt, p.t / (c.nnt * c.nnt)};
+  int32_t n[3];
+  for (int d = 0; d < 3; d++) {
+    n[d] = p.cs1[d] - p.cs0[d] + 1;
+    if (p.cs0[d] < 1 - c.ncb || p.cs1[d] > c.nt + c.ncb) return;  // reported by k_halo_prep
+  }
+  int64_t sum = 0;
+  for (int32_t i = lane; i < n[0] * n[1] * n[2]; i += 64) {
+    const int32_t ci = p.cs0[0] + i % n[0], cj = p.cs0[1] + (i / n[0]) % n[1], ck = p.cs0[2] + i / (n[0] * n[1]);
+    const int64_t r = rank_of(g, wrapn(T[0] * c.nt + ci - 1, c.nc), wrapn(T[1] * c.nt + cj - 1, c.nc),
+                              wrapn(T[2] * c.nt + ck - 1, c.nc));
+    sum += cstart[r + 1] - cstart[r];
+  }
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane == 0) atomicMax(most, (unsigned long long)sum);
+}
+
 // ------------------------------------------------------- block utilities
 __device__ __forceinline__ uint64_t block_scan_excl(uint64_t v, uint64_t* wsum, uint64_t& total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -264,6 +296,15 @@ __device__ __forceinline__ V block_reduce(V v, V* buf, Op op) {
 }
 
 // ------------------------------------------------------- peak processing
+// Until every memory operation this wavefront issued has been performed.
+// Peaks hand on nothing but particle tags, which are written and read by
+// device-scope atomics: once the atomics of a peak have been performed, its
+// `done` flag may be set, and who sees the flag sees the tags.  A device-scope
+// release or acquire fence would besides write back and invalidate the XCD's
+// L2; four of them per peak bounded the kernel (5.2 ms for 11485 peaks,
+// whatever else it did).
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+
 struct HWs {  // one workgroup's scratch in global memory
   int32_t* q;       // gathered particle index
   int32_t* rk;      // its cell rank
@@ -282,12 +323,16 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
                                                       int32_t* mq, int32_t* mrk, uint32_t* mbit, unsigned long long* mcount,
                                                       uint32_t* errf, char* wsbase, int64_t wsbytes) {
   __shared__ int32_t s_p;
-  __shared__ int64_t beg[HMAXCELLS];
-  __shared__ int32_t off[HMAXCELLS + 1];
-  __shared__ int32_t crk[HMAXCELLS];
+  // the search box's cells while particles are gathered, then the sort's keys
+  __shared__ __align__(16) char s_cells[HMAXCELLS * 16 + 16];
+  int64_t* const beg = (int64_t*)s_cells;
+  int32_t* const crk = (int32_t*)(s_cells + HMAXCELLS * 8);
+  int32_t* const off = (int32_t*)(s_cells + HMAXCELLS * 12);  // HMAXCELLS + 1
+  uint64_t* const skey = (uint64_t*)s_cells;
   __shared__ uint64_t wsum[HNT / 64];
   __shared__ long long rbuf[HNT / 64];
   __shared__ int64_t s_moff;
+  __shared__ int32_t s_cnt[HGU * (HNT / 64)];
   const int tid = threadIdx.x;
   HWs ws;
   {
@@ -327,7 +372,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
           const float rr = p.rs + q.rs + 1e-3f;
           if (d0 * d0 + d1 * d1 + d2 * d2 >= rr * rr) continue;
           uint32_t spins = 0;
-          while (__hip_atomic_load(done + Q, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+          while (__hip_atomic_load(done + Q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
             __builtin_amdgcn_s_sleep(2);
             if (++spins > HSPIN_LIMIT) { ok = false; break; }
           }
@@ -336,7 +381,6 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
         if (!ok) break;
       }
       if (!ok) atomicOr(errf, 8u);
-      __threadfence();
     }
     __syncthreads();
     const int32_t T[3] = {p.t % c.nnt, (p.t / c.nnt) % c.nnt, p.t / (c.nnt * c.nnt)};
@@ -376,49 +420,72 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
     const int32_t total = off[ncell];
     // gather untagged particles within rsearch, in the reference's order
     // (cells k, j, i; particles in cell order)
+    // HGU particles per thread and round: their searches, positions and tags
+    // are independent chains, and one barrier pair serves them all
     uint64_t n_odc = 0;
     bool over = false;
-    for (int32_t t0 = 0; t0 < total; t0 += HNT) {
-      const int32_t t = t0 + tid;
-      uint32_t flag = 0, bt = 0;
-      int64_t q = 0;
-      int32_t ci = 0;
-      float pos[3] = {0.f, 0.f, 0.f};
-      if (t < total) {
+    for (int32_t t0 = 0; t0 < total; t0 += HNT * HGU) {
+      uint32_t flag[HGU], bt[HGU];
+      int32_t q[HGU], ci[HGU];
+      float pos[HGU][3];
+#pragma unroll
+      for (int u = 0; u < HGU; u++) {
+        const int32_t t = t0 + u * HNT + tid;
+        flag[u] = 0;
+        bt[u] = 0;
+        q[u] = 0;
         int lo = 0, hi = ncell;
         while (hi - lo > 1) {
           const int mid = (lo + hi) >> 1;
           if (off[mid] <= t) lo = mid; else hi = mid;
         }
-        ci = lo;
-        q = beg[ci] + (t - off[ci]);
-        const int32_t cc[3] = {p.cs0[0] + ci % ncx, p.cs0[1] + (ci / ncx) % ncy, p.cs0[2] + ci / (ncx * ncy)};
+        ci[u] = lo;
+        if (t < total) q[u] = (int32_t)(beg[lo] + (t - off[lo]));
+        const int32_t cc[3] = {p.cs0[0] + lo % ncx, p.cs0[1] + (lo / ncx) % ncy, p.cs0[2] + lo / (ncx * ncy)};
         int32_t td[3];
+#pragma unroll
         for (int d = 0; d < 3; d++) {
-          pos[d] = (float)((double)(CUBE_NCELL * (cc[d] - 1)) + (double)CUBE_NCELL * xoff(load_xu(xp, 3 * q + d, g.izipx), g.izipx));
-          td[d] = cc[d] >= 1 ? (cc[d] - 1) / c.nt : -1;
+          const uint32_t x = t < total ? load_xu(xp, 3 * (int64_t)q[u] + d, g.izipx) : 0u;
+          pos[u][d] = (float)((double)(CUBE_NCELL * (cc[d] - 1)) + (double)CUBE_NCELL * xoff(x, g.izipx));
+          td[d] = cc[d] >= 1 ? (cc[d] > c.nt ? 1 : 0) : -1;  // ncb <= nt: at most one tile away
         }
-        bt = 1u << (uint32_t)(((td[2] + 1) * 3 + (td[1] + 1)) * 3 + (td[0] + 1));
-        const float rr = norm3(pos[0] - p.h[0], pos[1] - p.h[1], pos[2] - p.h[2]);
-        if (rr < p.rs) {
-          const uint32_t tg = __hip_atomic_load(tag + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          flag = (tg & bt) ? 0u : 1u;
+        bt[u] = 1u << (uint32_t)(((td[2] + 1) * 3 + (td[1] + 1)) * 3 + (td[0] + 1));
+        flag[u] = t < total && norm3(pos[u][0] - p.h[0], pos[u][1] - p.h[1], pos[u][2] - p.h[2]) < p.rs;
+      }
+#pragma unroll
+      for (int u = 0; u < HGU; u++)
+        if (flag[u]) {
+          const uint32_t tg = __hip_atomic_load(tag + q[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          flag[u] = (tg & bt[u]) ? 0u : 1u;
+        }
+#pragma unroll
+      for (int u = 0; u < HGU; u++) {
+        const unsigned long long bal = __ballot(flag[u]);
+        if ((tid & 63) == 0) s_cnt[u * (HNT / 64) + (tid >> 6)] = __popcll(bal);
+      }
+      __syncthreads();
+      uint64_t base = n_odc;
+#pragma unroll
+      for (int u = 0; u < HGU; u++) {
+        const unsigned long long bal = __ballot(flag[u]);
+        uint64_t slot = base + (uint64_t)__popcll(bal & ((1ull << (tid & 63)) - 1));
+#pragma unroll
+        for (int w = 0; w < HNT / 64; w++) {
+          const int32_t n = s_cnt[u * (HNT / 64) + w];
+          if (w < (tid >> 6)) slot += (uint64_t)n;
+          base += (uint64_t)n;
+        }
+        if (flag[u] && (int64_t)slot < c.capn) {
+          ws.q[slot] = q[u];
+          ws.rk[slot] = crk[ci[u]];
+          ws.bit[slot] = bt[u];
+          ws.x[3 * slot] = pos[u][0];
+          ws.x[3 * slot + 1] = pos[u][1];
+          ws.x[3 * slot + 2] = pos[u][2];
         }
       }
-      uint64_t cnt;
-      const uint64_t pre = block_scan_excl(flag, wsum, cnt);
-      if (flag) {
-        const uint64_t slot = n_odc + pre;
-        if ((int64_t)slot < c.capn) {
-          ws.q[slot] = (int32_t)q;
-          ws.rk[slot] = crk[ci];
-          ws.bit[slot] = bt;
-          ws.x[3 * slot] = pos[0];
-          ws.x[3 * slot + 1] = pos[1];
-          ws.x[3 * slot + 2] = pos[2];
-        }
-      }
-      n_odc += cnt;
+      n_odc = base;
+      __syncthreads();
     }
     if ((int64_t)n_odc > c.capn) over = true;
     HRes out;
@@ -434,7 +501,8 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
       // particles within r_proxy in 2^-40 fixed point
       const int32_t D0 = p.nb[0] + 2, D1 = p.nb[1] + 2, D2 = p.nb[2] + 2;
       const int64_t gcn = (int64_t)D0 * D1 * D2;
-      for (int64_t i = tid; i < gcn; i += HNT) ws.grid[i] = 0ull;
+      for (int64_t i = tid; 2 * i < gcn; i += HNT) ((ulonglong2*)ws.grid)[i] = make_ulonglong2(0ull, 0ull);
+      wait_memory();
       __syncthreads();
       const float ng = c.newgrid;
       for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
@@ -461,16 +529,34 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
           atomicAdd(ws.grid + ((int64_t)a2 * D1 + a1) * D0 + a0, (unsigned long long)llrint((double)w[k] * HFIX));
         }
       }
-      __threadfence();
+      wait_memory();
       __syncthreads();
       // maxloc over indices 1.. (column-major first maximum; all zero -> 1,1,1)
+      // The grid was summed by atomics; device-scope loads, HGL of them in
+      // flight, see the sums whatever L1 holds.  A thread's column, row and
+      // plane advance by carries, without divisions.
       long long best = -1;
       int64_t bl = INT64_MAX;
-      for (int64_t i = tid; i < gcn; i += HNT) {
-        const int32_t a0 = (int32_t)(i % D0), a1 = (int32_t)((i / D0) % D1), a2 = (int32_t)(i / ((int64_t)D0 * D1));
-        if (a0 < 1 || a1 < 1 || a2 < 1) continue;
-        const long long v = (long long)__hip_atomic_load(ws.grid + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (v > best || (v == best && i < bl)) { best = v; bl = i; }
+      {
+        const int32_t s0 = HNT % D0, s1 = (HNT / D0) % D1, s2 = HNT / (D0 * D1);
+        int32_t a0 = tid % D0, a1 = (tid / D0) % D1, a2 = tid / (D0 * D1);
+        for (int64_t i0 = tid; i0 < gcn; i0 += HNT * HGL) {
+          long long v[HGL];
+#pragma unroll
+          for (int u = 0; u < HGL; u++) 
+            v[u] = i0 + u * HNT < gcn ? (long long)__hip_atomic_load(ws.grid + i0 + u * HNT, __ATOMIC_RELAXED,
+                                                                     __HIP_MEMORY_SCOPE_AGENT)
+                                      : -1;
+#pragma unroll
+          for (int u = 0; u < HGL; u++) {
+            if (v[u] > best && a0 >= 1 && a1 >= 1 && a2 >= 1) { best = v[u]; bl = i0 + u * HNT; }
+            a0 += s0;
+            a1 += s1;
+            a2 += s2;
+            if (a0 >= D0) { a0 -= D0; a1++; }
+            if (a1 >= D1) { a1 -= D1; a2++; }
+          }
+        }
       }
       const long long bmax = block_reduce<long long>(best, rbuf, [](long long a, long long b) { return a > b ? a : b; });
       const long long lmin = block_reduce<long long>(best == bmax ? (long long)bl : (long long)INT64_MAX, rbuf,
@@ -499,14 +585,40 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
       for (int d = 0; d < 3; d++) hf[d] = (float)p.fr0[d] + ng * hf[d];
       const float nftf = (float)c.nft;
       const int phys = hf[0] > 0 && hf[1] > 0 && hf[2] > 0 && hf[0] < nftf && hf[1] < nftf && hf[2] < nftf;
-      // radii from the refined centre, sorted with gathering order kept
-      // for equal radii: stable LSD radix sort, 2 bits per pass
+      // radii from the refined centre, sorted with gathering order kept for
+      // equal radii.  Lists that fit the LDS: a bitonic network on (radius,
+      // gathering index), whose keys are distinct, so it gives the stable
+      // order.  Longer ones: stable LSD radix sort in memory, 2 bits per pass.
+      int cur = 0;
+      if (n_odc <= HSORT) {
+        const int nn = (int)n_odc;
+        int np2 = 2;
+        while (np2 < nn) np2 <<= 1;
+        for (int m = tid; m < np2; m += HNT)
+          skey[m] = m < nn ? ((uint64_t)__float_as_uint(norm3(ws.x[3 * m] - hf[0], ws.x[3 * m + 1] - hf[1],
+                                                              ws.x[3 * m + 2] - hf[2])) << 32) | (uint32_t)m
+                           : ~0ull;
+        __syncthreads();
+        for (int k = 2; k <= np2; k <<= 1)
+          for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int t = tid; t < (np2 >> 1); t += HNT) {
+              const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i + j;
+              const uint64_t a = skey[i], b = skey[l];
+              if ((a > b) == ((i & k) == 0)) { skey[i] = b; skey[l] = a; }
+            }
+            __syncthreads();
+          }
+        for (int m = tid; m < nn; m += HNT) {
+          ws.key[0][m] = (uint32_t)(skey[m] >> 32);
+          ws.idx[0][m] = (uint32_t)skey[m];
+        }
+        __syncthreads();
+      } else {
       for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
         ws.key[0][m] = __float_as_uint(norm3(ws.x[3 * m] - hf[0], ws.x[3 * m + 1] - hf[1], ws.x[3 * m + 2] - hf[2]));
         ws.idx[0][m] = (uint32_t)m;
       }
       __syncthreads();
-      int cur = 0;
       for (int bitpos = 0; bitpos < 32; bitpos += 2) {
         // bucket totals; a pass whose digits are all equal keeps the order
         uint32_t bc[4];
@@ -541,6 +653,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
         }
         __syncthreads();
         cur ^= 1;
+      }
       }
       // first ii >= 2 with enclosed density below den_odc
       const float kd = 0.75f / PI_F;
@@ -588,9 +701,9 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
       }
     }
     if (tid == 0) res[P] = out;
-    __threadfence();
+    wait_memory();
     __syncthreads();
-    if (tid == 0) __hip_atomic_store(done + P, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(done + P, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -744,25 +857,56 @@ __global__ __launch_bounds__(HNT) void k_halo_cat1(Geo g, HalopCfg c, int64_t np
   }
 }
 
-// running totals in catalogue order: inertia (x), dx_mean -> q_mean
-__global__ void k_halo_seq1(int64_t nhalo, const HSums* __restrict__ sums, int32_t N, float* rec, float* qmean) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double run[6] = {0, 0, 0, 0, 0, 0};
-  float dxm[3] = {0.f, 0.f, 0.f};
+// running totals in catalogue order: inertia (x), dx_mean -> q_mean.  One
+// workgroup: chunks of HSEQ halos go through LDS, where one lane per running
+// sum adds them in order, so the chain waits on LDS and arithmetic alone
+// (from memory, one thread for all sums, it took 2.6 ms for 4641 halos).
+#define HSEQ 128
+__global__ __launch_bounds__(HNT) void k_halo_seq1(int64_t nhalo, const HSums* __restrict__ sums, int32_t N, float* rec,
+                                                   float* qmean) {
+  __shared__ HSums S[HSEQ];
+  __shared__ float tot[HSEQ][6], dx[HSEQ][3];
+  __shared__ double rn[HSEQ];
+  const int tid = threadIdx.x;
   const float nfr = (float)N;
-  for (int64_t hh = 0; hh < nhalo; hh++) {
-    const HSums S = sums[hh];
-    float* H = rec + 42 * hh;
-    for (int k = 0; k < 6; k++) run[k] += S.in[k];
-    const float sym[9] = {(float)run[0], (float)run[3], (float)run[5], (float)run[3], (float)run[1],
-                          (float)run[4], (float)run[5], (float)run[4], (float)run[2]};
-    for (int k = 0; k < 9; k++) H[18 + k] = sym[k];
-    for (int d = 0; d < 3; d++) {
-      dxm[d] = (float)(((double)dxm[d] + S.sdx[d]) / (double)S.nptemp);
-      const float qm = fmodulo(S.xw[d] + dxm[d], nfr);
-      H[27 + d] = qm;
-      qmean[3 * hh + d] = qm;
+  double run = 0;
+  float dxm = 0.f;
+  for (int64_t h0 = 0; h0 < nhalo; h0 += HSEQ) {
+    const int n = (int)min((int64_t)HSEQ, nhalo - h0);
+    const uint32_t* src = (const uint32_t*)(sums + h0);
+    for (int i = tid; i < n * (int)(sizeof(HSums) / 4); i += HNT) ((uint32_t*)S)[i] = src[i];
+    __syncthreads();
+    if (tid < n) rn[tid] = 1.0 / (double)S[tid].nptemp;
+    __syncthreads();
+    if (tid < 6) {
+      for (int i = 0; i < n; i++) {
+        run += S[i].in[tid];
+        tot[i][tid] = (float)run;
+      }
+    } else if (tid >= 64 && tid < 67) {
+      const int d = tid - 64;
+      for (int i = 0; i < n; i++) {
+        // (dxm + sdx)/nptemp: with the correctly rounded reciprocal the
+        // corrected estimate is the correctly rounded quotient (Markstein
+        // 1990), in three operations of the chain; 0 particles keep x*inf
+        const double x = (double)dxm + S[i].sdx[d], y = rn[i], b = (double)S[i].nptemp;
+        const double q = x * y;
+        const double r = fma(fma(-q, b, x), y, q);
+        dxm = (float)(r == r ? r : q);
+        dx[i][d] = dxm;
+      }
     }
+    __syncthreads();
+    for (int i = tid; i < n * 9; i += HNT) {
+      const int sym[9] = {0, 3, 5, 3, 1, 4, 5, 4, 2};
+      rec[42 * (h0 + i / 9) + 18 + i % 9] = tot[i / 9][sym[i % 9]];
+    }
+    for (int i = tid; i < n * 3; i += HNT) {
+      const float qm = fmodulo(S[i / 3].xw[i % 3] + dx[i / 3][i % 3], nfr);
+      rec[42 * (h0 + i / 3) + 27 + i % 3] = qm;
+      qmean[3 * h0 + i] = qm;
+    }
+    __syncthreads();
   }
 }
 
@@ -797,29 +941,78 @@ __global__ __launch_bounds__(HNT) void k_halo_cat2(HalopCfg c, int64_t npk, cons
     }
   }
 }
-__global__ void k_halo_seq2(int64_t nhalo, const double* __restrict__ iq, float* rec) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double run[6] = {0, 0, 0, 0, 0, 0};
-  for (int64_t hh = 0; hh < nhalo; hh++) {
-    for (int k = 0; k < 6; k++) run[k] += iq[6 * hh + k];
-    float* H = rec + 42 * hh;
-    const float sym[9] = {(float)run[0], (float)run[3], (float)run[5], (float)run[3], (float)run[1],
-                          (float)run[4], (float)run[5], (float)run[4], (float)run[2]};
-    for (int k = 0; k < 9; k++) H[30 + k] = sym[k];
+__global__ __launch_bounds__(HNT) void k_halo_seq2(int64_t nhalo, const double* __restrict__ iq, float* rec) {
+  __shared__ double S[HSEQ * 6];
+  __shared__ float tot[HSEQ][6];
+  const int tid = threadIdx.x;
+  double run = 0;
+  for (int64_t h0 = 0; h0 < nhalo; h0 += HSEQ) {
+    const int n = (int)min((int64_t)HSEQ, nhalo - h0);
+    for (int i = tid; i < n * 6; i += HNT) S[i] = iq[6 * h0 + i];
+    __syncthreads();
+    if (tid < 6)
+      for (int i = 0; i < n; i++) {
+        run += S[6 * i + tid];
+        tot[i][tid] = (float)run;
+      }
+    __syncthreads();
+    for (int i = tid; i < n * 9; i += HNT) {
+      const int sym[9] = {0, 3, 5, 3, 1, 4, 5, 4, 2};
+      rec[42 * (h0 + i / 9) + 30 + i % 9] = tot[i / 9][sym[i % 9]];
+    }
+    __syncthreads();
   }
 }
 
-// one device allocation carved into aligned pieces
-struct Arena {
-  char* base = nullptr;
-  size_t used = 0, cap = 0;
+// Workspace of one call, carved in aligned pieces out of the fine mesh's idle
+// buffers (R, W and X; the density is in S) and, for pieces that do not fit
+// there, allocated and freed with the call.  Sizes follow the peaks found
+// and the largest search box.  (With everything allocated per call at its
+// largest possible size, 13 GB at 256^3 particles, allocation took 360 of the
+// call's 376 ms; the whole call takes 3.9 ms now.)
+class Scratch {
+ public:
+  explicit Scratch(const Mesh& m) {
+    for (void* b : {m.R, m.W, m.X})
+      if (b) idle_.push_back({(char*)b, m.bytes_big()});
+  }
+  ~Scratch() {
+    for (void* p : own_) (void)hipFree(p);
+  }
+  // pieces of a part of the call, from what the whole call's has left; they
+  // go back when it ends
+  Scratch(const Scratch& whole) : idle_(whole.idle_) {}
+  Scratch& operator=(const Scratch&) = delete;
+  // n elements, or nullptr when the device has no memory for them
   template <typename T>
   T* take(size_t n) {
-    used = (used + 255) & ~(size_t)255;
-    T* p = (T*)(base + used);
-    used += n * sizeof(T);
-    return p;
+    const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+    for (Idle& i : idle_)
+      if (i.left >= bytes) {
+        T* p = (T*)i.at;
+        i.at += bytes;
+        i.left -= bytes;
+        return p;
+      }
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    own_.push_back(p);
+    return (T*)p;
   }
+  // what the largest idle piece still holds
+  size_t largest() const {
+    size_t m = 0;
+    for (const Idle& i : idle_) m = std::max(m, i.left);
+    return m;
+  }
+
+ private:
+  struct Idle { char* at; size_t left; };
+  std::vector<Idle> idle_;
+  std::vector<void*> own_;
 };
 
 }  // namespace
@@ -852,129 +1045,116 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   int rc = cic_halo_density(h, rho);
   if (rc) return rc;
 
-  // offset table
-  const int32_t R = hp->nc_halo_max, Dt = 2 * R + 1;
-  const int64_t ngen = (int64_t)Dt * Dt * Dt;
-  int64_t ntab = 0;
-  for (int64_t i = -R; i <= R; i++)
-    for (int64_t j = -R; j <= R; j++) {
-      const int64_t rem = (int64_t)R * R - i * i - j * j;
-      if (rem < 0) continue;
-      int64_t k = 0;
-      while ((k + 1) * (k + 1) <= rem) k++;
-      ntab += 2 * k + 1;
-    }
   const int64_t cand_cap = std::max<int64_t>(1 << 16, std::min<int64_t>(n3 / 8, 1 << 23));
   const int64_t mcap = std::max<int64_t>(1 << 16, np + (np >> 2));
-  // first arena: everything whose size does not depend on the peaks
-  size_t sort_tmp = 0;
-  {
-    size_t a = 0, b = 0;
-    HIP_TRY(h, hipcub::DeviceRadixSort::SortKeys(nullptr, a, (uint64_t*)nullptr, (uint64_t*)nullptr, (int)ngen, 0, 41, st));
-    HIP_TRY(h, hipcub::DeviceRadixSort::SortPairs(nullptr, b, (uint64_t*)nullptr, (uint64_t*)nullptr, (int32_t*)nullptr,
-                                                  (int32_t*)nullptr, (int)cand_cap, 0, 43, st));
-    sort_tmp = std::max(a, b);
-  }
-  Arena A;
-  A.cap = 2 * sizeof(uint64_t) * ngen + sort_tmp + cand_cap * (sizeof(int4) + 4 * sizeof(int32_t) + 7 * sizeof(float) +
-                                                               2 * sizeof(uint64_t) + sizeof(HPk) + sizeof(HRes) + 32) +
-          (size_t)np * 4 + (size_t)mcap * 12 + (1 << 20);
-  Arena B;
-  char* wsbase = nullptr;
-  auto cleanup = [&]() {
-    (void)hipFree(A.base);
-    (void)hipFree(B.base);
-    (void)hipFree(wsbase);
-  };
-  HIP_TRY(h, hipMalloc(&A.base, A.cap));
-  uint64_t* tabk = A.take<uint64_t>(ngen);
-  uint64_t* tabs = A.take<uint64_t>(ngen);
-  void* tmp = A.take<char>(sort_tmp);
-  int4* cand = A.take<int4>(cand_cap);
-  uint32_t* ctr = A.take<uint32_t>(16);  // 0 ncand, 1 nvalid, 2 next, 3 errf
-  unsigned long long* uctr = A.take<unsigned long long>(4);  // 0 members, 1 grid max
-  int32_t* vidx = A.take<int32_t>(cand_cap);
-  float* cden = A.take<float>(cand_cap);
-  float* cmesh = A.take<float>(cand_cap);
-  float* chpos = A.take<float>(3 * cand_cap);
-  uint32_t* cloop = A.take<uint32_t>(cand_cap);
-  int32_t* perm0 = A.take<int32_t>(cand_cap);
-  int32_t* perm1 = A.take<int32_t>(cand_cap);
-  uint64_t* k0 = A.take<uint64_t>(cand_cap);
-  uint64_t* k1 = A.take<uint64_t>(cand_cap);
-  uint32_t* tag = A.take<uint32_t>(np);
-  int32_t* mq = A.take<int32_t>(mcap);
-  int32_t* mrk = A.take<int32_t>(mcap);
-  uint32_t* mbit = A.take<uint32_t>(mcap);
-  if (A.used > A.cap) { cleanup(); return cube_fail(h, CUBE_ERR_ARG, "halo arena sizing"); }
-#define HTRY(call)                                                                          \
-  do {                                                                                      \
-    hipError_t e_ = (call);                                                                 \
-    if (e_ != hipSuccess) {                                                                 \
-      cleanup();                                                                            \
-      return cube_fail(h, CUBE_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));     \
-    }                                                                                       \
-  } while (0)
+  // the workspaces come from the fine mesh's idle buffers as far as they fit
+  Scratch A(h->fine);
+#define HTRY(call) HIP_TRY(h, call)
+#define HTAKE(T, var, n)                                                                               \
+  T* var = A.take<T>(n);                                                                               \
+  if (!var) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for " #var " (%lld entries)", (long long)(n))
+  HTAKE(uint32_t, ctr, 16);                  // 0 ncand, 1 nvalid, 2 next, 3 errf, 4 walks longer than the table
+  HTAKE(unsigned long long, uctr, 4);        // 0 members, 1 grid max, 2 largest search box
+  HTAKE(int4, cand, cand_cap);
   HTRY(hipMemsetAsync(ctr, 0, 16 * sizeof(uint32_t), st));
   HTRY(hipMemsetAsync(uctr, 0, 4 * sizeof(unsigned long long), st));
-  HTRY(hipMemsetAsync(tag, 0, (size_t)np * 4, st));
-  k_hoff_gen<<<4096, 256, 0, st>>>(R, tabk);
-  {
-    size_t tb = sort_tmp;
-    HTRY(hipcub::DeviceRadixSort::SortKeys(tmp, tb, tabk, tabs, (int)ngen, 0, 41, st));
-  }
   // 2. peaks
   k_halo_peaks<<<8192, 256, 0, st>>>(rho, c, ctr + 0, cand_cap, cand);
   HTRY(hipGetLastError());
-  uint32_t hc[4];
+  uint32_t hc[5];
   HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
   HTRY(hipStreamSynchronize(st));
-  if ((int64_t)hc[0] > cand_cap) {
-    cleanup();
+  if ((int64_t)hc[0] > cand_cap)
     return cube_fail(h, CUBE_ERR_CAPACITY, "halo finder: %u candidate peaks exceed the table (%lld)", hc[0], (long long)cand_cap);
-  }
   const int64_t ncand = hc[0];
-  // 3. mesh walk
-  if (ncand > 0)
-    k_halo_walk<<<(unsigned)((ncand + 127) / 128), 128, 0, st>>>(rho, c, cand, ncand, tabs, ntab, R, ctr + 1, vidx, cden,
-                                                                  cmesh, chpos, cloop);
-  HTRY(hipGetLastError());
-  HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
-  HTRY(hipStreamSynchronize(st));
+  HTAKE(int32_t, vidx, ncand);
+  HTAKE(float, cden, ncand);
+  HTAKE(float, cmesh, ncand);
+  HTAKE(float, chpos, 3 * ncand);
+  HTAKE(uint32_t, cloop, ncand);
+  // 3. mesh walk over the radius-sorted offset table.  A table of offsets up
+  // to 32 cells (275 thousand keys) ends nearly every walk; it is a prefix of
+  // the table up to nc_halo_max (17 million keys at 128, 1.5 ms to sort), which is
+  // built only if a walk needs more.
+  if (ncand > 0) {
+    const int32_t rmax = hp->nc_halo_max;
+    for (int32_t R = std::min(rmax, 32);; R = rmax) {
+      const int64_t Dt = 2 * R + 1, ngen = Dt * Dt * Dt;
+      int64_t ntab = 0;
+      for (int64_t i = -R; i <= R; i++)
+        for (int64_t j = -R; j <= R; j++) {
+          const int64_t rem = (int64_t)R * R - i * i - j * j;
+          if (rem < 0) continue;
+          int64_t k = (int64_t)std::sqrt((double)rem);
+          while (k * k > rem) k--;
+          while ((k + 1) * (k + 1) <= rem) k++;
+          ntab += 2 * k + 1;
+        }
+      Scratch B(A);
+      size_t tb = 0;
+      HTRY(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int)ngen, 0, 41, st));
+      uint64_t* tabk = B.take<uint64_t>(ngen);
+      uint64_t* tabs = B.take<uint64_t>(ngen);
+      void* tmp = B.take<char>(tb);
+      if (!tabk || !tabs || !tmp) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for the offset table");
+      k_hoff_gen<<<(unsigned)std::min<int64_t>((ngen + 255) / 256, 4096), 256, 0, st>>>(R, tabk);
+      HTRY(hipcub::DeviceRadixSort::SortKeys(tmp, tb, tabk, tabs, (int)ngen, 0, 41, st));
+      k_halo_walk<<<(unsigned)((ncand + 127) / 128), 128, 0, st>>>(rho, c, cand, ncand, tabs, ntab, R, ctr + 1, vidx, cden,
+                                                                    cmesh, chpos, cloop, R < rmax ? ctr + 4 : nullptr);
+      HTRY(hipGetLastError());
+      HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
+      HTRY(hipStreamSynchronize(st));
+      if (hc[4] == 0) break;
+      HTRY(hipMemsetAsync(ctr + 1, 0, sizeof(uint32_t), st));  // walked again with the whole table
+      HTRY(hipMemsetAsync(ctr + 4, 0, sizeof(uint32_t), st));
+    }
+  }
   const int64_t npk = hc[1];
   out->npeaks = ncand;
   out->nprocessed = npk;
   out->nhalo = 0;
   out->npid_words = 0;
-  if (npk == 0) { cleanup(); return 0; }
+  if (npk == 0) return 0;
+  HTAKE(int32_t, perm0, npk);
   // 4. order: stable by loop index, then by (tile order, density descending)
   {
-    size_t tb = sort_tmp;
+    size_t tb = 0;
+    HTRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int32_t*)nullptr,
+                                            (int32_t*)nullptr, (int)npk, 0, 43, st));
+    Scratch B(A);
+    int32_t* perm1 = B.take<int32_t>(npk);
+    uint64_t* k0 = B.take<uint64_t>(npk);
+    uint64_t* k1 = B.take<uint64_t>(npk);
+    void* tmp = B.take<char>(tb);
+    if (!perm1 || !k0 || !k1 || !tmp) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for the peak order");
     k_halo_key_lo<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, cloop, k0, perm0);
-    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, perm0, perm1, (int)npk, 0, 32, st));
+    size_t tu = tb;
+    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm0, perm1, (int)npk, 0, 32, st));
     const int32_t ntiles = c.nnt * c.nnt * c.nnt;
     k_halo_key_hi<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, perm1, vidx, cand, cden, ntiles, k0);
-    tb = sort_tmp;
-    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, perm1, perm0, (int)npk, 0, 43, st));
+    tu = tb;
+    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm1, perm0, (int)npk, 0, 43, st));
   }
   // perm0[s] = valid slot of the s-th peak in processing order
   const float gs = std::max(2.0f * (float)(c.ncb - 1) * (float)CUBE_NCELL, 1.0f);
   const int32_t nbin = (int32_t)std::ceil((c.nft + 4.0f * CUBE_NCELL) / gs) + 1;
   const int64_t nbins = (int64_t)c.nnt * c.nnt * c.nnt * nbin * nbin * nbin;
-  B.cap = (size_t)npk * (sizeof(HPk) + sizeof(HRes) + 4 * sizeof(int32_t) + 2 * sizeof(int64_t) + 64) +
-          (size_t)(nbins + 1) * (sizeof(int64_t) + 2 * sizeof(uint32_t)) + (1 << 20);
-  HTRY(hipMalloc(&B.base, B.cap));
-  HPk* pk = B.take<HPk>(npk);
-  HRes* res = B.take<HRes>(npk);
-  int32_t* done = B.take<int32_t>(npk);
-  int32_t* binlist = B.take<int32_t>(npk);
-  uint32_t* bincnt = B.take<uint32_t>(nbins + 1);
-  uint32_t* binfill = B.take<uint32_t>(nbins + 1);
-  int64_t* binoff = B.take<int64_t>(nbins + 1);
-  int32_t* is_halo = B.take<int32_t>(npk);
-  int32_t* wcount = B.take<int32_t>(npk);
-  int64_t* hidx = B.take<int64_t>(npk + 1);
-  int64_t* woff = B.take<int64_t>(npk + 1);
+  HTAKE(HPk, pk, npk);
+  HTAKE(HRes, res, npk);
+  HTAKE(int32_t, done, npk);
+  HTAKE(int32_t, binlist, npk);
+  HTAKE(uint32_t, bincnt, nbins + 1);
+  HTAKE(uint32_t, binfill, nbins + 1);
+  HTAKE(int64_t, binoff, nbins + 1);
+  HTAKE(int32_t, is_halo, npk);
+  HTAKE(int32_t, wcount, npk);
+  HTAKE(int64_t, hidx, npk + 1);
+  HTAKE(int64_t, woff, npk + 1);
+  HTAKE(uint32_t, tag, np);
+  HTAKE(int32_t, mq, mcap);
+  HTAKE(int32_t, mrk, mcap);
+  HTAKE(uint32_t, mbit, mcap);
+  HTRY(hipMemsetAsync(tag, 0, (size_t)np * 4, st));
   HTRY(hipMemsetAsync(done, 0, sizeof(int32_t) * npk, st));
   HTRY(hipMemsetAsync(bincnt, 0, sizeof(uint32_t) * (nbins + 1), st));
   HTRY(hipMemsetAsync(binfill, 0, sizeof(uint32_t) * (nbins + 1), st));
@@ -983,94 +1163,94 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   HTRY(hipGetLastError());
   {
     const int r2 = scan_counts(h, (const int32_t*)bincnt, nbins, binoff);
-    if (r2) { cleanup(); return r2; }
+    if (r2) return r2;
   }
   k_halo_bin_fill<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, pk, binoff, binfill, binlist);
+  k_halo_box_count<<<(unsigned)((npk + HNT / 64 - 1) / (HNT / 64)), HNT, 0, st>>>(g, c, npk, pk, h->cstart, uctr + 2);
   HTRY(hipGetLastError());
-  unsigned long long gmax = 0;
+  unsigned long long um[2] = {0, 0};  // largest refined grid, largest search box
   HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
-  HTRY(hipMemcpyAsync(&gmax, uctr + 1, sizeof(gmax), hipMemcpyDeviceToHost, st));
+  HTRY(hipMemcpyAsync(um, uctr + 1, sizeof(um), hipMemcpyDeviceToHost, st));
   HTRY(hipStreamSynchronize(st));
-  if (hc[3] & 1u) { cleanup(); return cube_fail(h, CUBE_ERR_CHECK, "halo search box beyond the tile buffer (halofind.f90:245-252)"); }
-  if (hc[3] & 2u) { cleanup(); return cube_fail(h, CUBE_ERR_CHECK, "newbox>newbox_max (halofind.f90:259)"); }
-  if (hc[3] & 4u) { cleanup(); return cube_fail(h, CUBE_ERR_CAPACITY, "halo search box holds more than %d cells", HMAXCELLS); }
-  // 5. persistent processing: workgroup scratch sized for the largest
-  // refined grid and the search-list capacity
+  if (hc[3] & 1u) return cube_fail(h, CUBE_ERR_CHECK, "halo search box beyond the tile buffer (halofind.f90:245-252)");
+  if (hc[3] & 2u) return cube_fail(h, CUBE_ERR_CHECK, "newbox>newbox_max (halofind.f90:259)");
+  if (hc[3] & 4u) return cube_fail(h, CUBE_ERR_CAPACITY, "halo search box holds more than %d cells", HMAXCELLS);
+  // 5. persistent processing: workgroup scratch sized for the largest refined
+  // grid and the longest search list, which is bounded by the search-list
+  // capacity and by the particles of the largest search box
   int dev = 0, ncu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   c.capn = std::min<int64_t>(hp->max_halo_np, std::max<int64_t>(4096, std::min<int64_t>(np, 1 << 20)));
-  c.gcap = (int64_t)gmax;
+  c.capn = std::min<int64_t>(c.capn, std::max<int64_t>((int64_t)um[1], 64));
+  const int64_t gmax = (int64_t)um[0];
+  c.gcap = gmax;
   c.mcap = mcap;
-  const int64_t wsbytes = ((int64_t)c.capn * 40 + 512 + (int64_t)gmax * 8 + 255) & ~(int64_t)255;
-  size_t freeb = 0, totb = 0;
-  (void)hipMemGetInfo(&freeb, &totb);
-  int64_t nwg = std::min<int64_t>(std::max(ncu, 1), npk);
-  const int64_t budget = (int64_t)(freeb / 2);
-  if (nwg * wsbytes > budget) nwg = std::max<int64_t>(1, budget / wsbytes);
-  HTRY(hipMalloc(&wsbase, (size_t)(nwg * wsbytes)));
+  const int64_t wsbytes = ((int64_t)c.capn * 40 + 512 + gmax * 8 + 255) & ~(int64_t)255;
+  // four workgroups fit a CU (32 KB of LDS each); a smaller number, down to
+  // one workgroup, when the scratch would not fit an idle buffer or half of
+  // the free memory
+  int64_t nwg = std::min<int64_t>(4 * std::max(ncu, 1), npk);
+  int64_t fit = (int64_t)A.largest() / wsbytes;
+  if (fit < std::min<int64_t>(nwg, std::max(ncu, 1))) {
+    size_t freeb = 0, totb = 0;
+    (void)hipMemGetInfo(&freeb, &totb);
+    fit = std::max<int64_t>(fit, (int64_t)(freeb / 2) / wsbytes);
+    nwg = std::min<int64_t>(nwg, std::max(ncu, 1));
+  }
+  nwg = std::max<int64_t>(1, std::min(nwg, fit));
+  HTAKE(char, wsbase, nwg * wsbytes);
   const double* vdt = vtab_for(h, vcoef(h->sigma_vi));
   k_halo_process<<<(unsigned)nwg, HNT, 0, st>>>(g, c, h->xp, h->cstart, npk, pk, nbin, binoff, binlist, tag, done, ctr + 2,
                                                  res, mq, mrk, mbit, uctr + 0, ctr + 3, wsbase, wsbytes);
   hipError_t pe = hipGetLastError();
   if (pe == hipSuccess) pe = hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st);
   if (pe == hipSuccess) pe = hipStreamSynchronize(st);
-  if (pe != hipSuccess) { cleanup(); return cube_fail(h, CUBE_ERR_HIP, "halo processing failed: %s", hipGetErrorString(pe)); }
-  if (hc[3] & 8u) { cleanup(); return cube_fail(h, CUBE_ERR_CHECK, "halo finder: dependency wait exceeded its bound"); }
-  if (hc[3] & 16u) { cleanup(); return cube_fail(h, CUBE_ERR_CAPACITY, "halo search list longer than %lld particles", (long long)c.capn); }
-  if (hc[3] & 32u) { cleanup(); return cube_fail(h, CUBE_ERR_CHECK, "refined grid index outside 0..newbox+1"); }
-  if (hc[3] & 64u) { cleanup(); return cube_fail(h, CUBE_ERR_CAPACITY, "halo member list capacity"); }
+  if (pe != hipSuccess) return cube_fail(h, CUBE_ERR_HIP, "halo processing failed: %s", hipGetErrorString(pe));
+  if (hc[3] & 8u) return cube_fail(h, CUBE_ERR_CHECK, "halo finder: dependency wait exceeded its bound");
+  if (hc[3] & 16u) return cube_fail(h, CUBE_ERR_CAPACITY, "halo search list longer than %lld particles", (long long)c.capn);
+  if (hc[3] & 32u) return cube_fail(h, CUBE_ERR_CHECK, "refined grid index outside 0..newbox+1");
+  if (hc[3] & 64u) return cube_fail(h, CUBE_ERR_CAPACITY, "halo member list capacity");
   // 6. catalogue
   k_halo_flags<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, res, c.min_np, is_halo, wcount);
-  if ((rc = scan_counts(h, is_halo, npk, hidx)) || (rc = scan_counts(h, wcount, npk, woff))) { cleanup(); return rc; }
+  if ((rc = scan_counts(h, is_halo, npk, hidx)) || (rc = scan_counts(h, wcount, npk, woff))) return rc;
   int64_t nh = 0, nw = 0;
   HTRY(hipMemcpyAsync(&nh, hidx + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   HTRY(hipMemcpyAsync(&nw, woff + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   HTRY(hipStreamSynchronize(st));
-  if (nh > out->max_halos || nw > out->max_pid_words) {
-    cleanup();
+  if (nh > out->max_halos || nw > out->max_pid_words)
     return cube_fail(h, CUBE_ERR_CAPACITY, "halo catalogue: %lld halos / %lld pid words exceed the buffers", (long long)nh,
                      (long long)nw);
-  }
   out->nhalo = nh;
   out->npid_words = nw;
   if (nh > 0) {
-    float* rec = nullptr;
-    HSums* sums = nullptr;
-    float* qmean = nullptr;
-    double* iq = nullptr;
-    int32_t* words = nullptr;
+    HTAKE(float, rec, 42 * nh);
+    HTAKE(HSums, sums, nh);
+    HTAKE(float, qmean, 3 * nh);
+    HTAKE(double, iq, 6 * nh);
+    HTAKE(int32_t, words, nw);
     int16_t* hidd = nullptr;
-    hipError_t e = hipMalloc(&rec, sizeof(float) * 42 * nh);
-    if (e == hipSuccess) e = hipMalloc(&sums, sizeof(HSums) * nh);
-    if (e == hipSuccess) e = hipMalloc(&qmean, sizeof(float) * 3 * nh);
-    if (e == hipSuccess) e = hipMalloc(&iq, sizeof(double) * 6 * nh);
-    if (e == hipSuccess) e = hipMalloc(&words, sizeof(int32_t) * nw);
-    if (e == hipSuccess && out->hid && out->nhid > 0) {
-      e = hipMalloc(&hidd, sizeof(int16_t) * out->nhid);
-      if (e == hipSuccess) e = hipMemsetAsync(hidd, 0, sizeof(int16_t) * out->nhid, st);
+    if (out->hid && out->nhid > 0) {
+      hidd = A.take<int16_t>(out->nhid);
+      if (!hidd) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for hid");
+      HTRY(hipMemsetAsync(hidd, 0, sizeof(int16_t) * out->nhid, st));
     }
-    if (e == hipSuccess) {
-      const unsigned nb1 = (unsigned)std::min<int64_t>(npk, 65535);
-      k_halo_cat1<<<nb1, HNT, 0, st>>>(g, c, npk, pk, res, is_halo, hidx, woff, mq, mrk, mbit, h->xp, h->vp, h->vfield, vdt,
-                                       h->pid, hp->box, hp->h0, hp->a, hp->vsim2phys, hp->los_centre[0], hp->los_centre[1],
-                                       hp->los_centre[2], rec, sums, words, hidd, hidd ? out->nhid : 0);
-      k_halo_seq1<<<1, 1, 0, st>>>(nh, sums, c.N, rec, qmean);
-      k_halo_cat2<<<nb1, HNT, 0, st>>>(c, npk, res, is_halo, hidx, mq, h->pid, qmean, iq);
-      k_halo_seq2<<<1, 1, 0, st>>>(nh, iq, rec);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(out->halos, rec, sizeof(float) * 42 * nh, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(out->pid_words, words, sizeof(int32_t) * nw, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && hidd) e = hipMemcpyAsync(out->hid, hidd, sizeof(int16_t) * out->nhid, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(rec); (void)hipFree(sums); (void)hipFree(qmean); (void)hipFree(iq); (void)hipFree(words);
-    if (hidd) (void)hipFree(hidd);
-    if (e != hipSuccess) { cleanup(); return cube_fail(h, CUBE_ERR_HIP, "halo catalogue failed: %s", hipGetErrorString(e)); }
+    const unsigned nb1 = (unsigned)std::min<int64_t>(npk, 65535);
+    k_halo_cat1<<<nb1, HNT, 0, st>>>(g, c, npk, pk, res, is_halo, hidx, woff, mq, mrk, mbit, h->xp, h->vp, h->vfield, vdt,
+                                     h->pid, hp->box, hp->h0, hp->a, hp->vsim2phys, hp->los_centre[0], hp->los_centre[1],
+                                     hp->los_centre[2], rec, sums, words, hidd, hidd ? out->nhid : 0);
+    k_halo_seq1<<<1, HNT, 0, st>>>(nh, sums, c.N, rec, qmean);
+    k_halo_cat2<<<nb1, HNT, 0, st>>>(c, npk, res, is_halo, hidx, mq, h->pid, qmean, iq);
+    k_halo_seq2<<<1, HNT, 0, st>>>(nh, iq, rec);
+    HTRY(hipGetLastError());
+    HTRY(hipMemcpyAsync(out->halos, rec, sizeof(float) * 42 * nh, hipMemcpyDeviceToHost, st));
+    HTRY(hipMemcpyAsync(out->pid_words, words, sizeof(int32_t) * nw, hipMemcpyDeviceToHost, st));
+    if (hidd) HTRY(hipMemcpyAsync(out->hid, hidd, sizeof(int16_t) * out->nhid, hipMemcpyDeviceToHost, st));
+    HTRY(hipStreamSynchronize(st));
   } else if (out->hid && out->nhid > 0) {
     memset(out->hid, 0, sizeof(int16_t) * out->nhid);
   }
-  cleanup();
   return 0;
 #undef HTRY
+#undef HTAKE
 }
