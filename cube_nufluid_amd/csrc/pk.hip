@@ -15,41 +15,82 @@
 // sinc = prod_d sin(pi k_d/ng)/(pi k_d/ng).
 #include "cube_internal.hpp"
 #include <math.h>
+#include <algorithm>
 #include <mutex>
+#include <vector>
 
 #define PK_NT 256
 #define PK_MAXBIN 2048
 
+// One wavefront per (ky, kz) row, PK_U consecutive kx a lane and pass.  The
+// window factors sin(x)/x come from a table in LDS (N/2+1 of them instead of
+// three sines per mode), row and plane are uniform, and a lane adds its
+// modes to the bin sums only where the bin changes: neighbouring modes share
+// bins, and one atomic per mode met on the same addresses.  65 M modes
+// (512^3 mesh) take 0.29 instead of 1.04 ms.
+#define PK_U 4
 template <typename T>
-__global__ __launch_bounds__(PK_NT) void k_pk_bin(const cpx<T>* __restrict__ c, int64_t N, double inv_norm, int nbin,
-                                                  double* bins) {
-  __shared__ double sb[3 * (PK_MAXBIN + 1)];
+__global__ __launch_bounds__(PK_NT) void k_pk_bin(const cpx<T>* __restrict__ c, int N, double inv_norm, int nbin, double* bins) {
+  extern __shared__ double win[];  // N/2+1 window factors, then 3 (nbin+1) bin sums
+  const int H = N / 2 + 1, nyq = N / 2;
+  double* const sb = win + H;
   for (int i = threadIdx.x; i < 3 * (nbin + 1); i += PK_NT) sb[i] = 0;
+  for (int i = threadIdx.x; i < H; i += PK_NT) {
+    const double x = M_PI * (double)i / (double)N;
+    win[i] = i ? sin(x) / x : 1.0;
+  }
   __syncthreads();
-  const int64_t H = N / 2 + 1, tot = H * N * N, nyq = N / 2;
-  for (int64_t i = (int64_t)blockIdx.x * PK_NT + threadIdx.x; i < tot; i += (int64_t)gridDim.x * PK_NT) {
-    const int64_t kx = i % H, ky = (i / H) % N, kz = i / (H * N);
-    if (kx == 0 && ky == 0 && kz == 0) continue;
-    const bool edge = kx == 0 || kx == nyq;
-    if (edge && ky > nyq) continue;
-    if (edge && (ky == 0 || ky == nyq) && kz > nyq) continue;
-    const int64_t q[3] = {(kx + nyq) % N - nyq, (ky + nyq) % N - nyq, (kz + nyq) % N - nyq};
-    const float kr = sqrtf((float)(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]));
-    const int ib = (int)floorf(kr + 0.5f);
-    if (ib > nbin) continue;
-    double sinc = 1;
-    for (int d = 0; d < 3; d++)
-      if (q[d]) {
-        const double x = M_PI * (double)q[d] / (double)N;
-        sinc *= sin(x) / x;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int row = blockIdx.x * (PK_NT / 64) + wv; row < N * N; row += gridDim.x * (PK_NT / 64)) {
+    const int ky = row % N, kz = row / N;
+    const int qy = ky < nyq ? ky : ky - N, qz = kz < nyq ? kz : kz - N;
+    // on the kx = 0 and nyq planes the conjugate duplicates are skipped
+    const bool dup = ky > nyq || ((ky == 0 || ky == nyq) && kz > nyq);
+    const int q2 = qy * qy + qz * qz;
+    const double wy = win[abs(qy)], wz = win[abs(qz)];
+    const cpx<T>* src = c + (int64_t)row * H;
+    for (int k0 = 0; k0 < H; k0 += 64 * PK_U) {
+      cpx<T> v[PK_U];
+#pragma unroll
+      for (int u = 0; u < PK_U; u++) {
+        const int kx = k0 + lane * PK_U + u;
+        v[u] = kx < H ? src[kx] : cpx<T>{0, 0};
       }
-    const cpx<T> v = c[i];
-    const double re = (double)v.x * inv_norm, im = (double)v.y * inv_norm;
-    const double s2 = sinc * sinc;
-    const double amp = (re * re + im * im) / (s2 * s2) * 4.0 * M_PI * (double)kr * (double)kr * (double)kr;
-    atomicAdd(&sb[3 * ib], 1.0);
-    atomicAdd(&sb[3 * ib + 1], (double)kr);
-    atomicAdd(&sb[3 * ib + 2], amp);
+      int bin = -1;
+      double sk = 0, sa = 0, sn = 0;
+#pragma unroll
+      for (int u = 0; u < PK_U; u++) {
+        const int kx = k0 + lane * PK_U + u;
+        bool ok = kx < H && !((kx == 0 || kx == nyq) && dup) && (kx | q2) != 0;
+        const int qx = kx < nyq ? kx : kx - N;
+        const float kr = sqrtf((float)(qx * qx + q2));
+        const int ib = (int)floorf(kr + 0.5f);
+        ok = ok && ib <= nbin;
+        if (ok) {
+          if (ib != bin) {
+            if (bin >= 0) {
+              atomicAdd(&sb[3 * bin], sn);
+              atomicAdd(&sb[3 * bin + 1], sk);
+              atomicAdd(&sb[3 * bin + 2], sa);
+            }
+            bin = ib;
+            sk = sa = sn = 0;
+          }
+          const double sinc = win[abs(qx)] * wy * wz;
+          const double re = (double)v[u].x * inv_norm, im = (double)v[u].y * inv_norm;
+          const double s2 = sinc * sinc;
+          sa += (re * re + im * im) / (s2 * s2) * 4.0 * M_PI * (double)kr * (double)kr * (double)kr;
+          sk += (double)kr;
+          sn += 1.0;
+        }
+      }
+      if (bin >= 0) {
+        atomicAdd(&sb[3 * bin], sn);
+        atomicAdd(&sb[3 * bin + 1], sk);
+        atomicAdd(&sb[3 * bin + 2], sa);
+      }
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < 3 * (nbin + 1); i += PK_NT)
@@ -103,19 +144,24 @@ static int pk_run(cube_handle* h, int nbin, double* modes, double* ksum, double*
   HIP_TRY(h, hipGetLastError());
   const double mean = mass / ((double)N * N * N);
   const double inv_norm = 1.0 / ((double)N * N * N * mean);
-  const int64_t tot = (N / 2 + 1) * N * N;
-  const unsigned grid = (unsigned)std::min<int64_t>((tot + PK_NT - 1) / PK_NT, 4096);
+  // a workgroup clears and folds its LDS bins once, so there are no more of
+  // them than fill the GPU
+  const unsigned grid = (unsigned)std::min<int64_t>((N * N + PK_NT / 64 - 1) / (PK_NT / 64), 2048);
+  const size_t lds = sizeof(double) * (N / 2 + 1 + nv);
   if (h->prec == 4)
-    k_pk_bin<float><<<grid, PK_NT, 0, h->stream>>>((const cpx<float>*)h->fine.R, N, inv_norm, nbin, bins);
+    k_pk_bin<float><<<grid, PK_NT, lds, h->stream>>>((const cpx<float>*)h->fine.R, (int)N, inv_norm, nbin, bins);
   else
-    k_pk_bin<double><<<grid, PK_NT, 0, h->stream>>>((const cpx<double>*)h->fine.R, N, inv_norm, nbin, bins);
+    k_pk_bin<double><<<grid, PK_NT, lds, h->stream>>>((const cpx<double>*)h->fine.R, (int)N, inv_norm, nbin, bins);
   HIP_TRY(h, hipGetLastError());
-  // the reference reports bins 1..nbin (xip=xi(:,1:)); field f of bin b is bins[3b+f]
+  // one copy of all bins (a strided copy per field moves its rows one by
+  // one: 9 ms at 443 bins).  The reference reports bins 1..nbin (xip=xi(:,1:));
+  // field f of bin b is bins[3b+f].
+  std::vector<double> hb(nv);
+  HIP_TRY(h, hipMemcpyAsync(hb.data(), bins, sizeof(double) * nv, hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(h, hipStreamSynchronize(h->stream));
   double* dst[3] = {modes, ksum, d2sum};
   for (int f = 0; f < 3; f++)
-    HIP_TRY(h, hipMemcpy2DAsync(dst[f], sizeof(double), bins + 3 + f, 3 * sizeof(double), sizeof(double), (size_t)nbin,
-                                hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(h, hipStreamSynchronize(h->stream));
+    for (int b = 1; b <= nbin; b++) dst[f][b - 1] = hb[3 * b + f];
   return CUBE_OK;
 }
 
