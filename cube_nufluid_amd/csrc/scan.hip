@@ -86,13 +86,23 @@ int scan_counts(cube_handle* h, const int32_t* cnt, int64_t n, int64_t* cstart) 
   return 0;
 }
 
+#define RF_U 16
 // Sum nparts x nfields doubles (field-major within a part) in a fixed order:
 // one workgroup per field, fixed stride partition, fixed tree.
 __global__ void k_reduce_fields(const double* part, int64_t nparts, int nfields, double* out) {
   __shared__ double tmp[SCAN_NT];
   int f = blockIdx.x;
   double s = 0;
-  for (int64_t i = threadIdx.x; i < nparts; i += SCAN_NT) s += part[i * nfields + f];
+  // RF_U loads in flight, added in order: one at a time, 32768 partials take
+  // 46 us of memory latency
+  for (int64_t i0 = threadIdx.x; i0 < nparts; i0 += SCAN_NT * RF_U) {
+    double v[RF_U];
+#pragma unroll
+    for (int u = 0; u < RF_U; u++) v[u] = i0 + u * SCAN_NT < nparts ? part[(i0 + u * SCAN_NT) * nfields + f] : 0.0;
+#pragma unroll
+    for (int u = 0; u < RF_U; u++)
+      if (i0 + u * SCAN_NT < nparts) s += v[u];
+  }
   tmp[threadIdx.x] = s;
   __syncthreads();
   for (int off = SCAN_NT / 2; off > 0; off >>= 1) {
