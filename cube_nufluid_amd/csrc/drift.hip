@@ -27,7 +27,6 @@
 #include <algorithm>
 
 #define DR_NT 256
-#define DR_CH 256
 #define DMAX 7
 #define DR_LBITS 20  // particles per source cell < 2^20 (sort key field)
 #define DR_RBITS 27  // coarse cells < 2^27 (nc <= 512)
@@ -54,6 +53,10 @@ __device__ __forceinline__ WaveRun wave_run(int64_t key) {
 }
 
 #define DP_SL 2
+// Both per-particle passes take DR_CH source cells a workgroup: 256, or fewer
+// where that leaves CUs idle (drift_cells: at 16^3 cells 16 workgroups of 256
+// took 37 us, 128 of 32 take 17).
+template <int DR_CH>
 __global__ __launch_bounds__(DR_NT) void k_drift_pass1(Geo g, const void* __restrict__ xp, const void* __restrict__ vp,
                                                        const int64_t* __restrict__ cstart, int64_t n3c,
                                                        const float* __restrict__ vfield, float dt_mid, double c_old,
@@ -181,9 +184,9 @@ __device__ __forceinline__ uint64_t arrival_key(int ilayer, int dx, int dy, int 
 __device__ __forceinline__ int64_t key_rank(uint64_t k) { return (int64_t)(k & ((1ull << DR_RBITS) - 1)); }
 __device__ __forceinline__ int64_t key_l(uint64_t k) { return (int64_t)((k >> DR_RBITS) & ((1ull << DR_LBITS) - 1)); }
 
-#define DR_SMALL 16   // cells up to this many arrivals: one thread sorts
-#define DR_MED 1024   // up to this many: one wavefront; above: a 1024-thread workgroup
+#define DR_MED 1024   // cells up to this many arrivals are ranked in LDS; above: a 1024-thread workgroup
 
+template <int DR_CH>
 __global__ __launch_bounds__(DR_NT) void k_drift_scatter(Geo g, const int64_t* __restrict__ cstart, int64_t n3c,
                                                          const uint16_t* __restrict__ disp, const int64_t* __restrict__ cs_new,
                                                          int nlayer, int32_t* cnt, uint64_t* keys, int32_t* big,
@@ -231,20 +234,53 @@ __global__ __launch_bounds__(DR_NT) void k_drift_scatter(Geo g, const int64_t* _
 }
 
 // ---------------------------------------------------------------- sorting
-// Cells up to DR_SMALL arrivals: one thread each, insertion sort in LDS (the
-// small cells of a workgroup's DR_NT cells are packed into LDS, at most
-// DR_NT*DR_SMALL keys).  Up to DR_MED: the workgroup's wavefronts take them
-// in turn, bitonic in LDS.  Larger (listed by the scatter): one 1024-thread
+// k_drift_sort_cells takes DS_CELLS destination cells a workgroup, as many at a
+// time as fit DS_CAP keys of LDS, which they enter coalesced.  In cells up to
+// DS_RANK arrivals one thread per key ranks it (the keys are distinct); larger
+// ones are sorted by a wavefront each.  Cells above DR_MED arrivals (listed by
+// the scatter) are left to k_drift_sort_big: one 1024-thread
 // workgroup per cell; segments up to DR_SORT_LDS keys are bitonic-sorted in
 // LDS, longer ones sorted in DR_SORT_LDS chunks and then merged pairwise
 // between `keys` and `tmp` (an element's output position is its index in its
 // own run plus its rank in the partner run).
+//   Crowded workgroups bound the pass on clustered boxes.  512^3 particles at
+// z = 1.1 take 1.55 ms with the crowded cells' own kernel (1.80 with 256 cells a
+// workgroup and one fill of 4096 keys, or else a thread or a wavefront per
+// cell), 256^3 at z = 0.5 0.42 (0.50) and at z = 9 0.10 (0.12); ranking up to
+// DR_MED arrivals, quadratic in them, took 1.93, 0.68 and 0.09.
 __device__ __forceinline__ void wave_sync() {
   // a wavefront's LDS operations execute in order; this keeps the compiler
   // from moving them across the point
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// n keys in place by one wavefront: a bitonic merge network whose comparisons
+// all point up (each merge starts with a mirrored stage), so that the keys
+// that would fill n to a power of two stay where they are and need no room
+__device__ __forceinline__ void wave_sort(uint64_t* s, int n, int lane) {
+  int half = 1;
+  while (2 * half < n) half <<= 1;
+  for (int k = 1; k <= half; k <<= 1) {  // merge sorted runs of k
+    for (int t = lane; t < half; t += 64) {
+      const int b = (t & ~(k - 1)) << 1, o = t & (k - 1), i = b + o, l = b + 2 * k - 1 - o;
+      if (l < n) {
+        const uint64_t x = s[i], y = s[l];
+        if (x > y) { s[i] = y; s[l] = x; }
+      }
+    }
+    wave_sync();
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int t = lane; t < half; t += 64) {
+        const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i + j;
+        if (l < n) {
+          const uint64_t x = s[i], y = s[l];
+          if (x > y) { s[i] = y; s[l] = x; }
+        }
+      }
+      wave_sync();
+    }
+  }
 }
 // compare-exchange network over npow2 keys by NT cooperating lanes; sync()
 // separates the stages
@@ -264,102 +300,72 @@ __device__ __forceinline__ void bitonic(uint64_t* s, int n, int npow2, int tid, 
     }
 }
 
-#define DR_MED_LDS 1024
+#define DS_CELLS 64
+#define DS_CAP 2048
+#define DS_RANK 64
 __global__ __launch_bounds__(DR_NT) void k_drift_sort_cells(const int64_t* __restrict__ cs_new, int64_t n3c, uint64_t* keys) {
-  __shared__ uint64_t sk[DR_NT * DR_SMALL];  // small cells; then DR_NT/64 wavefront areas of DR_MED_LDS
-  __shared__ int32_t soff[DR_NT / 64];
-  __shared__ int32_t med[DR_NT];
-  __shared__ int32_t nmed;
-  __shared__ int32_t loff[DR_NT + 1];
-  const int64_t r = (int64_t)blockIdx.x * DR_NT + threadIdx.x;
-  int64_t base = 0;
-  int n = 0;
-  if (r < n3c) {
-    base = cs_new[r];
-    n = (int)(cs_new[r + 1] - base);
-  }
-  // Usual case: the workgroup's contiguous key range fits in LDS.  It is
-  // loaded coalesced, and each key is written to its cell's start plus its
-  // rank in the cell (the keys are distinct), one thread per key.  Keys of
-  // cells above DR_MED are left for k_drift_sort_big.
-  {
-    const int64_t rb = (int64_t)blockIdx.x * DR_NT;
-    const int ncell = (int)min((int64_t)DR_NT, n3c - rb);
-    const int64_t k0 = cs_new[rb], tot = cs_new[rb + ncell] - k0;
-    if (tot <= DR_NT * DR_SMALL) {
-      if ((int)threadIdx.x < ncell) loff[threadIdx.x] = (int32_t)(base - k0);
-      if (threadIdx.x == 0) loff[ncell] = (int32_t)tot;
-      constexpr int G = 8;
-      for (int64_t i0 = 0; i0 < tot; i0 += G * DR_NT) {
-        uint64_t v[G];
+  static_assert(DR_MED <= DS_CAP, "a cell fits");
+  __shared__ uint64_t sk[DS_CAP];
+  __shared__ int32_t loff[DS_CELLS + 1];
+  __shared__ int32_t large[DS_CELLS], nlarge;
+  const int64_t rb = (int64_t)blockIdx.x * DS_CELLS;
+  const int ncell = (int)min((int64_t)DS_CELLS, n3c - rb);
+  const int64_t k0 = cs_new[rb];
+  if ((int)threadIdx.x <= ncell) loff[threadIdx.x] = (int32_t)(cs_new[rb + threadIdx.x] - k0);
+  __syncthreads();
+  for (int ca = 0; ca < ncell;) {
+    const int32_t la = loff[ca];
+    if (loff[ca + 1] - la > DR_MED) { ca++; continue; }
+    int cb = ca + 1, hi = ncell + 1;  // last cb with loff[cb] - la <= DS_CAP
+    while (hi - cb > 1) {
+      const int m = (cb + hi) >> 1;
+      if (loff[m] - la <= DS_CAP) cb = m; else hi = m;
+    }
+    const int tot = loff[cb] - la;
+    uint64_t* const seg = keys + k0 + la;
+    constexpr int G = 4;
+    for (int i0 = 0; i0 < tot; i0 += G * DR_NT) {
+      uint64_t v[G];
 #pragma unroll
-        for (int q = 0; q < G; q++) {
-          const int64_t i = i0 + q * DR_NT + threadIdx.x;
-          v[q] = i < tot ? keys[k0 + i] : 0;
-        }
-#pragma unroll
-        for (int q = 0; q < G; q++) {
-          const int64_t i = i0 + q * DR_NT + threadIdx.x;
-          if (i < tot) sk[i] = v[q];
-        }
+      for (int q = 0; q < G; q++) {
+        const int i = i0 + q * DR_NT + threadIdx.x;
+        v[q] = i < tot ? seg[i] : 0;
       }
-      __syncthreads();
-      for (int i = threadIdx.x; i < (int)tot; i += DR_NT) {
-        int lo = 0, hi = ncell;  // last cell starting at or before i
-        while (hi - lo > 1) {
-          const int m = (lo + hi) >> 1;
-          if (loff[m] <= i) lo = m; else hi = m;
-        }
-        const int cb = loff[lo], ce = loff[lo + 1];
+#pragma unroll
+      for (int q = 0; q < G; q++) {
+        const int i = i0 + q * DR_NT + threadIdx.x;
+        if (i < tot) sk[i] = v[q];
+      }
+    }
+    if (threadIdx.x == 0) nlarge = 0;
+    __syncthreads();
+    if ((int)threadIdx.x < cb - ca) {
+      const int c = ca + threadIdx.x, n = loff[c + 1] - loff[c];
+      if (n > DS_RANK && n <= DR_MED) large[atomicAdd(&nlarge, 1)] = c;
+    }
+    for (int i = threadIdx.x; i < tot; i += DR_NT) {
+      int lo = ca, up = cb;  // last cell starting at or before i
+      while (up - lo > 1) {
+        const int m = (lo + up) >> 1;
+        if (loff[m] - la <= i) lo = m; else up = m;
+      }
+      const int c0 = loff[lo] - la, c1 = loff[lo + 1] - la;
+      if (c1 - c0 > 1 && c1 - c0 <= DS_RANK) {
         const uint64_t v = sk[i];
-        int rank = i - cb;
-        if (ce - cb <= DR_MED) {
-          rank = 0;
-          for (int j = cb; j < ce; j++) rank += sk[j] < v ? 1 : 0;
-        }
-        keys[k0 + cb + rank] = v;
+        int rank = c0;
+        for (int j = c0; j < c1; j++) rank += sk[j] < v ? 1 : 0;
+        if (rank != i) seg[rank] = v;
       }
-      return;
     }
-  }
-  if (threadIdx.x == 0) nmed = 0;
-  const int m = n <= DR_SMALL ? n : 0;  // keys this thread stages
-  int incl = m;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(incl, o);
-    if ((threadIdx.x & 63) >= o) incl += t;
-  }
-  if ((threadIdx.x & 63) == 63) soff[threadIdx.x >> 6] = incl;
-  __syncthreads();
-  if (n > DR_SMALL && n <= DR_MED) med[atomicAdd(&nmed, 1)] = threadIdx.x;
-  int wbase = 0;
-  for (int w = 0; w < (int)(threadIdx.x >> 6); w++) wbase += soff[w];
-  if (m > 1) {
-    uint64_t* a = sk + wbase + incl - m;
-    for (int i = 0; i < m; i++) a[i] = keys[base + i];
-    for (int i = 1; i < m; i++) {
-      const uint64_t v = a[i];
-      int j = i - 1;
-      while (j >= 0 && a[j] > v) { a[j + 1] = a[j]; j--; }
-      a[j + 1] = v;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < nlarge; q += DR_NT / 64) {
+      const int c0 = loff[large[q]] - la, n = loff[large[q] + 1] - la - c0;
+      wave_sort(sk + c0, n, lane);
+      for (int i = lane; i < n; i += 64) seg[c0 + i] = sk[c0 + i];
     }
-    for (int i = 0; i < m; i++) keys[base + i] = a[i];
-  }
-  __syncthreads();
-  // medium cells: wavefront w sorts list entries w, w + DR_NT/64, ...
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint64_t* ws = sk + wv * DR_MED_LDS;
-  const int nm = nmed;
-  for (int q = wv; q < nm; q += DR_NT / 64) {
-    const int64_t rr = (int64_t)blockIdx.x * DR_NT + med[q];
-    const int64_t b0 = cs_new[rr];
-    const int nn = (int)(cs_new[rr + 1] - b0);
-    int np2 = 64;
-    while (np2 < nn) np2 <<= 1;
-    for (int i = lane; i < nn; i += 64) ws[i] = keys[b0 + i];
-    bitonic<64>(ws, nn, np2, lane, [] __device__() { wave_sync(); });
-    for (int i = lane; i < nn; i += 64) keys[b0 + i] = ws[i];
-    wave_sync();
+    ca = cb;
+    if (ca < ncell) __syncthreads();
   }
 }
 
@@ -416,17 +422,20 @@ __global__ __launch_bounds__(DR_SORT_NT) void k_drift_sort_big(const int64_t* __
 
 // ---------------------------------------------------------- gather + cells
 // One workgroup per DW_CELLS destination cells; their slots (checkpoint
-// order after the drift) are contiguous.
+// order after the drift) are contiguous.  It takes as many cells at a time as
+// have DW_STAGE slots, whose full velocities stay in LDS:
 //   gather (one thread per slot, DG_SL slots per batch with each stage's
 //     loads issued together): the arrival's full velocity vreal
 //     (update_particle.f90:69), its new position code (:117) and PID.
-//     vreal stays in LDS when the workgroup's slots fit (else in HBM).
 //   cells (one thread per cell): vfield_new summed in arrival order
 //     (update_particle.f90:70-83).
 //   slots (DC_SL per batch): the velocity residual re-quantised with the old
 //     sigma (:119) and the sigma_v sums (:174-200).
+// A cell of more than DW_STAGE slots keeps its velocities in HBM, and its sum
+// takes them through LDS in pieces.  (With all cells of a crowded workgroup in
+// HBM, one thread per cell reading its velocities back, 512^3 particles at
+// z = 1.1 took 5.5 instead of 4.55 ms, 256^3 at z = 0.5 1.06 instead of 0.83.)
 // part: 3 doubles per workgroup, at its first cell's index / DW_CELLS.
-#define DW_CELLS 128
 #define DW_STAGE 1536
 #define DG_SL 4
 #define DC_SL 2
@@ -437,13 +446,13 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
                                                  const float* __restrict__ vfield, float dt_mid, double c_old,
                                                  const double* __restrict__ vdt, const double* __restrict__ venc,
                                                  int32_t kmax, void* xp_o, int32_t* pid_o, double* vr, void* vp_o,
-                                                 float* vfield_o, int32_t* rhoc_o, double* part, const int64_t* scs,
-                                                 float* svf, double (*red)[DR_NT / 64], double* svr, const double* sat) {
+                                                 float* vfield_o, int32_t* rhoc_o, const int64_t* scs,
+                                                 float* svf, double* svr, const double* sat, double sums[3]) {
   const int64_t qa = scs[0], q1 = scs[ncell];
   // vreal of slot q: LDS when the workgroup's slots fit, else the HBM scratch
   auto vr_at = [&](int64_t q, int e) -> double& { return STAGED ? svr[3 * (q - qa) + e] : vr[3 * q + e]; };
   // ---- gather
-  const double xscale = (g.izipx == 1 ? 1.0 / 256.0 : 1.0 / 65536.0) * (double)CUBE_NCELL;
+  const double xscale = (g.izipx == 1 ? 256.0 : 65536.0) / (double)CUBE_NCELL;  // position units per fine cell, a power of two
   for (int64_t q0 = qa + threadIdx.x; q0 < q1; q0 += (int64_t)DR_NT * DG_SL) {
     uint64_t key[DG_SL];
     bool ok[DG_SL];
@@ -483,10 +492,8 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
 #pragma unroll
       for (int e = 0; e < 3; e++) {
         const double vreal = vd[j][e] + (double)vf[j][e];
-        int64_t xn = (int64_t)xu[j][e];
-        xn = g.izipx == 1 ? (int64_t)(int8_t)xn : (int64_t)(int16_t)xn;
-        xn += (int64_t)nint_d((double)dt_mid * vreal / xscale);
-        store_x(xp_o, 3 * q + e, g.izipx, xn);
+        // a particle that moved further than 32 bits hold fails the drift
+        store_x(xp_o, 3 * q + e, g.izipx, (int64_t)((int32_t)xu[j][e] + (int32_t)nint_d((double)dt_mid * vreal * xscale)));
         vr_at(q, e) = vreal;
       }
       pid_o[q] = pv[j];
@@ -497,7 +504,33 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
   // ---- cells
   const double wv = (double)0.1f;  // weight_v=0.1 is a default-real literal
   double sum_c = 0, sum_r = 0, sum_s = 0;
-  if ((int)threadIdx.x < ncell) {
+  auto finish = [&](int64_t r, int c, const float vf[3], int64_t n) {
+    float vfn[3];
+    for (int e = 0; e < 3; e++) {
+      vfn[e] = (float)((double)vf[e] / ((double)n + wv));
+      svf[c * 3 + e] = vfn[e];
+      vfield_o[r * 3 + e] = vfn[e];
+    }
+    rhoc_o[r] = (int32_t)n;
+    sum_c = (double)(vfn[0] * vfn[0] + vfn[1] * vfn[1] + vfn[2] * vfn[2]);
+  };
+  if (!STAGED) {
+    // one cell: its velocities through LDS, a thread per component adding them
+    float vf = threadIdx.x < 3 ? (float)((double)vfield[r0 * 3 + threadIdx.x] * wv) : 0.f;
+    for (int64_t b = qa; b < q1; b += DW_STAGE) {
+      const int m = (int)min((int64_t)DW_STAGE, q1 - b);
+      for (int i = threadIdx.x; i < 3 * m; i += DR_NT) svr[i] = vr[3 * b + i];
+      __syncthreads();
+      if (threadIdx.x < 3)
+        for (int k = 0; k < m; k++) vf = (float)((double)vf + svr[3 * k + threadIdx.x]);
+      __syncthreads();
+    }
+    if (threadIdx.x < 3) svf[threadIdx.x] = vf;
+    __syncthreads();
+    const float sum3[3] = {svf[0], svf[1], svf[2]};
+    __syncthreads();
+    if (threadIdx.x == 0) finish(r0, 0, sum3, q1 - qa);
+  } else if ((int)threadIdx.x < ncell) {
     const int64_t r = r0 + threadIdx.x;
     const int64_t b = scs[threadIdx.x], n = scs[threadIdx.x + 1] - b;
     float vf[3];
@@ -516,14 +549,7 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
 #pragma unroll
           for (int e = 0; e < 3; e++) vf[e] = (float)((double)vf[e] + a[u][e]);
     }
-    float vfn[3];
-    for (int e = 0; e < 3; e++) {
-      vfn[e] = (float)((double)vf[e] / ((double)n + wv));
-      svf[threadIdx.x * 3 + e] = vfn[e];
-      vfield_o[r * 3 + e] = vfn[e];
-    }
-    rhoc_o[r] = (int32_t)n;
-    sum_c = (double)(vfn[0] * vfn[0] + vfn[1] * vfn[1] + vfn[2] * vfn[2]);
+    finish(r, threadIdx.x, vf, n);
   }
   __syncthreads();
   // ---- slots: re-quantisation and sigma sums, DC_SL per batch
@@ -569,20 +595,12 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
       sum_s += w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
     }
   }
-  double v3[3] = {sum_c, sum_r, sum_s};
-  for (int f = 0; f < 3; f++) {
-    double v = v3[f];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0) red[f][threadIdx.x >> 6] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) {
-    double t = 0;
-    for (int i = 0; i < DR_NT / 64; i++) t += red[threadIdx.x][i];
-    part[r0 / DW_CELLS * 3 + threadIdx.x] = t;
-  }
+  sums[0] += sum_c;
+  sums[1] += sum_r;
+  sums[2] += sum_s;
 }
 
+template <int DW_CELLS>
 __global__ __launch_bounds__(DR_NT) void k_drift_write(Geo g, const uint64_t* __restrict__ keys, const int64_t* __restrict__ cs_new,
                                                        int64_t n3c, const int64_t* __restrict__ cstart, const void* __restrict__ xp,
                                                        const void* __restrict__ vp, const int32_t* __restrict__ pid,
@@ -602,12 +620,33 @@ __global__ __launch_bounds__(DR_NT) void k_drift_write(Geo g, const uint64_t* __
   for (int i = threadIdx.x; i <= DW_CELLS; i += DR_NT) scs[i] = cs_new[r0 + min(i, ncell)];
   atan_tab_to_lds(sat);
   __syncthreads();
-  if (scs[ncell] - scs[0] <= DW_STAGE)
-    drift_write_body<true>(g, keys, r0, ncell, cstart, xp, vp, pid, vfield, dt_mid, c_old, vdt, venc, kmax, xp_o, pid_o, vr, vp_o,
-                           vfield_o, rhoc_o, part, scs, svf, red, svr, sat);
-  else
-    drift_write_body<false>(g, keys, r0, ncell, cstart, xp, vp, pid, vfield, dt_mid, c_old, vdt, venc, kmax, xp_o, pid_o, vr,
-                            vp_o, vfield_o, rhoc_o, part, scs, svf, red, svr, sat);
+  double sums[3] = {0, 0, 0};
+  for (int ca = 0; ca < ncell;) {
+    int cb = ca + 1, hi = ncell + 1;  // last cb whose cells ca..cb-1 have DW_STAGE slots, at least one cell
+    while (hi - cb > 1) {
+      const int m = (cb + hi) >> 1;
+      if (scs[m] - scs[ca] <= DW_STAGE) cb = m; else hi = m;
+    }
+    if (scs[cb] - scs[ca] <= DW_STAGE)
+      drift_write_body<true>(g, keys, r0 + ca, cb - ca, cstart, xp, vp, pid, vfield, dt_mid, c_old, vdt, venc, kmax, xp_o, pid_o,
+                             vr, vp_o, vfield_o, rhoc_o, scs + ca, svf, svr, sat, sums);
+    else
+      drift_write_body<false>(g, keys, r0 + ca, 1, cstart, xp, vp, pid, vfield, dt_mid, c_old, vdt, venc, kmax, xp_o, pid_o, vr,
+                              vp_o, vfield_o, rhoc_o, scs + ca, svf, svr, sat, sums);
+    ca = cb;
+    if (ca < ncell) __syncthreads();
+  }
+  for (int f = 0; f < 3; f++) {
+    double v = sums[f];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) red[f][threadIdx.x >> 6] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double t = 0;
+    for (int i = 0; i < DR_NT / 64; i++) t += red[threadIdx.x][i];
+    part[r0 / DW_CELLS * 3 + threadIdx.x] = t;
+  }
 }
 
 // sigma_vi_new = sqrt(sum v_res^2 / N) / sqrt(3) (update_particle.f90:213,
@@ -649,16 +688,21 @@ static int drift_launch(cube_handle* h, float dt_old, float dt, int* nlayer_out)
   const double* vdt = vtab_for(h, c_old);
   const int dmax = (int)(h->ncb < DMAX ? h->ncb : DMAX);
   uint32_t* flags = h->uflags;  // [0..2] max disp, [3] too far / crowded, [4] frame conflicts, [6] crowded cells
-  const int64_t nb1 = (h->n3c + DR_CH - 1) / DR_CH;
-  const int64_t nb3 = (h->n3c + DR_NT - 1) / DR_NT;
-  const int64_t nbw = (h->n3c + DW_CELLS - 1) / DW_CELLS;
-  if (nb3 * 3 > h->dred_n - 16 || nbw * 3 > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
+  // cells per workgroup: 256 source and 128 destination cells, fewer where
+  // that would leave most CUs without a workgroup (up to 32^3 cells)
+  const bool few = h->n3c <= 32768;
+  const int ch = few ? 32 : 256, dwc = few ? 32 : 128;
+  const int64_t nb1 = (h->n3c + ch - 1) / ch;
+  const int64_t nb3 = (h->n3c + DS_CELLS - 1) / DS_CELLS;
+  const int64_t nbw = (h->n3c + dwc - 1) / dwc;
+  if (nbw * 3 > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
   int r;
   if ((r = fill_u32(h, flags, 8, 0u)) || (r = fill_u32(h, h->rhoc2, h->n3c, 0u)) ||
       (r = fill_u32(h, h->mslots, MSLOTS * MSLOT_FIELDS, 0u)))
     return r;
   int pid1 = prof_begin(h, PS_DRIFT1);
-  k_drift_pass1<<<(unsigned)nb1, DR_NT, 0, h->stream>>>(g, h->xp, h->vp, h->cstart, h->n3c, h->vfield, dt_mid, c_old, vdt, dmax,
+  auto* pass1 = few ? k_drift_pass1<32> : k_drift_pass1<256>;
+  pass1<<<(unsigned)nb1, DR_NT, 0, h->stream>>>(g, h->xp, h->vp, h->cstart, h->n3c, h->vfield, dt_mid, c_old, vdt, dmax,
                                                          h->disp, h->rhoc2, h->mslots);
   prof_end(h, pid1);
   HIP_TRY(h, hipGetLastError());
@@ -670,7 +714,8 @@ static int drift_launch(cube_handle* h, float dt_old, float dt, int* nlayer_out)
   uint64_t* keys = (uint64_t*)h->order;
   uint32_t* nbig = flags + 6;
   int pid3 = prof_begin(h, PS_DRIFT_SCATTER);
-  k_drift_scatter<<<(unsigned)nb1, DR_NT, 0, h->stream>>>(g, h->cstart, h->n3c, h->disp, h->cstart2, nlayer, h->rhoc2, keys,
+  auto* scatter = few ? k_drift_scatter<32> : k_drift_scatter<256>;
+  scatter<<<(unsigned)nb1, DR_NT, 0, h->stream>>>(g, h->cstart, h->n3c, h->disp, h->cstart2, nlayer, h->rhoc2, keys,
                                                            h->dbig, nbig);
   prof_end(h, pid3);
   HIP_TRY(h, hipGetLastError());
@@ -680,7 +725,8 @@ static int drift_launch(cube_handle* h, float dt_old, float dt, int* nlayer_out)
   prof_end(h, pid4);
   HIP_TRY(h, hipGetLastError());
   int pid5 = prof_begin(h, PS_DRIFT_WRITE);
-  k_drift_write<<<(unsigned)nbw, DR_NT, 0, h->stream>>>(g, keys, h->cstart2, h->n3c, h->cstart, h->xp, h->vp, h->pid, h->vfield,
+  auto* write = few ? k_drift_write<32> : k_drift_write<128>;
+  write<<<(unsigned)nbw, DR_NT, 0, h->stream>>>(g, keys, h->cstart2, h->n3c, h->cstart, h->xp, h->vp, h->pid, h->vfield,
                                                          dt_mid, c_old, vdt, h->venc, h->vkmax, h->xp2, h->pid2,
                                                          (double*)h->dscratch, h->vp2, h->vfield2, h->rhoc2, h->dred);
   prof_end(h, pid5);
