@@ -425,11 +425,12 @@ __global__ __launch_bounds__(NT_FFT) void k_fft_zconv(const cpx<T>* src, cpx<T>*
 
 // ------------------------------------------------- kx-tiled complex layout
 // The per-step fine-mesh convolution keeps its spectrum in a kx-tiled
-// layout: element (kx, ky, kz) at ((kx/16 * N + kz) * N + ky) * 16 + kx%16,
+// layout: element (kx, ky, kz) at ((kx/16 * N + kz) * P + ky) * 16 + kx%16,
+// P = t_pitch(N),
 // KT = ceil((N/2+1)/16) tiles of 16 kx (slots past N/2 are padding).  Every
 // pass then moves whole cache lines: a y column strip of W kx is W*8 bytes
 // of each 128-byte group (neighbouring strips complete the group), a z
-// strip likewise at a stride of N*16 elements, and an x row block of W rows
+// strip likewise at a stride of P*16 elements, and an x row block of W rows
 // is written and read as 16*W contiguous elements per kx tile.  The R2C and
 // C2R passes run out of place (real rows <-> tiled spectrum).
 #define TB 16
@@ -450,7 +451,7 @@ template <typename T>
 constexpr int pick_ntz(int logn) { return pick_wz<T>(logn) > pick_w<T>(logn) ? 2 * NT_FFT : NT_FFT; }
 __host__ __device__ constexpr int64_t t_tiles(int64_t N) { return (N / 2 + 1 + TB - 1) / TB; }
 __host__ __device__ __forceinline__ int64_t t_index(int64_t N, int64_t kx, int64_t ky, int64_t kz) {
-  return (((kx / TB) * N + kz) * N + ky) * TB + kx % TB;
+  return (((kx / TB) * N + kz) * t_pitch(N) + ky) * TB + kx % TB;
 }
 
 // real rows src (pitch N+2) -> tiled spectrum dst
@@ -565,7 +566,7 @@ __global__ __launch_bounds__(pick_nty<T>(LOGN)) void k_ty(cpx<T>* data, const cp
   int bx, by;
   grid_block_xy(bx, by);
   const int kh = bx / NP, part = bx % NP, kz = by;
-  const int64_t base = (((int64_t)kh * N + kz) * N) * TB + part * W;
+  const int64_t base = (((int64_t)kh * N + kz) * t_pitch(N)) * TB + part * W;
   col_load<T, N, W, NTH>(s, data + base, TB, W);
   lds_fft<T, N, W, INV, W, NTH>(s, tw, 1);
   for (int idx = threadIdx.x; idx < N * W; idx += NTH) {
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(pick_nty<T>(LOGN)) void k_ty(cpx<T>* data, const cp
 }
 
 // tiled z convolution: dst = Zinv(i*K_d . Zfwd(src)), tile (kh, part, ky) =
-// W columns along kz (stride N*16); dst may be src
+// W columns along kz (stride t_pitch(N)*16); dst may be src
 template <typename T, int LOGN>
 __global__ __launch_bounds__(pick_ntz<T>(LOGN)) void k_tzconv(const cpx<T>* src, cpx<T>* dst, const T* __restrict__ K, int d,
                                                    const cpx<T>* __restrict__ tw) {
@@ -586,8 +587,8 @@ __global__ __launch_bounds__(pick_ntz<T>(LOGN)) void k_tzconv(const cpx<T>* src,
   int bx, by;
   grid_block_xy(bx, by);
   const int kh = bx / NP, part = bx % NP, ky = by, kx0 = kh * TB + part * W;
-  const int64_t stride = (int64_t)N * TB;
-  const int64_t base = ((int64_t)kh * N * N) * TB + (int64_t)ky * TB + part * W;
+  const int64_t stride = (int64_t)t_pitch(N) * TB;
+  const int64_t base = (int64_t)kh * N * stride + (int64_t)ky * TB + part * W;
   const int kyp = ky <= N / 2 ? ky : N - ky;
   const T sy = (d == 1 && ky > N / 2) ? (T)-1 : (T)1;
   // K in strips of W kx: K[d][kyp][kx / W][kzp][kx % W], so the strip's
@@ -647,8 +648,8 @@ __global__ __launch_bounds__(pick_ntz<T>(LOGN)) void k_tzconv3(const cpx<T>* src
   int bx, by;
   grid_block_xy(bx, by);
   const int kh = bx / NP, part = bx % NP, ky = by, kx0 = kh * TB + part * W;
-  const int64_t stride = (int64_t)N * TB;
-  const int64_t base = ((int64_t)kh * N * N) * TB + (int64_t)ky * TB + part * W;
+  const int64_t stride = (int64_t)t_pitch(N) * TB;
+  const int64_t base = (int64_t)kh * N * stride + (int64_t)ky * TB + part * W;
   const int kyp = ky <= N / 2 ? ky : N - ky;
   constexpr int G = (int)(t_tiles(N) * TB / WK);
   col_load<T, N, W, NTH>(sa, src + base, stride, W);
