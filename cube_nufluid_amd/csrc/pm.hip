@@ -11,38 +11,42 @@
 
 #define CIC_NT 256
 #define CIC_U 4  // particles per thread and batch in the CIC kernels
+#define CIC_FEW 32  // boxes of at most this many cells a side take half-width coarse blocks
 
 // --------------------------------------------------------------- helpers
-// Load cstart for the cells of a SPAN^3 region around block origin c0 (lo
-// cells below it) into LDS as per-cell begin/offset arrays (one segment per
-// cell).  The offsets are an exclusive scan over the whole workgroup:
-// each thread takes PER consecutive cells.
+// Load cstart for the cells of a SPAN^3 region around block origin c0 (one
+// cell below it) into LDS: the region's particles numbered t = 0, 1, ... in
+// cell order, cell i's from off[i], and del[i] + t the index of particle t of
+// cell i.  The offsets are an exclusive scan over the whole workgroup: each
+// thread takes PER consecutive cells.  own (zero before): a mark (cell_key) at
+// the first particle of every cell among the first CIC_NT*CIC_U particles.
 template <int SPAN>
-__device__ void load_region(const Geo& g, const int64_t* cstart, int c0x, int c0y, int c0z, int lo,
-                            int64_t* beg, int32_t* off) {
+__device__ __forceinline__ uint32_t cell_key(int i) {
+  return (uint32_t)((i / (SPAN * SPAN)) << 8 | (i / SPAN % SPAN) << 4 | i % SPAN) + 1u;
+}
+template <int SPAN>
+__device__ void load_region(const Geo& g, const int64_t* cstart, int c0x, int c0y, int c0z, int64_t* del, int32_t* off,
+                            uint16_t* own) {
   constexpr int NCELL = SPAN * SPAN * SPAN, PER = (NCELL + CIC_NT - 1) / CIC_NT;
   __shared__ int32_t wsum[CIC_NT / 64];
+  int64_t beg[PER];
   int32_t cnt[PER];
   int32_t tsum = 0;
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const int i = threadIdx.x * PER + k;
     cnt[k] = 0;
+    beg[k] = 0;
     if (i < NCELL) {
-      const int rx = i % SPAN - lo, ry = (i / SPAN) % SPAN - lo, rz = i / (SPAN * SPAN) - lo;
+      const int rx = i % SPAN - 1, ry = (i / SPAN) % SPAN - 1, rz = i / (SPAN * SPAN) - 1;
       const int64_t r = rank_of(g, wrapc(c0x + rx, g.nc), wrapc(c0y + ry, g.nc), wrapc(c0z + rz, g.nc));
-      const int64_t b = cstart[r];
-      beg[i] = b;
-      cnt[k] = (int32_t)(cstart[r + 1] - b);
+      beg[k] = cstart[r];
+      cnt[k] = (int32_t)(cstart[r + 1] - beg[k]);
     }
     tsum += cnt[k];
   }
   const int lane = threadIdx.x & 63;
-  int32_t incl = tsum;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int32_t t = __shfl_up(incl, o);
-    if (lane >= o) incl += t;
-  }
+  const int32_t incl = wave_incl_add(tsum);
   if (lane == 63) wsum[threadIdx.x >> 6] = incl;
   __syncthreads();
   int32_t run = incl - tsum;
@@ -50,44 +54,74 @@ __device__ void load_region(const Geo& g, const int64_t* cstart, int c0x, int c0
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const int i = threadIdx.x * PER + k;
-    if (i < NCELL) off[i] = run;
+    if (i < NCELL) {
+      off[i] = run;
+      del[i] = beg[k] - run;
+      if (cnt[k] > 0 && run < CIC_NT * CIC_U) own[run] = (uint16_t)cell_key<SPAN>(i);
+    }
     run += cnt[k];
   }
   if (threadIdx.x == CIC_NT - 1) off[NCELL] = run;
   __syncthreads();
 }
-__device__ __forceinline__ int seg_find(const int32_t* off, int n, int32_t t) {
-  int lo = 0, hi = n;  // off[lo] <= t < off[hi]
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (off[mid] <= t) lo = mid; else hi = mid;
-  }
-  return lo;
+// the last i < n with off[i] <= t, the same t in every lane of a wavefront
+// (n <= 64 * 64): each lane looks at one entry of every STEP, then at one of
+// the STEP found
+template <int N>
+__device__ __forceinline__ int wave_find(const int32_t* off, int32_t t) {
+  constexpr int STEP = (N + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const bool in1 = lane * STEP < N && off[lane * STEP < N ? lane * STEP : 0] <= t;
+  const int seg = __popcll(__ballot(in1)) - 1;
+  const int i = seg * STEP + lane;
+  const bool in2 = lane < STEP && i < N && off[i < N ? i : 0] <= t;
+  return seg * STEP + __popcll(__ballot(in2)) - 1;
 }
 
-// ------------------------------------------------------------- fine CIC
-// One workgroup per BC^3 coarse cells = (4BC)^3 fine nodes, binned in LDS.
-// Nodes sit on fine-cell left edges (pm.f90:87 has no -0.5); a particle in
-// coarse cell c touches fine nodes 4c..4c+4, so the block gathers cells
-// [c0-1, c0+BC) and keeps taps on its own nodes: every node is written once.
-// Each weight (the reference's float product) is accumulated as a 64-bit
-// fixed-point integer (2^-40 units), so node sums are exact and independent
-// of the order in which threads add them; the node value is the sum rounded
-// once to float.
+// ----------------------------------------------------- CIC mass assignment
+// One workgroup per BC^3 coarse cells = (S*BC)^3 nodes, binned in LDS: the
+// fine mesh has S = 4 nodes a cell on fine-cell left edges (pm.f90:87 has no
+// -0.5), the coarse mesh S = 1 at coarse-cell centres (CENTRE, pm.f90:255
+// '-0.5'), the halo finder's density S = 4 at fine-cell centres
+// (halofind.f90:159).  A particle in cell c touches nodes S*c..S*c + S
+// (CENTRE: S*c - 1..S*c + S), so the block gathers cells [c0-1, c0+BC)
+// (CENTRE: [c0-1, c0+BC]) and keeps taps on its own nodes: every node is
+// written once.  Each weight (the reference's float product) is accumulated
+// as a 64-bit fixed-point integer (2^-40 units), so node sums are exact and
+// independent of the order in which threads add them; the node value is the
+// sum rounded once to float.  R has row pitch `pitch`.
+//
+// Bound by VALU issue and by LDS atomics, not by memory.  Per visit of a
+// particle: its cell comes from a table with a mark at every cell's first
+// particle and a running maximum over the wavefront (a search of the offsets
+// cost 60 instructions); its frame is formed in T by one fused operation,
+// whose single rounding is that of the exact double sum; and a weight
+// becomes an integer by adding 1.5*2^52 (FAST: mass <= 1024 keeps it below
+// 2^51), which rounds as llrint does.  A cell's particles mostly add to the
+// same nodes, so where cells hold several they go to one thread (`dense`).
+// ms, a search of the offsets per visit and llrint -> this: with 8 particles
+// a cell coarse 1.55 -> 1.28 and fine 3.13 -> 2.89 at 256^3 cells, .240 ->
+// .176 and .403 -> .355 at 128^3; with 1 a cell .288 -> .267 and 2.02 -> 2.05
+// at 256^3, .048 -> .040 and .226 -> .215 at 128^3.  Lanes on consecutive
+// particles throughout: 1.37 and 3.17 with 8 a cell at 256^3; threads on
+// consecutive ones throughout: .336 and 2.05 with 1.
 #define CIC_FIX 1099511627776.0  // 2^40
-// CENTRE: the halo finder's density (halofind.f90:159), whose nodes sit at
-// fine-cell centres ('-0.5'): a particle in cell c then touches nodes
-// 4c-1..4c+4 and the block gathers cells [c0-1, c0+BC].  R has row pitch
-// `pitch`.
-template <int BC, typename T, bool CENTRE = false>
-__global__ __launch_bounds__(CIC_NT) void k_cic_fine(Geo g, const void* __restrict__ xp, const int64_t* __restrict__ cstart,
-                                                     float mass_f, T* R, int64_t N, int64_t pitch, double* part) {
+template <int BC, int S, bool CENTRE, typename T, int IZX, bool FAST>
+__global__ __launch_bounds__(CIC_NT) void k_cic(Geo g, const void* __restrict__ xp, const int64_t* __restrict__ cstart,
+                                                float mass_f, T* R, int64_t N, int64_t pitch, double* part) {
   const T mass = (T)mass_f;
-  constexpr int F = 4 * BC, SPAN = BC + (CENTRE ? 2 : 1), NCELL = SPAN * SPAN * SPAN;
-  __shared__ unsigned long long s[F * F * F];
-  __shared__ int64_t beg[NCELL];
+  constexpr int F = S * BC, SPAN = BC + (CENTRE ? 2 : 1), NCELL = SPAN * SPAN * SPAN;
+  static_assert(SPAN <= 16 && NCELL <= 4096, "cell coordinates in four bits");
+  // an unused run before the nodes, so a tap's address is its particle's
+  // lowest tap's and a constant
+  constexpr int PRE = F * F + F + 1;
+  __shared__ unsigned long long sn[PRE + F * F * F];
+  __shared__ int64_t del[NCELL];
   __shared__ int32_t off[NCELL + 1];
+  __shared__ uint16_t own[CIC_NT * CIC_U];
   __shared__ double red[CIC_NT / 64];
+  unsigned long long* const s = sn + PRE;
+  const int tid = threadIdx.x;
   const int nbx = g.nc / BC;
   // XCD-contiguous block order: x neighbours, which write the two halves of
   // shared 128-byte lines, run on one L2
@@ -95,197 +129,187 @@ __global__ __launch_bounds__(CIC_NT) void k_cic_fine(Geo g, const void* __restri
   const int bx = lb % nbx, by = (lb / nbx) % nbx, bz = lb / (nbx * nbx);
   const int c0x = bx * BC, c0y = by * BC, c0z = bz * BC;
   // block-local tile frame: 0-based offset of c0 inside its tile
-  const int l0x = c0x % g.nt, l0y = c0y % g.nt, l0z = c0z % g.nt;
-  for (int i = threadIdx.x; i < F * F * F; i += CIC_NT) s[i] = 0ull;
-  load_region<SPAN>(g, cstart, c0x, c0y, c0z, 1, beg, off);
+  const int l0[3] = {c0x % g.nt, c0y % g.nt, c0z % g.nt};
+  for (int i = tid; i < F * F * F; i += CIC_NT) s[i] = 0ull;
+#pragma unroll
+  for (int j = 0; j < CIC_U; j++) own[tid + j * CIC_NT] = 0;
+  load_region<SPAN>(g, cstart, c0x, c0y, c0z, del, off, own);
   const int32_t total = off[NCELL];
-  // CIC_U particles per thread and batch: their cell searches and position
-  // loads are issued together, then their taps added
-  for (int32_t t0 = threadIdx.x; t0 < total; t0 += CIC_NT * CIC_U) {
-    int cib[CIC_U];
-    uint32_t ub[CIC_U][3];
+  // a thread's particles are consecutive where cells hold several, so that
+  // the lanes of a wavefront seldom share a cell; else the lanes'
+  const bool dense = total > 3 * NCELL;
+  T fr0[3];
 #pragma unroll
-    for (int j = 0; j < CIC_U; j++) {
-      const int32_t t = t0 + j * CIC_NT;
-      cib[j] = t < total ? seg_find(off, NCELL, t) : 0;
-      const int64_t p = beg[cib[j]] + (t - off[cib[j]]);
-#pragma unroll
-      for (int e = 0; e < 3; e++) ub[j][e] = t < total ? load_xu(xp, 3 * p + e, g.izipx) : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < CIC_U; j++) {
-      if (t0 + j * CIC_NT >= total) break;
-      const int ci = cib[j];
-      int rel[3] = {ci % SPAN - 1, (ci / SPAN) % SPAN - 1, ci / (SPAN * SPAN) - 1};
-      int l0[3] = {l0x, l0y, l0z};
-      T dx1[3], dx2[3];
-      int n1[3];
-      for (int e = 0; e < 3; e++) {
-        int il = l0[e] + rel[e] + 1;  // tile-local 1-based cell index (0 = left ghost)
-        uint32_t u = ub[j][e];
-        T tx;
-        if constexpr (CENTRE)
-          tx = (T)((double)(CUBE_NCELL * (il - 1)) + (double)CUBE_NCELL * xoff(u, g.izipx) - 0.5);
-        else
-          tx = (T)((double)(CUBE_NCELL * (il - 1)) + (double)CUBE_NCELL * xoff(u, g.izipx));
-        int a1 = (int)floor(tx) + 1;
-        dx1[e] = (T)a1 - tx;
-        dx2[e] = 1 - dx1[e];
-        n1[e] = (a1 - 1) - CUBE_NCELL * l0[e];  // block-local node of tap 1
+  for (int e = 0; e < 3; e++) fr0[e] = (T)(S * (l0[e] - 1)) - (CENTRE ? (T)0.5 : (T)0);
+  for (int32_t T0 = 0; T0 < total; T0 += CIC_NT * CIC_U) {
+    if (T0 > 0) {  // the next batch's marks
+      __syncthreads();
+      for (int i = tid; i < NCELL; i += CIC_NT) {
+        const int32_t o = off[i] - T0;
+        if ((uint32_t)o < (uint32_t)(CIC_NT * CIC_U) && off[i + 1] > off[i]) own[o] = (uint16_t)cell_key<SPAN>(i);
       }
-      const T w[8] = {dx1[0] * dx1[1] * dx1[2] * mass, dx2[0] * dx1[1] * dx1[2] * mass,
-                      dx1[0] * dx2[1] * dx1[2] * mass, dx1[0] * dx1[1] * dx2[2] * mass,
-                      dx1[0] * dx2[1] * dx2[2] * mass, dx2[0] * dx1[1] * dx2[2] * mass,
-                      dx2[0] * dx2[1] * dx1[2] * mass, dx2[0] * dx2[1] * dx2[2] * mass};
-      const int o[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 1, 1}, {1, 0, 1}, {1, 1, 0}, {1, 1, 1}};
+      __syncthreads();
+    }
+    const int32_t left = total - T0;
+    const int u = left >= CIC_NT * CIC_U ? CIC_U : (left + CIC_NT - 1) / CIC_NT;  // particles per thread
+    const int32_t tw = T0 + (tid & ~63) * u;                                      // the wavefront's first
+    if (tw < total) {
+      // particle j of a thread: t = tw + lane*jl + j*js
+      const int lane = tid & 63, jl = dense ? u : 1, js = dense ? 1 : 64, ow = tw - T0 + lane * jl;
+      int32_t key[CIC_U];
+      int32_t before = (int32_t)cell_key<SPAN>(wave_find<NCELL>(off, tw));
+      if (dense) {
+        int32_t mx = 0;
 #pragma unroll
-      for (int q = 0; q < 8; q++) {
-        int x = n1[0] + o[q][0], y = n1[1] + o[q][1], z = n1[2] + o[q][2];
-        if ((unsigned)x < (unsigned)F && (unsigned)y < (unsigned)F && (unsigned)z < (unsigned)F)
-          atomicAdd(&s[(z * F + y) * F + x], (unsigned long long)llrint((double)w[q] * CIC_FIX));
+        for (int j = 0; j < CIC_U; j++) {
+          if (j < u) {
+            mx = max(mx, (int32_t)own[ow + j]);
+            own[ow + j] = 0;
+          }
+          key[j] = mx;
+        }
+        const int32_t up = __shfl_up(wave_incl_max(mx), 1);
+        if (lane > 0) before = max(before, up);
+#pragma unroll
+        for (int j = 0; j < CIC_U; j++) key[j] = max(key[j], before) - 1;
+      } else {
+#pragma unroll
+        for (int j = 0; j < CIC_U; j++) {
+          key[j] = 0;
+          if (j < u) {
+            const int32_t inc = max(before, wave_incl_max((int32_t)own[ow + j * 64]));
+            own[ow + j * 64] = 0;
+            before = __builtin_amdgcn_readlane(inc, 63);
+            key[j] = inc - 1;
+          }
+        }
+      }
+      uint32_t ub[CIC_U][3];
+#pragma unroll
+      for (int j = 0; j < CIC_U; j++) {
+        const int32_t t = tw + lane * jl + j * js;
+        const int ci = (int)((key[j] >> 8) * (SPAN * SPAN) + (key[j] >> 4 & 15) * SPAN + (key[j] & 15));
+        const bool in = j < u && t < total;
+        const int64_t p = in ? del[ci] + t : 0;
+#pragma unroll
+        for (int e = 0; e < 3; e++) ub[j][e] = in ? load_xu(xp, 3 * p + e, IZX) : 0u;
+      }
+#pragma unroll
+      for (int j = 0; j < CIC_U; j++) {
+        if (j >= u || tw + lane * jl + j * js >= total) break;
+        T d1[3], d2[3];
+        int n1[3];
+        bool in1[3], in2[3];
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+          // S*(il + xoff) - 0.5 of tile-local cell il (-1 = left ghost): u + 0.5
+          // and the frame are exact in T
+          const T fr = fma((T)(key[j] >> 4 * e & 15), (T)S, fr0[e]);
+          const T tx = fma((T)ub[j][e] + (T)0.5, (T)S * (IZX == 1 ? (T)(1.0 / 256.0) : (T)(1.0 / 65536.0)), fr);
+          const T fl = floor(tx);
+          d1[e] = fl + (T)1 - tx;
+          d2[e] = 1 - d1[e];
+          n1[e] = (int)fl - S * l0[e];  // block-local node of tap 1
+          in1[e] = (unsigned)n1[e] < (unsigned)F;
+          in2[e] = (unsigned)(n1[e] + 1) < (unsigned)F;
+        }
+        unsigned long long* const t0 = sn + (PRE + (n1[2] * F + n1[1]) * F + n1[0]);
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          const int ox = q & 1, oy = q >> 1 & 1, oz = q >> 2;
+          const T w = (ox ? d2[0] : d1[0]) * (oy ? d2[1] : d1[1]) * (oz ? d2[2] : d1[2]) * mass;
+          long long f;
+          if constexpr (FAST) {
+            const double M = 6755399441055744.0;  // 1.5*2^52
+            f = __double_as_longlong(fma((double)w, CIC_FIX, M)) - __double_as_longlong(M);
+          } else {
+            f = llrint((double)w * CIC_FIX);
+          }
+          if ((ox ? in2[0] : in1[0]) && (oy ? in2[1] : in1[1]) && (oz ? in2[2] : in1[2]))
+            atomicAdd(t0 + ((oz * F + oy) * F + ox), (unsigned long long)f);
+        }
       }
     }
   }
   __syncthreads();
   double ms = 0;
-  for (int i = threadIdx.x; i < F * F * F; i += CIC_NT) {
-    int x = i % F, y = (i / F) % F, z = i / (F * F);
-    int64_t gx = 4 * c0x + x, gy = 4 * c0y + y, gz = 4 * c0z + z;
-    double vd = (double)(long long)s[i] * (1.0 / CIC_FIX);
-    R[(gz * N + gy) * pitch + gx] = (T)vd;
-    ms += vd;
+  // node tid + it * CIC_NT, it = 0, 1, ...: the same x and y, ZS planes on
+  T* const R0 = R + ((int64_t)(S * c0z) * N + S * c0y) * pitch + S * c0x;
+  constexpr int PL = F * F, ZS = CIC_NT / PL;
+  static_assert(CIC_NT % PL == 0, "whole planes a round");
+  const int64_t ro = (int64_t)(tid / PL) * N * pitch + (int64_t)(tid / F % F) * pitch + tid % F;
+  if (PL * F >= CIC_NT || tid < PL * F) {
+#pragma unroll 4
+    for (int it = 0; it < (PL * F + CIC_NT - 1) / CIC_NT; it++) {
+      const double vd = (double)(long long)s[tid + it * CIC_NT] * (1.0 / CIC_FIX);
+      R0[ro + (int64_t)(it * ZS) * N * pitch] = (T)vd;
+      ms += vd;
+    }
   }
   for (int off2 = 32; off2 > 0; off2 >>= 1) ms += __shfl_xor(ms, off2);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ms;
+  if ((tid & 63) == 0) red[tid >> 6] = ms;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     double m = 0;
     for (int i = 0; i < CIC_NT / 64; i++) m += red[i];
     part[blockIdx.x] = m;
   }
 }
-
-// ------------------------------------------------------------ coarse CIC
-// Nodes at coarse-cell centres (pm.f90:255 '-0.5'); a particle in cell c
-// touches nodes c-1..c+1, so the block gathers cells [c0-1, c0+BC].
-template <int BC, typename T>
-__global__ __launch_bounds__(CIC_NT) void k_cic_coarse(Geo g, const void* __restrict__ xp, const int64_t* __restrict__ cstart,
-                                                       float mass_f, T* R, double* part) {
-  const T mass = (T)mass_f;
-  constexpr int SPAN = BC + 2, NCELL = SPAN * SPAN * SPAN;
-  __shared__ unsigned long long s[BC * BC * BC];
-  __shared__ int64_t beg[NCELL];
-  __shared__ int32_t off[NCELL + 1];
-  __shared__ double red[CIC_NT / 64];
-  const int nbx = g.nc / BC;
-  // XCD-contiguous block order: x neighbours, which write the two halves of
-  // shared 128-byte lines, run on one L2
-  const int lb = (int)xcd_remap(blockIdx.x, gridDim.x);
-  const int bx = lb % nbx, by = (lb / nbx) % nbx, bz = lb / (nbx * nbx);
-  const int c0x = bx * BC, c0y = by * BC, c0z = bz * BC;
-  const int l0x = c0x % g.nt, l0y = c0y % g.nt, l0z = c0z % g.nt;
-  for (int i = threadIdx.x; i < BC * BC * BC; i += CIC_NT) s[i] = 0ull;
-  load_region<SPAN>(g, cstart, c0x, c0y, c0z, 1, beg, off);
-  const int32_t total = off[NCELL];
-  for (int32_t t0 = threadIdx.x; t0 < total; t0 += CIC_NT * CIC_U) {
-    int cib[CIC_U];
-    uint32_t ub[CIC_U][3];
-#pragma unroll
-    for (int j = 0; j < CIC_U; j++) {
-      const int32_t t = t0 + j * CIC_NT;
-      cib[j] = t < total ? seg_find(off, NCELL, t) : 0;
-      const int64_t p = beg[cib[j]] + (t - off[cib[j]]);
-#pragma unroll
-      for (int e = 0; e < 3; e++) ub[j][e] = t < total ? load_xu(xp, 3 * p + e, g.izipx) : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < CIC_U; j++) {
-      if (t0 + j * CIC_NT >= total) break;
-      const int ci = cib[j];
-      int rel[3] = {ci % SPAN - 1, (ci / SPAN) % SPAN - 1, ci / (SPAN * SPAN) - 1};
-      int l0[3] = {l0x, l0y, l0z};
-      T dx1[3], dx2[3];
-      int n1[3];
-      for (int e = 0; e < 3; e++) {
-        int il = l0[e] + rel[e] + 1;
-        uint32_t u = ub[j][e];
-        T tx = (T)(((double)(il - 1) + xoff(u, g.izipx)) - 0.5);
-        int a1 = (int)floor(tx) + 1;  // 1-based tile-local node
-        dx1[e] = (T)a1 - tx;
-        dx2[e] = 1 - dx1[e];
-        n1[e] = (a1 - 1) - l0[e];
-      }
-      const T w[8] = {dx1[0] * dx1[1] * dx1[2] * mass, dx2[0] * dx1[1] * dx1[2] * mass,
-                      dx1[0] * dx2[1] * dx1[2] * mass, dx1[0] * dx1[1] * dx2[2] * mass,
-                      dx1[0] * dx2[1] * dx2[2] * mass, dx2[0] * dx1[1] * dx2[2] * mass,
-                      dx2[0] * dx2[1] * dx1[2] * mass, dx2[0] * dx2[1] * dx2[2] * mass};
-      const int o[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 1, 1}, {1, 0, 1}, {1, 1, 0}, {1, 1, 1}};
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        int x = n1[0] + o[q][0], y = n1[1] + o[q][1], z = n1[2] + o[q][2];
-        if ((unsigned)x < (unsigned)BC && (unsigned)y < (unsigned)BC && (unsigned)z < (unsigned)BC)
-          atomicAdd(&s[(z * BC + y) * BC + x], (unsigned long long)llrint((double)w[q] * CIC_FIX));
-      }
-    }
-  }
-  __syncthreads();
-  const int64_t N = g.nc;
-  double ms = 0;
-  for (int i = threadIdx.x; i < BC * BC * BC; i += CIC_NT) {
-    int x = i % BC, y = (i / BC) % BC, z = i / (BC * BC);
-    double vd = (double)(long long)s[i] * (1.0 / CIC_FIX);
-    R[((int64_t)(c0z + z) * N + (c0y + y)) * (N + 2) + (c0x + x)] = (T)vd;
-    ms += vd;
-  }
-  for (int off2 = 32; off2 > 0; off2 >>= 1) ms += __shfl_xor(ms, off2);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ms;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = 0;
-    for (int i = 0; i < CIC_NT / 64; i++) m += red[i];
-    part[blockIdx.x] = m;
-  }
+template <int BC, int S, bool CENTRE, typename T>
+static int cic_launch(cube_handle* h, T* R, int64_t N, int64_t pitch, int64_t* nblocks) {
+  const int64_t nb = (h->nc / BC) * (h->nc / BC) * (h->nc / BC);
+  if (nb > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
+  const Geo g = geo_of(h);
+  auto go = [&](auto kernel) {
+    kernel<<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, R, N, pitch, h->dred);
+  };
+  const bool fast = h->mass_p >= 0.f && h->mass_p <= 1024.f;
+  if (h->p.izipx == 1)
+    fast ? go(k_cic<BC, S, CENTRE, T, 1, true>) : go(k_cic<BC, S, CENTRE, T, 1, false>);
+  else
+    fast ? go(k_cic<BC, S, CENTRE, T, 2, true>) : go(k_cic<BC, S, CENTRE, T, 2, false>);
+  HIP_TRY(h, hipGetLastError());
+  *nblocks = nb;
+  return 0;
 }
 
 int cic_fine(cube_handle* h, double* mass, double* mass_dev) {
-  Geo g = geo_of(h);
   if (h->nt % 4) return cube_fail(h, CUBE_ERR_ARG, "nt=%lld must be a multiple of 4", (long long)h->nt);
-  int64_t nb = (h->nc / 4) * (h->nc / 4) * (h->nc / 4);
-  if (nb > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
+  int64_t nb = 0;
+  const int64_t N = h->fine.N;
   int pr = prof_begin(h, PS_CIC_F);
-  if (h->prec == 4)
-    k_cic_fine<4, float><<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, (float*)h->fine.R, h->fine.N,
-                                                                h->fine.N + 2, h->dred);
-  else
-    k_cic_fine<4, double><<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, (double*)h->fine.R, h->fine.N,
-                                                                 h->fine.N + 2, h->dred);
+  const int r = h->prec == 4 ? cic_launch<4, 4, false>(h, (float*)h->fine.R, N, N + 2, &nb)
+                             : cic_launch<4, 4, false>(h, (double*)h->fine.R, N, N + 2, &nb);
   prof_end(h, pr);
-  HIP_TRY(h, hipGetLastError());
+  if (r) return r;
   if (mass_dev) return reduce_doubles_dev(h, h->dred, nb, 1, mass_dev);
   if (mass) return reduce_doubles(h, h->dred, nb, 1, mass);
   return 0;
 }
 // halo-finder density at fine-cell centres into out (nf^3 float, pitch nf)
 int cic_halo_density(cube_handle* h, float* out) {
-  Geo g = geo_of(h);
   if (h->nt % 4) return cube_fail(h, CUBE_ERR_ARG, "nt=%lld must be a multiple of 4", (long long)h->nt);
-  int64_t nb = (h->nc / 4) * (h->nc / 4) * (h->nc / 4);
-  if (nb > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
-  k_cic_fine<4, float, true><<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, out, h->fine.N, h->fine.N,
-                                                                    h->dred);
-  HIP_TRY(h, hipGetLastError());
-  return 0;
+  int64_t nb = 0;
+  return cic_launch<4, 4, true>(h, out, h->fine.N, h->fine.N, &nb);
 }
+// small boxes take half-width blocks: 8^3 cells a workgroup leave 8 workgroups
+// at 16^3 cells and 64 at 32^3.  ms, 8^3 -> 4^3 cells a workgroup: 16^3 .049 ->
+// .014, 32^3 .055 -> .018, 64^3 .050 -> .045, 128^3 .176 -> .276 (a narrow
+// block gathers 3.4 particles for each of its own, a wide one 1.95).
 int cic_coarse(cube_handle* h, double* mass, double* mass_dev) {
-  Geo g = geo_of(h);
-  int64_t nb = (h->nc / 8) * (h->nc / 8) * (h->nc / 8);
+  int64_t nb = 0;
+  const int64_t N = h->coarse.N;
+  const bool few = h->nc <= CIC_FEW;
   int pr = prof_begin(h, PS_CIC_C);
+  int r;
   if (h->prec == 4)
-    k_cic_coarse<8, float><<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, (float*)h->coarse.R, h->dred);
+    r = few ? cic_launch<4, 1, true>(h, (float*)h->coarse.R, N, N + 2, &nb)
+            : cic_launch<8, 1, true>(h, (float*)h->coarse.R, N, N + 2, &nb);
   else
-    k_cic_coarse<8, double><<<(unsigned)nb, CIC_NT, 0, h->stream>>>(g, h->xp, h->cstart, h->mass_p, (double*)h->coarse.R, h->dred);
+    r = few ? cic_launch<4, 1, true>(h, (double*)h->coarse.R, N, N + 2, &nb)
+            : cic_launch<8, 1, true>(h, (double*)h->coarse.R, N, N + 2, &nb);
   prof_end(h, pr);
-  HIP_TRY(h, hipGetLastError());
+  if (r) return r;
   if (mass_dev) return reduce_doubles_dev(h, h->dred, nb, 1, mass_dev);
   if (mass) return reduce_doubles(h, h->dred, nb, 1, mass);
   return 0;
