@@ -76,44 +76,51 @@ static const CodecTables& codec_tables(int izipv) {
   });
   return tabs[izipv];
 }
-__global__ void k_fill_u32(uint32_t* p, int64_t n, uint32_t v) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
-}
-__global__ __launch_bounds__(256) void k_slots_reduce(const uint32_t* __restrict__ slots, int nf, uint32_t or_mask,
-                                                      uint32_t add_mask, uint32_t* out) {
-  __shared__ uint32_t red[256];
-  for (int f = 0; f < nf; f++) {
-    const bool is_or = (or_mask >> f) & 1, is_add = (add_mask >> f) & 1;
-    uint32_t a = 0;
-    for (int s = threadIdx.x; s < MSLOTS; s += 256) {
-      const uint32_t v = slots[s * MSLOT_FIELDS + f];
-      a = is_or ? (a | v) : (is_add ? a + v : max(a, v));
-    }
-    red[threadIdx.x] = a;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) {
-        const uint32_t b = red[threadIdx.x + o];
-        red[threadIdx.x] = is_or ? (red[threadIdx.x] | b) : (is_add ? red[threadIdx.x] + b : max(red[threadIdx.x], b));
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      if (is_or) atomicOr(out + f, red[0]);
-      else if (is_add) atomicAdd(out + f, red[0]);
-      else atomicMax(out + f, red[0]);
-    }
-    __syncthreads();
+__global__ void k_clear_u32(uint32_t* a, int64_t na, uint32_t* b, int64_t nb, uint32_t* c, int64_t nc) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < na + nb + nc; i += (int64_t)gridDim.x * blockDim.x) {
+    if (i < na) a[i] = 0u;
+    else if (i < na + nb) b[i - na] = 0u;
+    else c[i - na - nb] = 0u;
   }
 }
-int slots_reduce(cube_handle* h, int nf, uint32_t or_mask, uint32_t add_mask, uint32_t* out) {
-  k_slots_reduce<<<1, 256, 0, h->stream>>>(h->mslots, nf, or_mask, add_mask, out);
+// A wavefront per field (8.9 us with one workgroup reducing field after field
+// through LDS, half of it the launch).
+__global__ __launch_bounds__(64 * MSLOT_FIELDS) void k_slots_reduce(const uint32_t* __restrict__ slots, int nf, uint32_t or_mask,
+                                                                    uint32_t add_mask, uint32_t* out, uint32_t* rep, int lead,
+                                                                    int nrep) {
+  const int f = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  uint32_t v = 0;
+  if (f < nf) {
+    const bool is_or = (or_mask >> f) & 1, is_add = (add_mask >> f) & 1;
+    auto fold = [&](uint32_t x, uint32_t y) { return is_or ? (x | y) : (is_add ? x + y : max(x, y)); };
+    uint32_t a[MSLOTS / 64];
+#pragma unroll
+    for (int k = 0; k < MSLOTS / 64; k++) a[k] = slots[(k * 64 + lane) * MSLOT_FIELDS + f];
+#pragma unroll
+    for (int k = 0; k < MSLOTS / 64; k++) v = fold(v, a[k]);
+    for (int o = 32; o > 0; o >>= 1) v = fold(v, __shfl_xor(v, o));
+    if (lane == 0) {
+      v = fold(v, out[f]);
+      out[f] = v;
+    }
+  } else if (rep && f < nrep - lead && lane == 0) {
+    v = out[f];
+  }
+  if (rep && lane == 0) {
+    if (f < nrep - lead) rep[lead + f] = v;
+    if (f < lead) rep[f] = out[f - lead];
+  }
+}
+int slots_reduce(cube_handle* h, int nf, uint32_t or_mask, uint32_t add_mask, uint32_t* out, uint32_t* rep, int lead, int nrep) {
+  if (nf > MSLOT_FIELDS || lead > MSLOT_FIELDS || nrep - lead > MSLOT_FIELDS) return cube_fail(h, CUBE_ERR_ARG, "slot fields");
+  k_slots_reduce<<<1, 64 * MSLOT_FIELDS, 0, h->stream>>>(h->mslots, nf, or_mask, add_mask, out, rep, lead, nrep);
   HIP_TRY(h, hipGetLastError());
   return 0;
 }
-int fill_u32(cube_handle* h, void* p, int64_t n, uint32_t v) {
-  const int64_t nb = std::min<int64_t>((n + 255) / 256, 4096);
-  k_fill_u32<<<(unsigned)std::max<int64_t>(nb, 1), 256, 0, h->stream>>>((uint32_t*)p, n, v);
+int clear_u32(cube_handle* h, U32Run a, U32Run b, U32Run c) {
+  const int64_t nb = std::min<int64_t>((a.n + b.n + c.n + 255) / 256, 4096);
+  k_clear_u32<<<(unsigned)std::max<int64_t>(nb, 1), 256, 0, h->stream>>>((uint32_t*)a.p, a.n, (uint32_t*)b.p, b.n,
+                                                                         (uint32_t*)c.p, c.n);
   HIP_TRY(h, hipGetLastError());
   return 0;
 }
@@ -121,30 +128,31 @@ __global__ void k_vtab_fill(const float* __restrict__ dec, int n, double c, doub
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = (double)dec[i] / c;
 }
+// Three tables: the kick needs the old- and the new-sigma one at once, and a
+// drift writes the next sigma's while the step still reads the old one; after
+// the step that table is the old-sigma one and is not formed again.
 const double* vtab_for(cube_handle* h, double c) {
   const int n = h->p.izipv == 1 ? 256 : 65536;
-  // two slots, least recently used replaced: the kick needs the old- and
-  // new-sigma tables at once
-  for (int s = 0; s < 2; s++)
+  for (int s = 0; s < 3; s++)
     if (h->vdt_c[s] == c) {
-      h->vdt_next = s ^ 1;
-      return h->vdt + (size_t)s * n;
+      h->vdt_old = s;
+      return h->vdt_at(s);
     }
-  const int s = h->vdt_next;
-  h->vdt_next = s ^ 1;
-  k_vtab_fill<<<(n + 255) / 256, 256, 0, h->stream>>>(h->vdec, n, c, h->vdt + (size_t)s * n);
+  int s = 0;  // neither the newest table nor the last given
+  while (s == h->vdt_ni || s == h->vdt_old) s++;
+  k_vtab_fill<<<(n + 255) / 256, 256, 0, h->stream>>>(h->vdec, n, c, h->vdt_at(s));
   h->vdt_c[s] = c;
-  return h->vdt + (size_t)s * n;
+  h->vdt_old = s;
+  return h->vdt_at(s);
 }
 int codec_build(cube_handle* h) {
   const CodecTables& t = codec_tables((int)h->p.izipv);
   HIP_TRY(h, hipMalloc(&h->vdec, sizeof(float) * t.dec.size()));
   HIP_TRY(h, hipMalloc(&h->venc, sizeof(double) * t.thr.size()));
-  HIP_TRY(h, hipMalloc(&h->vdt, sizeof(double) * 2 * t.dec.size()));
+  HIP_TRY(h, hipMalloc(&h->vdt, sizeof(double) * 3 * t.dec.size()));
   HIP_TRY(h, hipMemcpy(h->vdec, t.dec.data(), sizeof(float) * t.dec.size(), hipMemcpyHostToDevice));
   HIP_TRY(h, hipMemcpy(h->venc, t.thr.data(), sizeof(double) * t.thr.size(), hipMemcpyHostToDevice));
   h->vkmax = t.kmax;
-  HIP_TRY(h, hipMalloc(&h->vdt_new, sizeof(double) * t.dec.size()));
   HIP_TRY(h, hipMalloc(&h->dscal, sizeof(double) * 4));
   HIP_TRY(h, hipMalloc(&h->drep, sizeof(StepReport)));
   HIP_TRY(h, hipMalloc(&h->dred_l1, sizeof(double) * 256 * 8));  // first-level sums (scan.hip)
@@ -225,7 +233,7 @@ extern "C" int cube_init(const cube_params* p, const float* kern_f_table, const 
 #undef TRY
   if ((rc = codec_build(h))) return fail(rc);
   if ((rc = mesh_alloc(h, h->fine, h->nf, h->prec, true, true))) return fail(rc);
-  if ((rc = mesh_alloc(h, h->coarse, h->nc, h->prec, false, true))) return fail(rc);
+  if ((rc = mesh_alloc(h, h->coarse, h->nc, h->prec, false, true, false))) return fail(rc);
   // the fine work mesh is idle during the drift and serves as its scratch
   // (crowded-cell merges, then three doubles per particle)
   if (h->fine.bytes_R() >= 3 * sizeof(double) * (size_t)npm) {
@@ -304,7 +312,7 @@ extern "C" int cube_finalize(cube_handle* h) {
   if (h->rep) (void)hipHostFree(h->rep);
   void* bufs[] = {h->xp, h->vp, h->pid, h->xp2, h->vp2, h->pid2, h->disp, h->order, h->rhoc, h->rhoc2, h->vfield, h->vfield2,
                   h->cstart, h->cstart2, h->fc, h->dred, h->uflags, h->scan_tmp, h->vdec, h->venc, h->vdt, h->dbig,
-                  h->dscratch_own ? h->dscratch : nullptr, h->pp_meta, h->pp_red, h->vdt_new, h->dscal, h->drep, h->dred_l1, h->mslots};
+                  h->dscratch_own ? h->dscratch : nullptr, h->pp_meta, h->pp_red, h->dscal, h->drep, h->dred_l1, h->mslots};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   mesh_free(h->fine);
@@ -411,6 +419,11 @@ extern "C" int cube_pp(cube_handle* h, float a_mid, float dt, cube_pp_out* out) 
   return r;
 }
 
+// A small box's step is bound by its launches, 4.5 us each whatever they do
+// and as much again of the host's capture and graph update: clears share a
+// launch, reductions put their results into the report themselves, the three
+// coarse components and the three y inversions go together (57 launches a step
+// -> 39; 24 steps of a 32^3-particle box 9.35 -> 7.34 ms, 16 of 64^3 8.2 -> 7.5).
 // particle_mesh (pm.f90:2-443) as one launch sequence; the masses, f2
 // maxima and vmax go to h->drep for pm_finish
 static int pm_launch(cube_handle* h, float a_mid, float dt, double* probe_f, double* probe_c) {
@@ -419,24 +432,17 @@ static int pm_launch(cube_handle* h, float a_mid, float dt, double* probe_f, dou
   uint32_t* f2f = h->uflags + 33;
   uint32_t* vmx = h->uflags + 34;  // 3 entries
   StepReport* dr = h->drep;
-  if ((r = fill_u32(h, h->uflags + 32, 8, 0u))) return r;
+  if ((r = clear_u32(h, {h->uflags + 32, 8}, {h->mslots, MSLOTS * MSLOT_FIELDS}))) return r;
   const bool nu = h->nu.on;
-  // coarse mesh: force_c for all three components (pm.f90:188-326); the
-  // third inverse also forms max |force_c|^2 from the two already written
+  // coarse mesh: force_c for all three components (pm.f90:188-326), their
+  // spectra in the idle fine work mesh
   if ((r = cic_coarse(h, nullptr, &dr->mass[0]))) return r;
   int prd = nu ? prof_begin(h, PS_FLUID_DENS) : -1;
   if (nu && (r = fl_density_coarse(h, a_mid, nullptr, &dr->mass[1]))) return r;
   if (nu) prof_end(h, prd);
   if ((r = mesh_fwd_xy(h, h->coarse))) return r;
-  const int64_t Nc = h->coarse.N;
-  const char* fc = (const char*)h->fc;
-  const size_t fcs = (size_t)h->n3c * h->prec;
-  for (int d = 0; d < 3; d++) {
-    if ((r = mesh_zconv(h, h->coarse, d, h->coarse.W))) return r;
-    if ((r = mesh_inv_yx(h, h->coarse, h->coarse.W, (void*)(fc + d * fcs), Nc, fc, Nc, fc + fcs, Nc,
-                         d == 2 ? f2c : nullptr)))
-      return r;
-  }
+  if (h->fine.bytes_big() < 3 * h->coarse.bytes_R()) return cube_fail(h, CUBE_ERR_ARG, "fine work mesh below three coarse spectra");
+  if ((r = mesh_conv3(h, h->coarse, h->fine.X, h->fc, f2c))) return r;
   // fine mesh, kx-tiled spectrum: the density in R goes to a tiled
   // spectrum in W.  FP32 meshes of 32^3 and up: one z pass convolves all
   // three components into X, R and W (the spectrum's last use), and each is
@@ -457,14 +463,15 @@ static int pm_launch(cube_handle* h, float a_mid, float dt, double* probe_f, dou
     void* const spec[3] = {h->fine.X, h->fine.R, h->fine.W};
     Fw[0] = h->fine.S, Fw[1] = h->fine.X, Fw[2] = h->fine.R;
     if ((r = mesh_t_zconv3(h, h->fine, h->fine.W, spec))) return r;
+    if ((r = mesh_t_inv_y(h, h->fine, spec, 3))) return r;
     for (int d = 0; d < 3; d++)
-      if ((r = mesh_t_inv(h, h->fine, spec[d], Fw[d], pf[d]))) return r;
+      if ((r = mesh_t_inv_x(h, h->fine, spec[d], Fw[d], pf[d]))) return r;
   } else {
     Fw[0] = h->fine.S, Fw[1] = h->fine.R, Fw[2] = h->fine.X;
     for (int d = 0; d < 3; d++) {
       void* spec = d == 2 ? h->fine.W : h->fine.X;
       if ((r = mesh_t_zconv(h, h->fine, d, h->fine.W, spec))) return r;
-      if ((r = mesh_t_inv(h, h->fine, spec, Fw[d], pf[d]))) return r;
+      if ((r = mesh_t_inv_y(h, h->fine, &spec, 1)) || (r = mesh_t_inv_x(h, h->fine, spec, Fw[d], pf[d]))) return r;
     }
   }
   const void* Ff[3] = {Fw[0], Fw[1], Fw[2]};
@@ -477,7 +484,6 @@ static int pm_launch(cube_handle* h, float a_mid, float dt, double* probe_f, dou
   if (nu_kick && (r = fl_gravity_fine(h, Ff, pf, a_mid, dt))) return r;
   if (nu_kick && (r = fl_gravity_finish(h, Fw, pf, a_mid, dt))) return r;
   if (nu_kick) prof_end(h, prg);
-  HIP_TRY(h, hipMemcpyAsync(dr->pmflags, h->uflags + 32, sizeof(dr->pmflags), hipMemcpyDeviceToDevice, h->stream));
   return 0;
 }
 

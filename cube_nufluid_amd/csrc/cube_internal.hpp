@@ -1,6 +1,7 @@
 // Internal declarations shared by the HIP translation units of libcubehip.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <mutex>
 #include <shared_mutex>
@@ -39,7 +40,7 @@ struct Mesh {
   int64_t N = 0;
   int prec = 4;          // sizeof(real)
   void* R = nullptr;     // real N*N*(N+2) padded rows; complex view N*N*(N/2+1)
-  void* W = nullptr;     // complex work, same size as R
+  void* W = nullptr;     // (fine, initial conditions) complex work, bytes_big()
   void* S = nullptr;     // unpadded N^3 real mesh (fine: force component 0)
   void* X = nullptr;     // (fine) second spectrum / real work mesh, bytes_big()
   void* K = nullptr;     // kernel [3][H][H][H], layout [d][ky'][kx][kz'], scaled 1/N^3
@@ -107,9 +108,11 @@ struct cube_handle {
   int32_t* rhoc2 = nullptr; float* vfield2 = nullptr; int64_t* cstart2 = nullptr;
   // codec tables
   float* vdec = nullptr;      // tanf((pi*vp)/(nvbin-1)) for every code
-  double* vdt = nullptr;      // two decoded-velocity tables (vdec/c), see vtab_for
-  double vdt_c[2] = {0, 0};
-  int vdt_next = 0;
+  double* vdt = nullptr;      // three decoded-velocity tables (vdec/c), see vtab_for
+  double vdt_c[3] = {NAN, NAN, NAN};  // their coefficients (NaN: unknown)
+  int vdt_old = 0;            // the table vtab_for gave last
+  int vdt_ni = 2;             // the table of dscal[0]
+  double* vdt_at(int s) const { return vdt + (size_t)s * (p.izipv == 1 ? 256 : 65536); }
   double* venc = nullptr;     // encode thresholds (see codec.cpp)
   int32_t vkmax = 0;          // largest |code| produced by the encoder
   // meshes
@@ -127,12 +130,11 @@ struct cube_handle {
   int64_t* scan_tmp = nullptr;
   int64_t scan_tmp_n = 0;
   // step report (device) and its pinned host copy; the new-sigma velocity
-  // coefficient and decode table, formed on the device by the drift and
-  // read by the kick
+  // coefficient and decode table (vdt_at(vdt_ni)), formed on the device by the
+  // drift and read by the kick
   StepReport* drep = nullptr;
   StepReport* rep = nullptr;
   double* dscal = nullptr;    // [0] vcoef(sigma_vi_new)
-  double* vdt_new = nullptr;  // decoded-velocity table for dscal[0]
   // step mode: 0 each call synchronises; 1 drift, PP and PM are launched
   // back to back and checked after one synchronisation; 2 as 1, the
   // launches captured into a hipGraph and replayed (kernel arguments
@@ -182,18 +184,21 @@ int cube_fail(cube_handle* h, int code, const char* fmt, ...);
 
 // ------------------------------------------------------------- codec (host)
 int codec_build(cube_handle* h);  // vdec/venc tables from the host libm
-// dscal[0] and vdt_new from the host's sigma_vi_new (after an upload, an IC
+// dscal[0] and its table from the host's sigma_vi_new (after an upload, an IC
 // or a failed drift); the drift forms them on the device otherwise
 int sigma_new_to_device(cube_handle* h);
-// fill n 32-bit words with v on the handle's stream (a kernel, so that a
-// captured step holds no memset node)
-int fill_u32(cube_handle* h, void* p, int64_t n, uint32_t v);
+// clear three runs of 32-bit words on the handle's stream in one launch (a
+// kernel, so that a captured step holds no memset node)
+struct U32Run { void* p = nullptr; int64_t n = 0; };
+int clear_u32(cube_handle* h, U32Run a, U32Run b = {}, U32Run c = {});
 #define MSLOTS 1024
 #define MSLOT_FIELDS 8
 // out[f] (f < nf) combined with the fold of field f over the MSLOTS slots
 // (slot s, field f at slots[s * MSLOT_FIELDS + f]): OR where bit f of
-// or_mask is set, sum where bit f of add_mask is, max otherwise
-int slots_reduce(cube_handle* h, int nf, uint32_t or_mask, uint32_t add_mask, uint32_t* out);
+// or_mask is set, sum where bit f of add_mask is, max otherwise.  With rep,
+// the `lead` words before out and the nrep - lead from it go to rep as well.
+int slots_reduce(cube_handle* h, int nf, uint32_t or_mask, uint32_t add_mask, uint32_t* out, uint32_t* rep = nullptr,
+                 int lead = 0, int nrep = 0);
 // While one thread captures a step into a hipGraph, no other thread may run
 // a legacy-stream operation (synchronous copies and memsets) or a
 // device-synchronising one (hipFree): the runtime rejects them.  Captures
@@ -425,7 +430,7 @@ __device__ __forceinline__ int32_t venc_fast(const double* thr, const double* at
 }
 
 // ------------------------------------------------------------- launchers
-// decoded-velocity table for coefficient c (one of two cached slots)
+// decoded-velocity table for coefficient c (one of three kept)
 const double* vtab_for(cube_handle* h, double c);
 // scan.hip
 int scan_counts(cube_handle* h, const int32_t* cnt, int64_t n, int64_t* cstart);
@@ -433,28 +438,27 @@ int reduce_doubles(cube_handle* h, const double* part, int64_t nparts, int nfiel
 // the same fixed-order sums into device memory, no synchronisation
 int reduce_doubles_dev(cube_handle* h, const double* part, int64_t nparts, int nfields, double* dev_out);
 // fft.hip
-int mesh_alloc(cube_handle* h, Mesh& m, int64_t N, int prec, bool with_S, bool with_K);
+int mesh_alloc(cube_handle* h, Mesh& m, int64_t N, int prec, bool with_S, bool with_K, bool with_W = true);
 int mesh_pass(cube_handle* h, Mesh& m, void* buf, int axis, bool inverse);    // strided y (1) / z (2) pass
 int mesh_c2r(cube_handle* h, Mesh& m, const void* src, void* dst, int64_t opitch);
 void mesh_free(Mesh& m);
 int mesh_fwd_xy(cube_handle* h, Mesh& m);                  // R: X r2c then Y, in place
-// dst (R or W) = Zinv(i*K_d * Zfwd(R))
-int mesh_zconv(cube_handle* h, Mesh& m, int d, void* dst);
-// buf (R or W): Y inverse in place, then X c2r into out (row pitch opitch);
-// with f2max, also max(F0^2+F1^2+F2^2) from the other two components
-int mesh_inv_yx(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch, const void* F0, int64_t p0,
-                const void* F1, int64_t p1, uint32_t* f2max);
+// the three force components from the spectrum in R: spec[d] = Zinv(i*K_d *
+// Zfwd(R)) in three spectra of bytes_R() each from spec, Y inverse in place, X
+// c2r into out[d] (rows of N) from out, max(F0^2+F1^2+F2^2) into *f2max
+int mesh_conv3(cube_handle* h, Mesh& m, void* spec, void* out, uint32_t* f2max);
 int mesh_fft3_r2c(cube_handle* h, Mesh& m);                  // full forward on R (for kernel build)
 // kx-tiled spectrum pipeline (fine mesh, per step): real rows src (pitch
 // N+2) -> tiled spectrum dst with the y transform; z convolution src ->
-// dst (may alias); y inverse in place then C2R into out (pitch opitch)
+// dst (may alias); y inverse in place (of n spectra), then C2R into out (pitch opitch)
 int mesh_t_fwd(cube_handle* h, Mesh& m, const void* src, void* dst);
 int mesh_t_zconv(cube_handle* h, Mesh& m, int d, const void* src, void* dst);
 // all three components of the fine convolution from one read of src
 // (FP32 meshes of 32^3 and up: mesh_t_zconv3_fits)
 bool mesh_t_zconv3_fits(const Mesh& m);
 int mesh_t_zconv3(cube_handle* h, Mesh& m, const void* src, void* const dst[3]);
-int mesh_t_inv(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch);
+int mesh_t_inv_y(cube_handle* h, Mesh& m, void* const* buf, int n);
+int mesh_t_inv_x(cube_handle* h, Mesh& m, const void* buf, void* out, int64_t opitch);
 int fine_kernel_build(cube_handle* h, const float* table);
 int coarse_kernel_build(cube_handle* h, const float* table);
 // pm.hip
@@ -465,7 +469,8 @@ int pk_scratch_setup(cube_handle* h);  // device address of the P(k) scratch arr
 int cic_coarse(cube_handle* h, double* mass, double* mass_dev = nullptr);
 // fine force components Ff[d] (row pitch pf[d]) and the coarse force fc
 // f2max_bits (optional): max |F|^2 over all fine nodes, from the staged slabs
-// new-sigma coefficient and table from h->dscal / h->vdt_new
+// new-sigma coefficient and table from h->dscal and the handle's newest table;
+// h->mslots zero before; the maxima go to the report as well
 int kick_all(cube_handle* h, const void* const Ff[3], const int64_t pf[3], float a_mid, float dt, double c_old,
              uint32_t* vmax_bits, uint32_t* f2max_bits, double* probe_f, double* probe_c);
 // pp.hip

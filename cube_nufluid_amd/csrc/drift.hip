@@ -650,25 +650,34 @@ __global__ __launch_bounds__(DR_NT) void k_drift_write(Geo g, const uint64_t* __
 }
 
 // sigma_vi_new = sqrt(sum v_res^2 / N) / sqrt(3) (update_particle.f90:213,
-// in the host's operation order) and the new velocity coefficient
-// vcoef(sigma_vi_new) = sqrt(pi/2) / (sigma * 2.5), formed on the device so
-// that the kick can read them without a host round trip
-__global__ void k_sigma_new(const double* __restrict__ dsum, double npg, float sqrt3f, float sqrtpi2f, float* sigma_out,
-                            double* cnew_out) {
-  const float sg = (float)(sqrt(dsum[1] / npg) / (double)sqrt3f);
-  *sigma_out = sg;
-  *cnew_out = (double)sqrtpi2f / ((double)sg * 2.5);
-}
-__global__ void k_vtab_fill_dev(const float* __restrict__ dec, int n, const double* __restrict__ c, double* out) {
+// in the host's operation order), the new velocity coefficient
+// vcoef(sigma_vi_new) = sqrt(pi/2) / (sigma * 2.5) and its decode table, formed
+// on the device so that the kick can read them without a host round trip; the
+// first workgroup also puts the drift's flags and count into the report
+__global__ void k_sigma_new(StepReport* d, const uint32_t* __restrict__ flags, const int64_t* __restrict__ npnew, double npg,
+                            float sqrt3f, float sqrtpi2f, double* cnew_out, const float* __restrict__ dec, int n, double* out) {
+  const float sg = (float)(sqrt(d->dsum[1] / npg) / (double)sqrt3f);
+  const double c = (double)sqrtpi2f / ((double)sg * 2.5);
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (double)dec[i] / *c;
+  if (i < n) out[i] = (double)dec[i] / c;
+  if (i < (int)(sizeof(d->dflags) / 4)) d->dflags[i] = flags[i];
+  if (i == 0) {
+    d->sigma_new = sg;
+    d->npnew = *npnew;
+    *cnew_out = c;
+  }
 }
-__global__ void k_set_double(double* p, double v) { *p = v; }
+__global__ void k_vtab_fill_dev(const float* __restrict__ dec, int n, double c, double* c_out, double* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = (double)dec[i] / c;
+  if (i == 0) *c_out = c;
+}
 
 int sigma_new_to_device(cube_handle* h) {
   const int n = h->p.izipv == 1 ? 256 : 65536;
-  k_set_double<<<1, 1, 0, h->stream>>>(h->dscal, vcoef(h->sigma_vi_new));
-  k_vtab_fill_dev<<<(n + 255) / 256, 256, 0, h->stream>>>(h->vdec, n, h->dscal, h->vdt_new);
+  const double c = vcoef(h->sigma_vi_new);
+  k_vtab_fill_dev<<<(n + 255) / 256, 256, 0, h->stream>>>(h->vdec, n, c, h->dscal, h->vdt_at(h->vdt_ni));
+  h->vdt_c[h->vdt_ni] = c;
   HIP_TRY(h, hipGetLastError());
   return 0;
 }
@@ -697,9 +706,7 @@ static int drift_launch(cube_handle* h, float dt_old, float dt, int* nlayer_out)
   const int64_t nbw = (h->n3c + dwc - 1) / dwc;
   if (nbw * 3 > h->dred_n - 16) return cube_fail(h, CUBE_ERR_ARG, "reduction buffer too small");
   int r;
-  if ((r = fill_u32(h, flags, 8, 0u)) || (r = fill_u32(h, h->rhoc2, h->n3c, 0u)) ||
-      (r = fill_u32(h, h->mslots, MSLOTS * MSLOT_FIELDS, 0u)))
-    return r;
+  if ((r = clear_u32(h, {flags, 8}, {h->mslots, MSLOTS * MSLOT_FIELDS}, {h->rhoc2, h->n3c}))) return r;
   int pid1 = prof_begin(h, PS_DRIFT1);
   auto* pass1 = few ? k_drift_pass1<32> : k_drift_pass1<256>;
   pass1<<<(unsigned)nb1, DR_NT, 0, h->stream>>>(g, h->xp, h->vp, h->cstart, h->n3c, h->vfield, dt_mid, c_old, vdt, dmax,
@@ -734,11 +741,13 @@ static int drift_launch(cube_handle* h, float dt_old, float dt, int* nlayer_out)
   StepReport* d = h->drep;
   if ((r = reduce_doubles_dev(h, h->dred, nbw, 3, d->dsum))) return r;
   const int n = h->p.izipv == 1 ? 256 : 65536;
-  k_sigma_new<<<1, 1, 0, h->stream>>>(d->dsum, (double)h->np, sqrtf(3.0f), sqrtf(PI_F / 2), &d->sigma_new, h->dscal);
-  k_vtab_fill_dev<<<(n + 255) / 256, 256, 0, h->stream>>>(h->vdec, n, h->dscal, h->vdt_new);
+  int s = 0;  // the table neither of this step's old sigma nor of the last new one
+  while (s == h->vdt_ni || s == h->vdt_old) s++;
+  h->vdt_ni = s;
+  h->vdt_c[s] = NAN;  // known once the report is
+  k_sigma_new<<<(n + 255) / 256, 256, 0, h->stream>>>(d, flags, h->cstart2 + h->n3c, (double)h->np, sqrtf(3.0f), sqrtf(PI_F / 2),
+                                                      h->dscal, h->vdec, n, h->vdt_at(s));
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(&d->npnew, h->cstart2 + h->n3c, sizeof(int64_t), hipMemcpyDeviceToDevice, h->stream));
-  HIP_TRY(h, hipMemcpyAsync(d->dflags, flags, sizeof(d->dflags), hipMemcpyDeviceToDevice, h->stream));
   std::swap(h->xp, h->xp2);
   std::swap(h->vp, h->vp2);
   std::swap(h->pid, h->pid2);
@@ -789,6 +798,7 @@ int drift_finish(cube_handle* h, const StepReport* rp, int nlayer, cube_drift_ou
   double std_vsim_c = sqrt(rp->dsum[0] / (double)h->nc / (double)h->nc / (double)h->nc);
   double std_vsim_res = sqrt(rp->dsum[1] / npg);
   h->sigma_vi_new = rp->sigma_new;
+  h->vdt_c[h->vdt_ni] = vcoef(h->sigma_vi_new);
   if (out) {
     out->sigma_vi_new = h->sigma_vi_new;
     out->nlayer = nlayer;

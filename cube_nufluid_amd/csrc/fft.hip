@@ -231,19 +231,16 @@ __global__ __launch_bounds__(NT_FFT) void k_fft_x_r2c(cpx<T>* data, const cpx<T>
 
 // ------------------------------------------------------------------ X C2R
 // rows of N/2+1 complex (src) -> N reals at dst[row*opitch + x] (src may be
-// dst: every row is read into LDS before it is written).  With f2max set,
-// the other two force components F0, F1 (row pitches p0, p1) are read at the
-// same nodes and max(F0^2 + F1^2 + f^2), summed in float in component
-// order, goes into *f2max as float bits.
+// dst: every row is read into LDS before it is written); mesh blockIdx.z of
+// those ss and ds apart.
 template <typename T, int LOGN>
-__global__ __launch_bounds__(NT_FFT) void k_fft_x_c2r(const cpx<T>* src, T* dst, int64_t opitch,
-                                                       const cpx<T>* __restrict__ tw, int64_t nrows,
-                                                       const T* __restrict__ F0, int64_t p0,
-                                                       const T* __restrict__ F1, int64_t p1, uint32_t* f2max) {
+__global__ __launch_bounds__(NT_FFT) void k_fft_x_c2r(const cpx<T>* src, int64_t ss, T* dst, int64_t ds, int64_t opitch,
+                                                       const cpx<T>* __restrict__ tw, int64_t nrows) {
   constexpr int N = 1 << LOGN, H = N / 2, W = pick_w<T>(LOGN - 1), LD = W + 1;
   __shared__ cpx<T> s[H * LD];
   __shared__ cpx<T> xnyq[W];
-  __shared__ float red[NT_FFT / 64];
+  src += blockIdx.z * ss;
+  dst += blockIdx.z * ds;
   const int64_t r0 = (int64_t)blockIdx.x * W;
   {
     // all loads of a thread are issued before its LDS stores
@@ -289,52 +286,32 @@ __global__ __launch_bounds__(NT_FFT) void k_fft_x_c2r(const cpx<T>* src, T* dst,
   }
   __syncthreads();
   lds_fft<T, H, W, true, LD>(s, tw, 2);
-  float mymax = 0.f;
-  if (!f2max) {
-    for (int idx = threadIdx.x; idx < H * W; idx += NT_FFT) {
-      int w = idx / H, m = idx % H;
-      int64_t row = r0 + w;
-      if (row < nrows) *reinterpret_cast<cpx<T>*>(dst + row * opitch + 2 * m) = s[m * LD + w];
-    }
-  } else {
-    // groups of FG nodes: their F0, F1 loads are issued together
-    constexpr int PER = H * W / NT_FFT, FG = PER < 8 ? PER : 8;
-    static_assert(PER % FG == 0, "whole groups");
-    for (int q0 = 0; q0 < PER; q0 += FG) {
-      cpx<T> a[FG], b[FG];
-#pragma unroll
-      for (int q = 0; q < FG; q++) {
-        const int idx = threadIdx.x + (q0 + q) * NT_FFT, w = idx / H, m = idx % H;
-        const int64_t row = r0 + w < nrows ? r0 + w : nrows - 1;
-        a[q] = *reinterpret_cast<const cpx<T>*>(F0 + row * p0 + 2 * m);
-        b[q] = *reinterpret_cast<const cpx<T>*>(F1 + row * p1 + 2 * m);
-      }
-#pragma unroll
-      for (int q = 0; q < FG; q++) {
-        const int idx = threadIdx.x + (q0 + q) * NT_FFT, w = idx / H, m = idx % H;
-        const int64_t row = r0 + w;
-        if (row >= nrows) continue;
-        const cpx<T> z = s[m * LD + w];
-        *reinterpret_cast<cpx<T>*>(dst + row * opitch + 2 * m) = z;
-        float s0 = (float)a[q].x * (float)a[q].x, s1 = (float)a[q].y * (float)a[q].y;
-        s0 = fmaf((float)b[q].x, (float)b[q].x, s0);
-        s1 = fmaf((float)b[q].y, (float)b[q].y, s1);
-        s0 = fmaf((float)z.x, (float)z.x, s0);
-        s1 = fmaf((float)z.y, (float)z.y, s1);
-        mymax = fmaxf(mymax, fmaxf(s0, s1));
-      }
-    }
+  for (int idx = threadIdx.x; idx < H * W; idx += NT_FFT) {
+    int w = idx / H, m = idx % H;
+    int64_t row = r0 + w;
+    if (row < nrows) *reinterpret_cast<cpx<T>*>(dst + row * opitch + 2 * m) = s[m * LD + w];
   }
-  if (f2max) {
-    for (int off = 32; off > 0; off >>= 1) mymax = fmaxf(mymax, __shfl_xor(mymax, off));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mymax;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      float m = red[0];
-      for (int i = 1; i < NT_FFT / 64; i++) m = fmaxf(m, red[i]);
-      atomicMax(f2max, __float_as_uint(m));
-    }
+}
+
+// max(F0^2 + F1^2 + F2^2) over n nodes, summed in float in component order,
+// into *f2max as float bits (F: the three components one after the other)
+template <typename T>
+__global__ __launch_bounds__(256) void k_f2_max(const T* __restrict__ F, int64_t n, uint32_t* f2max) {
+  __shared__ float red[4];
+  float m = 0.f;
+  const int64_t step = (int64_t)gridDim.x * 256;
+#pragma unroll 4
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
+    const float a = (float)F[i], b = (float)F[n + i], c = (float)F[2 * n + i];
+    float s = a * a;
+    s = fmaf(b, b, s);
+    s = fmaf(c, c, s);
+    m = fmaxf(m, s);
   }
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(f2max, __float_as_uint(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]))));
 }
 
 // Load W columns of N complex values at stride `stride` into s[n*W + w]
@@ -357,16 +334,17 @@ __device__ __forceinline__ void col_load(cpx<T>* s, const cpx<T>* __restrict__ s
 
 // ----------------------------------------------------------- strided Y / Z
 // AXIS 1: columns along y (stride H+1) in plane by = z.
-// AXIS 2: columns along z (stride N(H+1)) at by = y; (bx, by) is the XCD-remapped block.
+// AXIS 2: columns along z (stride N(H+1)) at by = y; (bx, by) is the XCD-remapped block;
+// mesh blockIdx.z of those ms apart.
 template <typename T, int LOGN, int AXIS, bool INV>
-__global__ __launch_bounds__(NT_FFT) void k_fft_strided(cpx<T>* data, const cpx<T>* __restrict__ tw) {
+__global__ __launch_bounds__(NT_FFT) void k_fft_strided(cpx<T>* data, int64_t ms, const cpx<T>* __restrict__ tw) {
   constexpr int N = 1 << LOGN, KX = N / 2 + 1, W = pick_w<T>(LOGN);
   __shared__ cpx<T> s[N * W];
   int bx, by;
   grid_block_xy(bx, by);
   const int kx0 = bx * W;
   const int64_t stride = AXIS == 1 ? (int64_t)KX : (int64_t)N * KX;
-  const int64_t base = AXIS == 1 ? (int64_t)by * N * KX + kx0 : (int64_t)by * KX + kx0;
+  const int64_t base = (AXIS == 1 ? (int64_t)by * N * KX + kx0 : (int64_t)by * KX + kx0) + blockIdx.z * ms;
   col_load<T, N, W>(s, data + base, stride, KX - kx0);
   lds_fft<T, N, W, INV>(s, tw, 1);
   for (int idx = threadIdx.x; idx < N * W; idx += NT_FFT) {
@@ -376,20 +354,22 @@ __global__ __launch_bounds__(NT_FFT) void k_fft_strided(cpx<T>* data, const cpx<
 }
 
 // ------------------------------------------------------ fused Z convolution
-// dst = Zinv( i*K_d . Zfwd(src) ) along z for columns (kx0.., ky = by).
-// dst may be src: a workgroup reads all its columns before writing them.
+// dst_d = Zinv( i*K_d . Zfwd(src) ) along z for columns (kx0.., ky = by) and
+// component d = blockIdx.z; the dst_d lie ds apart and away from src.
 // K is the imaginary part of the kernel transform over one octant,
 // [d][ky'][kx][kz'] with ky'=min(ky,N-ky), kz'=min(kz,N-kz); component d is
 // odd in its own axis and even in the other two.
 template <typename T, int LOGN>
-__global__ __launch_bounds__(NT_FFT) void k_fft_zconv(const cpx<T>* src, cpx<T>* dst, const T* __restrict__ K,
-                                                       int d, const cpx<T>* __restrict__ tw) {
+__global__ __launch_bounds__(NT_FFT) void k_fft_zconv(const cpx<T>* src, cpx<T>* dst, int64_t ds, const T* __restrict__ K,
+                                                       const cpx<T>* __restrict__ tw) {
   constexpr int N = 1 << LOGN, KX = N / 2 + 1, H = N / 2 + 1, W = pick_w<T>(LOGN);
   __shared__ cpx<T> s[N * W];
   int bx, by;
   grid_block_xy(bx, by);
   const int kx0 = bx * W;
   const int ky = by;
+  const int d = blockIdx.z;
+  dst += d * ds;
   const int64_t stride = (int64_t)N * KX;
   const int64_t base = (int64_t)ky * KX + kx0;
   // the kernel values of this thread's elements are loaded before the
@@ -557,15 +537,17 @@ __global__ __launch_bounds__(NT_FFT) void k_tx_c2r(const cpx<T>* __restrict__ sr
   }
 }
 
-// tiled y pass, in place: tile (kh, part, kz) = W columns kx = kh*16 +
+// tiled y pass, in place, of the spectrum d0, d1 or d2 that blockIdx.z
+// picks: tile (kh, part, kz) = W columns kx = kh*16 +
 // part*W + w along ky (stride 16)
 template <typename T, int LOGN, bool INV>
-__global__ __launch_bounds__(pick_nty<T>(LOGN)) void k_ty(cpx<T>* data, const cpx<T>* __restrict__ tw) {
+__global__ __launch_bounds__(pick_nty<T>(LOGN)) void k_ty(cpx<T>* d0, cpx<T>* d1, cpx<T>* d2, const cpx<T>* __restrict__ tw) {
   constexpr int N = 1 << LOGN, W = pick_wy<T>(LOGN), NP = TB / W, NTH = pick_nty<T>(LOGN);
   __shared__ cpx<T> s[N * W];
   int bx, by;
   grid_block_xy(bx, by);
   const int kh = bx / NP, part = bx % NP, kz = by;
+  cpx<T>* const data = blockIdx.z == 0 ? d0 : (blockIdx.z == 1 ? d1 : d2);
   const int64_t base = (((int64_t)kh * N + kz) * t_pitch(N)) * TB + part * W;
   col_load<T, N, W, NTH>(s, data + base, TB, W);
   lds_fft<T, N, W, INV, W, NTH>(s, tw, 1);
@@ -716,7 +698,7 @@ static int fwd_xy_t(cube_handle* h, Mesh& m) {
     prof_end(h, p1);
     constexpr int WS = pick_w<T>(L);
     int p2 = prof_begin(h, fine ? PS_FFT_YF : PS_FFT_C);
-    k_fft_strided<T, L, 1, false><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(c, tw);
+    k_fft_strided<T, L, 1, false><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(c, 0, tw);
     prof_end(h, p2);
   });
   HIP_TRY(h, hipGetLastError());
@@ -736,7 +718,7 @@ static int fft3_r2c_t(cube_handle* h, Mesh& m) {
   const cpx<T>* tw = (const cpx<T>*)m.tw;
   LOGN_SWITCH(logn, {
     constexpr int WS = pick_w<T>(L);
-    k_fft_strided<T, L, 2, false><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(c, tw);
+    k_fft_strided<T, L, 2, false><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(c, 0, tw);
   });
   HIP_TRY(h, hipGetLastError());
   return 0;
@@ -745,54 +727,31 @@ int mesh_fft3_r2c(cube_handle* h, Mesh& m) {
   return m.prec == 4 ? fft3_r2c_t<float>(h, m) : fft3_r2c_t<double>(h, m);
 }
 
+// All three components in one launch a pass: on small meshes each launch is
+// 4.5 us whatever it does, and three times the workgroups run at once.
 template <typename T>
-static int zconv_t(cube_handle* h, Mesh& m, int d, void* dst) {
-  int logn = ilog2(m.N);
-  int64_t N = m.N;
-  int p1 = prof_begin(h, &m == &h->fine ? PS_FFT_ZCONV : PS_FFT_C);
-  LOGN_SWITCH(logn, {
-    constexpr int WS = pick_w<T>(L);
-    k_fft_zconv<T, L><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(
-        (const cpx<T>*)m.R, (cpx<T>*)dst, (const T*)m.K, d, (const cpx<T>*)m.tw);
-  });
-  prof_end(h, p1);
-  HIP_TRY(h, hipGetLastError());
-  return 0;
-}
-int mesh_zconv(cube_handle* h, Mesh& m, int d, void* dst) {
-  if (dst != m.R && dst != m.W) return cube_fail(h, CUBE_ERR_ARG, "z convolution target must be R or W");
-  return m.prec == 4 ? zconv_t<float>(h, m, d, dst) : zconv_t<double>(h, m, d, dst);
-}
-
-template <typename T>
-static int inv_yx_t(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch, const void* F0, int64_t p0,
-                    const void* F1, int64_t p1, uint32_t* f2max) {
-  int logn = ilog2(m.N);
-  int64_t N = m.N, nrows = N * N;
-  cpx<T>* c = (cpx<T>*)buf;
+static int conv3_t(cube_handle* h, Mesh& m, void* spec, void* out, uint32_t* f2max) {
+  const int logn = ilog2(m.N);
+  const int64_t N = m.N, nrows = N * N, n3 = N * N * N, ss = N * N * (N / 2 + 1);
+  cpx<T>* c = (cpx<T>*)spec;
   const cpx<T>* tw = (const cpx<T>*)m.tw;
-  const bool fine = &m == &h->fine;
+  const int pr = prof_begin(h, PS_FFT_C);
   LOGN_SWITCH(logn, {
     constexpr int WS = pick_w<T>(L);
-    int pa = prof_begin(h, fine ? PS_FFT_YI : PS_FFT_C);
-    k_fft_strided<T, L, 1, true><<<dim3((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N), NT_FFT, 0, h->stream>>>(c, tw);
-    prof_end(h, pa);
+    const dim3 g((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N, 3);
+    k_fft_zconv<T, L><<<g, NT_FFT, 0, h->stream>>>((const cpx<T>*)m.R, c, ss, (const T*)m.K, tw);
+    k_fft_strided<T, L, 1, true><<<g, NT_FFT, 0, h->stream>>>(c, ss, tw);
     constexpr int WX = pick_w<T>(L - 1);
-    int pb = prof_begin(h, fine ? PS_FFT_XI : PS_FFT_C);
-    k_fft_x_c2r<T, L><<<dim3((unsigned)((nrows + WX - 1) / WX)), NT_FFT, 0, h->stream>>>(
-        c, (T*)out, opitch, tw, nrows, (const T*)F0, p0, (const T*)F1, p1, f2max);
-    prof_end(h, pb);
+    k_fft_x_c2r<T, L><<<dim3((unsigned)((nrows + WX - 1) / WX), 1, 3), NT_FFT, 0, h->stream>>>(c, ss, (T*)out, n3, N, tw, nrows);
   });
+  k_f2_max<T><<<(unsigned)std::min<int64_t>((n3 + 1023) / 1024, 2048), 256, 0, h->stream>>>((const T*)out, n3, f2max);
+  prof_end(h, pr);
   HIP_TRY(h, hipGetLastError());
   return 0;
 }
-int mesh_inv_yx(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch, const void* F0, int64_t p0,
-                const void* F1, int64_t p1, uint32_t* f2max) {
-  if (buf != m.R && buf != m.W) return cube_fail(h, CUBE_ERR_ARG, "inverse transform source must be R or W");
-  if (out == buf && opitch != m.N + 2) return cube_fail(h, CUBE_ERR_ARG, "in-place C2R needs pitch N+2");
-  if (f2max && (!F0 || !F1)) return cube_fail(h, CUBE_ERR_ARG, "force maximum needs both other components");
-  return m.prec == 4 ? inv_yx_t<float>(h, m, buf, out, opitch, F0, p0, F1, p1, f2max)
-                     : inv_yx_t<double>(h, m, buf, out, opitch, F0, p0, F1, p1, f2max);
+int mesh_conv3(cube_handle* h, Mesh& m, void* spec, void* out, uint32_t* f2max) {
+  if (spec == m.R || spec == out) return cube_fail(h, CUBE_ERR_ARG, "convolution spectra must lie apart");
+  return m.prec == 4 ? conv3_t<float>(h, m, spec, out, f2max) : conv3_t<double>(h, m, spec, out, f2max);
 }
 
 // ---------------------------------------- tiled fine-mesh convolution host
@@ -808,7 +767,8 @@ static int t_fwd_t(cube_handle* h, Mesh& m, const void* src, void* dst) {
     prof_end(h, p1);
     constexpr int WY = pick_wy<T>(L);
     int p2 = prof_begin(h, PS_FFT_YF);
-    k_ty<T, L, false><<<dim3((unsigned)(t_tiles(N) * (TB / WY)), (unsigned)N), pick_nty<T>(L), 0, h->stream>>>((cpx<T>*)dst, tw);
+    k_ty<T, L, false><<<dim3((unsigned)(t_tiles(N) * (TB / WY)), (unsigned)N), pick_nty<T>(L), 0, h->stream>>>((cpx<T>*)dst, nullptr,
+                                                                                                                    nullptr, tw);
     prof_end(h, p2);
   });
   HIP_TRY(h, hipGetLastError());
@@ -873,15 +833,32 @@ int mesh_t_zconv3(cube_handle* h, Mesh& m, const void* src, void* const dst[3]) 
 }
 
 template <typename T>
-static int t_inv_t(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch) {
-  int logn = ilog2(m.N);
-  int64_t N = m.N, nrows = N * N;
+static int t_inv_y_t(cube_handle* h, Mesh& m, void* const* buf, int n) {
+  const int logn = ilog2(m.N);
+  const int64_t N = m.N;
   const cpx<T>* tw = (const cpx<T>*)m.tw;
+  cpx<T>* b[3];
+  for (int d = 0; d < 3; d++) b[d] = (cpx<T>*)(d < n ? buf[d] : nullptr);
   LOGN_SWITCH(logn, {
     constexpr int WY = pick_wy<T>(L);
     int pa = prof_begin(h, PS_FFT_YI);
-    k_ty<T, L, true><<<dim3((unsigned)(t_tiles(N) * (TB / WY)), (unsigned)N), pick_nty<T>(L), 0, h->stream>>>((cpx<T>*)buf, tw);
+    k_ty<T, L, true><<<dim3((unsigned)(t_tiles(N) * (TB / WY)), (unsigned)N, (unsigned)n), pick_nty<T>(L), 0, h->stream>>>(
+        b[0], b[1], b[2], tw);
     prof_end(h, pa);
+  });
+  HIP_TRY(h, hipGetLastError());
+  return 0;
+}
+int mesh_t_inv_y(cube_handle* h, Mesh& m, void* const* buf, int n) {
+  if (n < 1 || n > 3) return cube_fail(h, CUBE_ERR_ARG, "one to three spectra");
+  return m.prec == 4 ? t_inv_y_t<float>(h, m, buf, n) : t_inv_y_t<double>(h, m, buf, n);
+}
+template <typename T>
+static int t_inv_x_t(cube_handle* h, Mesh& m, const void* buf, void* out, int64_t opitch) {
+  const int logn = ilog2(m.N);
+  const int64_t N = m.N, nrows = N * N;
+  const cpx<T>* tw = (const cpx<T>*)m.tw;
+  LOGN_SWITCH(logn, {
     constexpr int WX = pick_wtx<T>(L);
     int pb = prof_begin(h, PS_FFT_XI);
     k_tx_c2r<T, L><<<dim3((unsigned)((nrows + WX - 1) / WX)), NT_FFT, 0, h->stream>>>((const cpx<T>*)buf, (T*)out, opitch, tw,
@@ -891,18 +868,18 @@ static int t_inv_t(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch
   HIP_TRY(h, hipGetLastError());
   return 0;
 }
-int mesh_t_inv(cube_handle* h, Mesh& m, void* buf, void* out, int64_t opitch) {
+int mesh_t_inv_x(cube_handle* h, Mesh& m, const void* buf, void* out, int64_t opitch) {
   if (out == buf) return cube_fail(h, CUBE_ERR_ARG, "tiled C2R runs out of place");
-  return m.prec == 4 ? t_inv_t<float>(h, m, buf, out, opitch) : t_inv_t<double>(h, m, buf, out, opitch);
+  return m.prec == 4 ? t_inv_x_t<float>(h, m, buf, out, opitch) : t_inv_x_t<double>(h, m, buf, out, opitch);
 }
 
 // -------------------------------------------------------------- allocation
-int mesh_alloc(cube_handle* h, Mesh& m, int64_t N, int prec, bool with_S, bool with_K) {
+int mesh_alloc(cube_handle* h, Mesh& m, int64_t N, int prec, bool with_S, bool with_K, bool with_W) {
   m.N = N;
   m.prec = prec;
   int64_t H = N / 2 + 1;
   HIP_TRY(h, hipMalloc(&m.R, m.bytes_big()));
-  HIP_TRY(h, hipMalloc(&m.W, m.bytes_big()));
+  if (with_W) HIP_TRY(h, hipMalloc(&m.W, m.bytes_big()));
   if (with_S) {
     HIP_TRY(h, hipMalloc(&m.S, (size_t)prec * N * N * N));
     HIP_TRY(h, hipMalloc(&m.X, m.bytes_big()));
@@ -1083,7 +1060,7 @@ __global__ void k_ck_correct(const double* kc, const double* ku, int64_t N, int 
 int coarse_kernel_build(cube_handle* h, const float* table) {
   Mesh tmp;
   int64_t N = h->coarse.N, H = N / 2 + 1, H3 = H * H * H;
-  int r = mesh_alloc(h, tmp, N, 8, false, false);
+  int r = mesh_alloc(h, tmp, N, 8, false, false, false);
   if (r) return r;
   float* dtab;
   double *kc, *ku;
@@ -1122,10 +1099,10 @@ static int pass_t(cube_handle* h, Mesh& m, void* buf, int axis, bool inv) {
   LOGN_SWITCH(logn, {
     constexpr int WS = pick_w<T>(L);
     dim3 g((unsigned)((N / 2 + 1 + WS - 1) / WS), (unsigned)N);
-    if (axis == 1 && !inv) k_fft_strided<T, L, 1, false><<<g, NT_FFT, 0, h->stream>>>(c, tw);
-    if (axis == 1 && inv) k_fft_strided<T, L, 1, true><<<g, NT_FFT, 0, h->stream>>>(c, tw);
-    if (axis == 2 && !inv) k_fft_strided<T, L, 2, false><<<g, NT_FFT, 0, h->stream>>>(c, tw);
-    if (axis == 2 && inv) k_fft_strided<T, L, 2, true><<<g, NT_FFT, 0, h->stream>>>(c, tw);
+    if (axis == 1 && !inv) k_fft_strided<T, L, 1, false><<<g, NT_FFT, 0, h->stream>>>(c, 0, tw);
+    if (axis == 1 && inv) k_fft_strided<T, L, 1, true><<<g, NT_FFT, 0, h->stream>>>(c, 0, tw);
+    if (axis == 2 && !inv) k_fft_strided<T, L, 2, false><<<g, NT_FFT, 0, h->stream>>>(c, 0, tw);
+    if (axis == 2 && inv) k_fft_strided<T, L, 2, true><<<g, NT_FFT, 0, h->stream>>>(c, 0, tw);
   });
   HIP_TRY(h, hipGetLastError());
   return 0;
@@ -1141,7 +1118,7 @@ static int c2r_t(cube_handle* h, Mesh& m, const void* src, void* dst, int64_t op
   LOGN_SWITCH(logn, {
     constexpr int WX = pick_w<T>(L - 1);
     k_fft_x_c2r<T, L><<<dim3((unsigned)((nrows + WX - 1) / WX)), NT_FFT, 0, h->stream>>>(
-        (const cpx<T>*)src, (T*)dst, opitch, (const cpx<T>*)m.tw, nrows, nullptr, 0, nullptr, 0, nullptr);
+        (const cpx<T>*)src, 0, (T*)dst, 0, opitch, (const cpx<T>*)m.tw, nrows);
   });
   HIP_TRY(h, hipGetLastError());
   return 0;

@@ -758,17 +758,15 @@ static int kick_pick(cube_handle* h, const void* const Ff[3], const int64_t pf[3
 int kick_all(cube_handle* h, const void* const Ff[3], const int64_t pf[3], float a_mid, float dt, double c_old,
              uint32_t* vmax_bits, uint32_t* f2max_bits, double* probe_f, double* probe_c) {
   const double* vo = vtab_for(h, c_old);
-  const double* c_new = h->dscal;  // and its table h->vdt_new, both written by the drift
-  const double* vn = h->vdt_new;
+  const double* c_new = h->dscal;  // and its table, both written by the drift
+  const double* vn = h->vdt_at(h->vdt_ni);
   if (vmax_bits != f2max_bits + 1) return cube_fail(h, CUBE_ERR_ARG, "kick: vmax must follow f2max");
   if (!probe_f != !probe_c) return cube_fail(h, CUBE_ERR_ARG, "kick: probe both force arrays or neither");
-  int r0 = fill_u32(h, h->mslots, MSLOTS * MSLOT_FIELDS, 0u);
-  if (r0) return r0;
   int r = h->prec == 4
               ? kick_pick<float>(h, Ff, pf, a_mid, dt, c_new, vo, vn, probe_f, probe_c)
               : kick_pick<double>(h, Ff, pf, a_mid, dt, c_new, vo, vn, probe_f, probe_c);
   if (r) return r;
   HIP_TRY(h, hipGetLastError());
   // max |F|^2 always; vmax only for a kick (a probe leaves it unset)
-  return slots_reduce(h, probe_f ? 1 : 4, 0u, 0u, f2max_bits);
+  return slots_reduce(h, probe_f ? 1 : 4, 0u, 0u, f2max_bits, h->drep->pmflags, 1, 5);
 }

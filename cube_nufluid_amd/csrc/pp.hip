@@ -1040,7 +1040,8 @@ static int pp_launch(cube_handle* h, const Geo& g, const PPctx& c, uint32_t* f2,
 // their bit patterns)
 __global__ __launch_bounds__(256) void k_pp_totals(const unsigned long long* __restrict__ npr,
                                                    const unsigned long long* __restrict__ nup,
-                                                   const uint32_t* __restrict__ f2, StepReport* d) {
+                                                   const uint32_t* __restrict__ f2, const uint32_t* __restrict__ flags,
+                                                   StepReport* d) {
   __shared__ unsigned long long sp[256], st[256];
   __shared__ uint32_t sf[256];
   unsigned long long a = 0, b = 0;
@@ -1062,6 +1063,7 @@ __global__ __launch_bounds__(256) void k_pp_totals(const unsigned long long* __r
     }
     __syncthreads();
   }
+  if (threadIdx.x < sizeof(d->ppflags) / 4) d->ppflags[threadIdx.x] = flags[threadIdx.x];
   if (threadIdx.x == 0) {
     d->pp_pairs = sp[0];
     d->pp_targets = st[0];
@@ -1089,8 +1091,8 @@ int pp_launch_step(cube_handle* h, float a_mid, float dt, double c_old, double* 
   unsigned long long* nup = npr + PP_SLOTS;
   uint32_t* f2 = (uint32_t*)(nup + PP_SLOTS);
   int rc;
-  if ((rc = fill_u32(h, h->uflags + 8, 12, 0u))) return rc;
-  if ((rc = fill_u32(h, h->pp_red, PP_SLOTS * (2 * sizeof(unsigned long long) + sizeof(uint32_t)) / 4, 0u))) return rc;
+  if ((rc = clear_u32(h, {h->uflags + 8, 12}, {h->pp_red, PP_SLOTS * (2 * sizeof(unsigned long long) + sizeof(uint32_t)) / 4})))
+    return rc;
   // pp_meta: per 2^3-cell block (the finer of the two block sizes) 2 int64 of
   // info and 2 int32 list entries, plus the work items
   const int64_t nb2 = (h->nc / 2) * (h->nc / 2) * (h->nc / 2);
@@ -1120,9 +1122,8 @@ int pp_launch_step(cube_handle* h, float a_mid, float dt, double c_old, double* 
                                      h->vkmax, f2, npr, nup, probe, fall, nfall, bscale);
   HIP_TRY(h, hipGetLastError());
   prof_end(h, pr);
-  k_pp_totals<<<1, 256, 0, h->stream>>>(npr, nup, f2, h->drep);
+  k_pp_totals<<<1, 256, 0, h->stream>>>(npr, nup, f2, h->uflags + 8, h->drep);
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(h->drep->ppflags, h->uflags + 8, sizeof(h->drep->ppflags), hipMemcpyDeviceToDevice, h->stream));
   return 0;
 }
 

@@ -161,6 +161,9 @@ static int step_deferred(cube_handle* h, cube_clock* c) {
       std::swap(h->vfield, h->vfield2);
       std::swap(h->cstart, h->cstart2);
     }
+    // what the step's launches were to leave in the tables may not be there
+    for (double& c : h->vdt_c) c = NAN;
+    (void)sigma_new_to_device(h);
     return r;
   }
   if ((r = drift_finish(h, h->rep, nlayer, nullptr))) return r;
@@ -207,7 +210,7 @@ extern "C" int64_t cube_footprint(const cube_params* p, int32_t ic_np_nc) {
   auto mesh = [&](int64_t N, bool with_S) {
     const int64_t H = N / 2 + 1;
     const int64_t big = std::max(N * N * (N + 2) * prec, (H + 15) / 16 * 16 * N * t_pitch(N) * 2 * prec);  // Mesh::bytes_big
-    return 2 * big + (with_S ? N * N * N * prec + big : 0) + 3 * H * ((H + 15) / 16 * 16) * H * prec + 2 * N * prec;
+    return big + (with_S ? N * N * N * prec + 2 * big : 0) + 3 * H * ((H + 15) / 16 * 16) * H * prec + 2 * N * prec;
   };
   const int64_t nb2 = (nc / 2) * (nc / 2) * (nc / 2);
   int64_t b = 0;
