@@ -427,8 +427,8 @@ __global__ __launch_bounds__(DR_SORT_NT) void k_drift_sort_big(const int64_t* __
 //   gather (one thread per slot, DG_SL slots per batch with each stage's
 //     loads issued together): the arrival's full velocity vreal
 //     (update_particle.f90:69), its new position code (:117) and PID.
-//   cells (one thread per cell): vfield_new summed in arrival order
-//     (update_particle.f90:70-83).
+//   cells (one thread per component of a cell): vfield_new summed in arrival
+//     order (update_particle.f90:70-83).
 //   slots (DC_SL per batch): the velocity residual re-quantised with the old
 //     sigma (:119) and the sigma_v sums (:174-200).
 // A cell of more than DW_STAGE slots keeps its velocities in HBM, and its sum
@@ -439,6 +439,28 @@ __global__ __launch_bounds__(DR_SORT_NT) void k_drift_sort_big(const int64_t* __
 #define DW_STAGE 1536
 #define DG_SL 4
 #define DC_SL 2
+// vf + get(0) + ... + get(n-1), rounded to float after every addition as the
+// reference does, so a chain of three dependent operations a value; the next
+// CH_U values are requested while a block is added.
+#define CH_U 8
+template <typename Get>
+__device__ __forceinline__ float chain_add(float vf, int n, const Get& get) {
+  if (n <= 0) return vf;
+  double a[CH_U], b[CH_U];
+#pragma unroll
+  for (int u = 0; u < CH_U; u++) a[u] = get(min(u, n - 1));
+  for (int k = 0; k < n; k += CH_U) {
+#pragma unroll
+    for (int u = 0; u < CH_U; u++) b[u] = get(min(k + CH_U + u, n - 1));
+#pragma unroll
+    for (int u = 0; u < CH_U; u++) {
+      const float x = (float)((double)vf + a[u]);
+      vf = k + u < n ? x : vf;
+      a[u] = b[u];
+    }
+  }
+  return vf;
+}
 template <bool STAGED>
 __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restrict__ keys, int64_t r0, int ncell,
                                                  const int64_t* __restrict__ cstart, const void* __restrict__ xp,
@@ -521,8 +543,7 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
       const int m = (int)min((int64_t)DW_STAGE, q1 - b);
       for (int i = threadIdx.x; i < 3 * m; i += DR_NT) svr[i] = vr[3 * b + i];
       __syncthreads();
-      if (threadIdx.x < 3)
-        for (int k = 0; k < m; k++) vf = (float)((double)vf + svr[3 * k + threadIdx.x]);
+      if (threadIdx.x < 3) vf = chain_add(vf, m, [&](int k) { return svr[3 * k + threadIdx.x]; });
       __syncthreads();
     }
     if (threadIdx.x < 3) svf[threadIdx.x] = vf;
@@ -530,26 +551,20 @@ __device__ __forceinline__ void drift_write_body(Geo g, const uint64_t* __restri
     const float sum3[3] = {svf[0], svf[1], svf[2]};
     __syncthreads();
     if (threadIdx.x == 0) finish(r0, 0, sum3, q1 - qa);
-  } else if ((int)threadIdx.x < ncell) {
-    const int64_t r = r0 + threadIdx.x;
-    const int64_t b = scs[threadIdx.x], n = scs[threadIdx.x + 1] - b;
-    float vf[3];
-    for (int e = 0; e < 3; e++) vf[e] = (float)((double)vfield[r * 3 + e] * wv);
-    // in arrival order; the loads of U arrivals are issued together
-    constexpr int U = 4;
-    for (int64_t k0 = 0; k0 < n; k0 += U) {
-      double a[U][3];
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int e = 0; e < 3; e++) a[u][e] = k0 + u < n ? vr_at(b + k0 + u, e) : 0.0;
-#pragma unroll
-      for (int u = 0; u < U; u++)
-        if (k0 + u < n)
-#pragma unroll
-          for (int e = 0; e < 3; e++) vf[e] = (float)((double)vf[e] + a[u][e]);
+  } else {
+    // a thread per component of a cell, in arrival order
+    for (int i = threadIdx.x; i < 3 * ncell; i += DR_NT) {
+      const int c = i / 3, e = i % 3;
+      const int64_t b = scs[c];
+      svf[i] = chain_add((float)((double)vfield[3 * r0 + i] * wv), (int)(scs[c + 1] - b),
+                         [&](int k) { return vr_at(b + k, e); });
     }
-    finish(r, threadIdx.x, vf, n);
+    __syncthreads();
+    if ((int)threadIdx.x < ncell) {
+      const int c = threadIdx.x;
+      const float sum3[3] = {svf[c * 3], svf[c * 3 + 1], svf[c * 3 + 2]};
+      finish(r0 + c, c, sum3, scs[c + 1] - scs[c]);
+    }
   }
   __syncthreads();
   // ---- slots: re-quantisation and sigma sums, DC_SL per batch
