@@ -257,6 +257,23 @@ __device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
   return v;
 }
 
+// Lanes of a wave hold consecutive particles, so equal destination cells in
+// neighbouring lanes form runs; one atomic per run instead of per particle.
+// key < 0 marks an idle lane (made unique per lane by the caller).
+struct WaveRun { int head, len; };
+__device__ __forceinline__ WaveRun wave_run(int64_t key) {
+  const int lane = threadIdx.x & 63;
+  const int64_t prev = __shfl_up(key, 1);
+  const bool is_head = lane == 0 || key != prev;
+  const unsigned long long H = __ballot(is_head);
+  const unsigned long long upto = ~0ull >> (63 - lane);  // bits 0..lane
+  const unsigned long long above = H & ~upto;
+  WaveRun w;
+  w.head = 63 - __clzll(H & upto);
+  w.len = (above ? __ffsll((long long)above) - 1 : 64) - lane;  // meaningful in the head lane
+  return w;
+}
+
 // Cell indices stay below 2^27 (nc <= 512), so index arithmetic is 32-bit;
 // nc is a power of two and so, in the usual layouts, are nt and nnt.
 __host__ __device__ __forceinline__ int32_t wrapc(int32_t a, int32_t n) { return a & (n - 1); }

@@ -35,23 +35,6 @@ __device__ __forceinline__ uint16_t pack_disp(int dx, int dy, int dz) {
   return (uint16_t)((dx + 8) | ((dy + 8) << 4) | ((dz + 8) << 8));
 }
 
-// Lanes of a wave hold consecutive particles, so equal destination cells in
-// neighbouring lanes form runs; one atomic per run instead of per particle.
-// key < 0 marks an idle lane (made unique per lane by the caller).
-struct WaveRun { int head, len; };
-__device__ __forceinline__ WaveRun wave_run(int64_t key) {
-  const int lane = threadIdx.x & 63;
-  const int64_t prev = __shfl_up(key, 1);
-  const bool is_head = lane == 0 || key != prev;
-  const unsigned long long H = __ballot(is_head);
-  const unsigned long long upto = ~0ull >> (63 - lane);  // bits 0..lane
-  const unsigned long long above = H & ~upto;
-  WaveRun w;
-  w.head = 63 - __clzll(H & upto);
-  w.len = (above ? __ffsll((long long)above) - 1 : 64) - lane;  // meaningful in the head lane
-  return w;
-}
-
 #define DP_SL 2
 // Both per-particle passes take DR_CH source cells a workgroup: 256, or fewer
 // where that leaves CUs idle (drift_cells: at 16^3 cells 16 workgroups of 256
