@@ -59,7 +59,7 @@ def algorithmic_bytes(slot, cfg, npart):
         # one launch for all three components on FP32 meshes: the spectrum
         # read once, three convolved spectra written, three kernel octants
         "fft_zconv": 17.5 * mf,
-        "fft_y_inv": 8 * mf,
+        "fft_y_inv": 24 * mf,  # the three components in one launch
         "fft_x_c2r": 8 * mf,
         # fine pass: xp, vp read + write, three fine force meshes, cell
         # offsets; coarse pass: the same particle arrays, three coarse
