@@ -30,7 +30,8 @@ __host__ __device__ inline cpx<T> cmul(cpx<T> a, cpx<T> b) {
 // Three-component z convolution with N, N+1, N+2, N+4, N+8 lines a plane:
 // 0.935, 0.824, 0.807, 0.946, 0.812 ms at 512^3, 8.78, 7.46, 7.13, 7.43,
 // 8.28 ms at 1024^3, 80.1, 69.7, 70.5, 72.1, 69.6 ms at 2048^3; the y and x
-// passes move by less than 8 % either way.
+// passes move by less than 8 % either way.  At 2048^3 the z pass's HBM traffic
+// falls from 210 to 166 GB, against 150 it cannot do without.
 __host__ __device__ constexpr int64_t t_pitch(int64_t N) { return N + 2; }
 
 // ---------------------------------------------------------------- mesh
