@@ -48,14 +48,20 @@ __device__ __forceinline__ float press(float r, float m1, float m2, float m3, fl
 // Several quotients by one denominator b: with y the correctly rounded 1/b,
 // the estimate x*y corrected by its exact remainder is the correctly rounded
 // x/b (Markstein 1990), in three operations instead of some eleven.  That
-// needs a remainder above the smallest denormal: |x| > 1e-30 and a finite
-// result, which the caller checks with div_safe for all numerators at once;
-// otherwise the plain division gives the same quotient.
+// needs a remainder above the smallest denormal and a quotient that is neither
+// denormal nor beyond the largest float (an infinite estimate leaves a NaN, and
+// a denormal one may be a unit off).  The caller checks with div_safe that all
+// numerators lie between 1e-30 and 1e30 in magnitude and b between 1e-7 and
+// 1e7; otherwise it divides.
 __device__ __forceinline__ float div_by(float x, float b, float y) {
   const float q = x * y;
   return fmaf(fmaf(-q, b, x), y, q);
 }
-__device__ __forceinline__ bool div_safe(float least, float b) { return least > 1e-30f && b > 1e-15f && b < 1e15f; }
+__device__ __forceinline__ bool div_safe(float least, float most, float b) {
+  return least > 1e-30f && most < 1e30f && b > 1e-7f && b < 1e7f;
+}
+__device__ __forceinline__ float min3abs(float a, float b, float c) { return fminf(fminf(fabsf(a), fabsf(b)), fabsf(c)); }
+__device__ __forceinline__ float max3abs(float a, float b, float c) { return fmaxf(fmaxf(fabsf(a), fabsf(b)), fabsf(c)); }
 
 // primitives v = m/rho, p of one cell
 template <bool FAST>
@@ -82,7 +88,7 @@ __device__ __forceinline__ void fl_side(const float b[5], float y, float g, floa
   f[2] = h[1] * div(h[2]);
   f[3] = h[1] * div(h[3]);
   f[4] = h[4] * v;
-  s = sqrtf(FAST ? (p > 1e-30f ? div_by(p, b[0], y) : p / b[0]) : p / b[0]);
+  s = sqrtf(FAST && p > 1e-30f && p < 1e30f ? div_by(p, b[0], y) : p / b[0]);
 }
 
 // One sweep along axis AX over W adjacent lines of nc = 2^lnc cells, W nc <=
@@ -128,9 +134,9 @@ __global__ __launch_bounds__(FL_SNT) void k_fl_sweep(float* F, int nc, int lnc, 
     const float r = F[c], m1 = F[(int64_t)c1 * n3 + c], m2 = F[(int64_t)c2 * n3 + c], m3 = F[(int64_t)c3 * n3 + c],
                 en = F[4 * n3 + c];
     float u[5];
-    // the squared momenta must stay in range too
-    const float least = fminf(fminf(fabsf(m1), fabsf(m2)), fabsf(m3));
-    if (div_safe(least * least, r)) fl_prim<true>(r, 1.0f / r, m1, m2, m3, en, g, u);
+    // the momenta and half the sum of their squares are divided
+    const float least = min3abs(m1, m2, m3), most = max3abs(m1, m2, m3);
+    if (div_safe(least * least, 2.0f * (most * most), r)) fl_prim<true>(r, 1.0f / r, m1, m2, m3, en, g, u);
     else fl_prim<false>(r, 0.0f, m1, m2, m3, en, g, u);
 #pragma unroll
     for (int q = 0; q < 5; q++) S(q, w, t) = u[q];
@@ -154,9 +160,11 @@ __global__ __launch_bounds__(FL_SNT) void k_fl_sweep(float* F, int nc, int lnc, 
       br[q] = u2 - 0.5f * minmod(l, 0.5f * (u3 - u1), H_LIM * (u3 - u2));
     }
     float hl[5], hr[5], fl[5], fr[5], vl, vr, sl, sr;
-    const float ml = fminf(fminf(fabsf(bl[1]), fabsf(bl[2])), fabsf(bl[3])), mr = fminf(fminf(fabsf(br[1]), fabsf(br[2])), fabsf(br[3]));
-    const float mh = fminf(ml * bl[0], mr * br[0]);
-    const bool fast = div_safe(fminf(fminf(bl[4], br[4]), mh * mh), bl[0]) && div_safe(1.0f, br[0]);
+    // momenta, half the sum of their squares, and pressures (by gamma - 1)
+    const float mh = fminf(min3abs(bl[1], bl[2], bl[3]) * bl[0], min3abs(br[1], br[2], br[3]) * br[0]);
+    const float xh = fmaxf(max3abs(bl[1], bl[2], bl[3]) * bl[0], max3abs(br[1], br[2], br[3]) * br[0]);
+    const bool fast = div_safe(fminf(fminf(bl[4], br[4]), mh * mh), fmaxf(fmaxf(bl[4], br[4]), 2.0f * (xh * xh)), bl[0]) &&
+                      div_safe(1.0f, 1.0f, br[0]) && g < 1e7f;
     if (fast) {
       fl_side<true>(bl, 1.0f / bl[0], g, yg, hl, fl, vl, sl);
       fl_side<true>(br, 1.0f / br[0], g, yg, hr, fr, vr, sr);
@@ -167,13 +175,14 @@ __global__ __launch_bounds__(FL_SNT) void k_fl_sweep(float* F, int nc, int lnc, 
     const float ap = fmaxf(fmaxf(0.0f, vl + sl), vr + sr);
     const float am = fmaxf(fmaxf(0.0f, -vl + sl), -vr + sr);
     const float as = ap + am;
-    float nu[5], least = 1.0f;
+    float nu[5], least = 1.0f, most = 1.0f;
 #pragma unroll
     for (int q = 0; q < 5; q++) {
       nu[q] = ap * fl[q] + am * fr[q] - ap * am * (hr[q] - hl[q]);
       least = fminf(least, fabsf(nu[q]));
+      most = fmaxf(most, fabsf(nu[q]));
     }
-    if (div_safe(least, as)) {
+    if (div_safe(least, most, as)) {
       const float ya = 1.0f / as;
 #pragma unroll
       for (int q = 0; q < 5; q++) fx[k][q] = div_by(nu[q], as, ya);
