@@ -27,6 +27,9 @@
 //      (inertia, dx_mean, inert) carried by single-thread scans.
 // A particle's tag is a 27-bit mask, one bit per tile holding a copy of it
 // (the tile's displacement -1..1 per axis from the particle's own tile).
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "k_halo_process orders its peaks by what gfx950 guarantees for agent-scope atomics and vmcnt"
+#endif
 #include <hipcub/hipcub.hpp>
 
 #include "cube_internal.hpp"
@@ -297,13 +300,31 @@ __device__ __forceinline__ V block_reduce(V v, V* buf, Op op) {
 
 // ------------------------------------------------------- peak processing
 // Until every memory operation this wavefront issued has been performed.
-// Peaks hand on nothing but particle tags, which are written and read by
-// device-scope atomics: once the atomics of a peak have been performed, its
-// `done` flag may be set, and who sees the flag sees the tags.  A device-scope
-// release or acquire fence would besides write back and invalidate the XCD's
-// L2; four of them per peak bounded the kernel (5.2 ms for 11485 peaks,
-// whatever else it did).
+// Peaks on different workgroups hand on two words, a particle's tag and a
+// peak's done flag, and these only through the three functions below; whatever
+// else a peak stores is read by itself or by later kernels.  The language
+// orders relaxed atomics by nothing, so the order rests on what LLVM's memory
+// model states for gfx942 and gfx950: agent-scope atomics are coherent between
+// the XCDs' L2s, loads among them do not read the L1, and vmcnt counts stores
+// and atomics without a result too, so that after s_waitcnt vmcnt(0) they have
+// been performed.  A peak's tags are therefore in place before the barrier
+// after which its flag is set; a peak that waits has the flag's value before
+// its own barrier, and issues its tag loads after it.  A plain load or store of
+// tag or done, or of any other word that a peak reads from another, would not
+// be ordered.  An agent-scope release or acquire fence would add the write-back
+// and invalidation of the XCD's L2 that plain data need; four of them per peak
+// bounded the kernel (5.2 ms for 11485 peaks, whatever else it did).
 __device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+template <typename V>
+__device__ __forceinline__ V peak_word(const V* w) {
+  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void peak_mark(uint32_t* tag, uint32_t bit) {
+  (void)__hip_atomic_fetch_or(tag, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void peak_finish(int32_t* done) {
+  __hip_atomic_store(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 struct HWs {  // one workgroup's scratch in global memory
   int32_t* q;       // gathered particle index
@@ -372,7 +393,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
           const float rr = p.rs + q.rs + 1e-3f;
           if (d0 * d0 + d1 * d1 + d2 * d2 >= rr * rr) continue;
           uint32_t spins = 0;
-          while (__hip_atomic_load(done + Q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+          while (peak_word(done + Q) == 0) {
             __builtin_amdgcn_s_sleep(2);
             if (++spins > HSPIN_LIMIT) { ok = false; break; }
           }
@@ -455,7 +476,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
 #pragma unroll
       for (int u = 0; u < HGU; u++)
         if (flag[u]) {
-          const uint32_t tg = __hip_atomic_load(tag + q[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const uint32_t tg = peak_word(tag + q[u]);
           flag[u] = (tg & bt[u]) ? 0u : 1u;
         }
 #pragma unroll
@@ -681,7 +702,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
       for (int d = 0; d < 3; d++) out.hfin[d] = hf[d];
       out.phys = phys;
       if (out.i_odc >= c.min_np) {
-        for (int64_t m = tid; m < out.i_odc; m += HNT) atomicOr(tag + ws.q[ws.idx[cur][m]], ws.bit[ws.idx[cur][m]]);
+        for (int64_t m = tid; m < out.i_odc; m += HNT) peak_mark(tag + ws.q[ws.idx[cur][m]], ws.bit[ws.idx[cur][m]]);
         if (phys) {
           if (tid == 0) {
             const unsigned long long o = atomicAdd(mcount, (unsigned long long)out.i_odc);
@@ -703,7 +724,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
     if (tid == 0) res[P] = out;
     wait_memory();
     __syncthreads();
-    if (tid == 0) __hip_atomic_store(done + P, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) peak_finish(done + P);
   }
 }
 
