@@ -41,7 +41,7 @@ struct Mesh {
   int64_t N = 0;
   int prec = 4;          // sizeof(real)
   void* R = nullptr;     // real N*N*(N+2) padded rows; complex view N*N*(N/2+1)
-  void* W = nullptr;     // (fine, initial conditions) complex work, bytes_big()
+  void* W = nullptr;     // (fine, initial conditions) complex work, the size of R
   void* S = nullptr;     // unpadded N^3 real mesh (fine: force component 0)
   void* X = nullptr;     // (fine) second spectrum / real work mesh, bytes_big()
   void* K = nullptr;     // kernel [3][H][H][H], layout [d][ky'][kx][kz'], scaled 1/N^3
@@ -52,6 +52,17 @@ struct Mesh {
   size_t bytes_big() const {
     const size_t t = (size_t)((N / 2 + 1 + 15) / 16) * 16 * N * t_pitch(N) * 2 * prec;
     return t > bytes_R() ? t : bytes_R();
+  }
+  size_t bytes_S() const { return (size_t)N * N * N * prec; }
+  // kx padded to whole 16-wide tiles: the fine mesh's strip layout needs it
+  size_t bytes_K() const { return (size_t)3 * (N / 2 + 1) * ((N / 2 + 1 + 15) / 16 * 16) * (N / 2 + 1) * prec; }
+  size_t bytes_tw() const { return (size_t)N * 2 * prec; }
+  // R, W and X each: only the fine mesh (with S) holds tiled spectra
+  size_t bytes_work(bool with_S) const { return with_S ? bytes_big() : bytes_R(); }
+  // all that mesh_alloc takes
+  size_t bytes_all(bool with_S, bool with_K, bool with_W = true) const {
+    return (1 + (with_W ? 1 : 0) + (with_S ? 1 : 0)) * bytes_work(with_S) + (with_S ? bytes_S() : 0) + (with_K ? bytes_K() : 0) +
+           bytes_tw();
   }
 };
 

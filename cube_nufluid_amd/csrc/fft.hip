@@ -877,16 +877,14 @@ int mesh_t_inv_x(cube_handle* h, Mesh& m, const void* buf, void* out, int64_t op
 int mesh_alloc(cube_handle* h, Mesh& m, int64_t N, int prec, bool with_S, bool with_K, bool with_W) {
   m.N = N;
   m.prec = prec;
-  int64_t H = N / 2 + 1;
-  HIP_TRY(h, hipMalloc(&m.R, m.bytes_big()));
-  if (with_W) HIP_TRY(h, hipMalloc(&m.W, m.bytes_big()));
+  HIP_TRY(h, hipMalloc(&m.R, m.bytes_work(with_S)));
+  if (with_W) HIP_TRY(h, hipMalloc(&m.W, m.bytes_work(with_S)));
   if (with_S) {
-    HIP_TRY(h, hipMalloc(&m.S, (size_t)prec * N * N * N));
-    HIP_TRY(h, hipMalloc(&m.X, m.bytes_big()));
+    HIP_TRY(h, hipMalloc(&m.S, m.bytes_S()));
+    HIP_TRY(h, hipMalloc(&m.X, m.bytes_work(with_S)));
   }
-  // kx padded to whole 16-wide tiles: the fine mesh's strip layout needs it
-  if (with_K) HIP_TRY(h, hipMalloc(&m.K, (size_t)3 * H * t_tiles(N) * TB * H * prec));
-  HIP_TRY(h, hipMalloc(&m.tw, (size_t)N * 2 * prec));
+  if (with_K) HIP_TRY(h, hipMalloc(&m.K, m.bytes_K()));
+  HIP_TRY(h, hipMalloc(&m.tw, m.bytes_tw()));
   std::vector<double> tw(2 * N);
   for (int64_t j = 0; j < N; j++) {
     double a = -2.0 * M_PI * (double)j / (double)N;

@@ -207,10 +207,11 @@ extern "C" int cube_step(cube_handle* h, cube_clock* c) {
 extern "C" int64_t cube_footprint(const cube_params* p, int32_t ic_np_nc) {
   if (!p) return -1;
   const int64_t npm = p->np_max, nc = p->nc, n3c = nc * nc * nc, nf = 4 * nc, prec = p->precision;
-  auto mesh = [&](int64_t N, bool with_S) {
-    const int64_t H = N / 2 + 1;
-    const int64_t big = std::max(N * N * (N + 2) * prec, (H + 15) / 16 * 16 * N * t_pitch(N) * 2 * prec);  // Mesh::bytes_big
-    return big + (with_S ? N * N * N * prec + 2 * big : 0) + 3 * H * ((H + 15) / 16 * 16) * H * prec + 2 * N * prec;
+  auto mesh = [](int64_t N, int32_t prec) {
+    Mesh m;
+    m.N = N;
+    m.prec = prec;
+    return m;
   };
   const int64_t nb2 = (nc / 2) * (nc / 2) * (nc / 2);
   int64_t b = 0;
@@ -218,13 +219,13 @@ extern "C" int64_t cube_footprint(const cube_params* p, int32_t ic_np_nc) {
   b += 2 * npm + 8 * npm + 4 * (npm / 1025 + 2);             // drift displacement, keys, lists
   b += 8 * (2 * nb2 + npm / 256 + nb2 + 1) + 8 * nb2 + 20480;  // PP lists, totals
   b += 2 * (4 * n3c + 12 * n3c + 8 * (n3c + 1)) + 3 * n3c * prec + 8 * (std::max<int64_t>(n3c, 65536) + 16);
-  b += 4 * 65536 + 8 * 131072 + 16 * 65536;  // codec tables
-  b += mesh(nf, true) + mesh(nc, false);
+  b += 4 * 65536 + 8 * 131072 + 24 * 65536;  // codec tables
+  b += (int64_t)(mesh(nf, p->precision).bytes_all(true, true) + mesh(nc, p->precision).bytes_all(false, true, false));
   const int64_t fine_R = nf * nf * (nf + 2) * prec;
   if (fine_R < 24 * npm) b += 24 * npm;  // drift scratch outside the fine work mesh
   if (ic_np_nc > 0) {  // Zel'dovich generator's temporary mesh
     const int64_t ng = (int64_t)ic_np_nc * nc;
-    b += 2 * ng * ng * (ng + 2) * 4 + 16 * ng;
+    b += (int64_t)mesh(ng, 4).bytes_all(false, false);
   }
   return b + b / 16 + (64 << 20);  // allocation granularity and runtime slack
 }

@@ -1,0 +1,58 @@
+"""What the Zel'dovich generator allocates, and what cube_footprint counts for
+it: two plain padded spectra of its ng^3 lattice (ng^2 (ng+2) floats each) and ng
+twiddles, beside tables and partial sums of less than 8 MB."""
+import ctypes
+import threading
+
+import pytest
+
+from cube_nufluid_amd import _lib
+
+
+@pytest.mark.parametrize("nc,np_nc", [(16, 1), (32, 2), (64, 1), (128, 2), (256, 2), (512, 2)])
+def test_generator_meshes_are_counted(nc, np_nc):
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    lib.cube_footprint.restype, lib.cube_footprint.argtypes = _lib.SIGNATURES["cube_footprint"]
+    p = _lib.CubeParams()
+    ng = nc * np_nc
+    p.nc, p.nnt, p.ncb, p.izipx, p.izipv, p.np_max, p.precision = nc, 2, 6, 2, 2, ng ** 3, 4
+    meshes = 2 * ng * ng * (ng + 2) * 4 + 8 * ng
+    got = lib.cube_footprint(ctypes.byref(p), np_nc) - lib.cube_footprint(ctypes.byref(p), 0)
+    assert meshes + meshes // 16 <= got <= 1.07 * meshes + 16 * ng  # a sixteenth for the allocator's rounding
+
+
+@pytest.mark.gpu
+def test_generator_allocates_what_is_counted():
+    import torch
+    from cube_nufluid_amd.driver import Cube
+    from cube_nufluid_amd.ic import power_table, velocity_factor
+    from cube_nufluid_amd.params import BoxConfig
+    cfg = BoxConfig(nc=128, nnt=4, ncb=6, box=400.0)
+    cube = Cube.from_ic(cfg, 11, 49.0)
+    ng = cfg.nc * cfg.np_nc
+    lnk, lnp = power_table(cfg, 0.02)
+    ip = _lib.ICParams()
+    ip.seed, ip.np_nc, ip.nk, ip.a, ip.box = 11, cfg.np_nc, len(lnk), 0.02, cfg.box
+    ip.vfac, ip.lnk, ip.lnp, ip.f_cdm = velocity_factor(cfg, 0.02), _lib.ptr(lnk), _lib.ptr(lnp), cfg.f_cdm
+    stop, least = threading.Event(), []
+
+    def watch():
+        low = torch.cuda.mem_get_info()[0]
+        while not stop.is_set():
+            low = min(low, torch.cuda.mem_get_info()[0])
+        least.append(low)
+
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    t = threading.Thread(target=watch)
+    t.start()
+    try:
+        for _ in range(5):
+            _lib.check(cube.lib, cube.h, cube.lib.cube_ic_zeldovich(cube.h, ctypes.byref(ip), None))
+    finally:
+        stop.set()
+        t.join()
+        cube.close()
+    used = free - least[0]
+    print("generator's allocations, MB:", used / 1e6, "lattice spectra:", 2 * ng * ng * (ng + 2) * 4 / 1e6, flush=True)
+    assert used <= 2 * ng * ng * (ng + 2) * 4 + 8e6
