@@ -74,8 +74,9 @@ enum ProfSlot {
 struct ProfRec { int slot; hipEvent_t a, b; };
 
 // Neutrino dispersive fluid: three fluids of nf/2, nf/4, nf/8 cells per
-// dimension, fields [5][nc^3] (rho, mx, my, mz, E) and gravity accumulators
-// [4][nc^3] (J0, J1, J2, Q) in double.
+// dimension, fields [5][nc^3] (rho, mx, my, mz, E), and gravity accumulators
+// [4][nc^3] (J0, J1, J2, Q) in double where the gather does not update the
+// cells itself (fl_sep_applies).
 struct NuState {
   bool on = false;
   cube_nu_params par{};

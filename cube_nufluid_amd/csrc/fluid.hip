@@ -761,8 +761,10 @@ extern "C" int cube_nu_init(cube_handle* h, const cube_nu_params* p) {
   for (int n = 0; n < 3; n++) {
     const int64_t n3 = (int64_t)s.nc[n] * s.nc[n] * s.nc[n];
     if (!s.F[n]) HIP_TRY(h, hipMalloc(&s.F[n], sizeof(float) * 5 * n3));
-    if (!s.acc[n]) HIP_TRY(h, hipMalloc(&s.acc[n], sizeof(double) * 4 * n3));
-    HIP_TRY(h, hipMemsetAsync(s.acc[n], 0, sizeof(double) * 4 * n3, h->stream));
+    if (!fl_sep_applies(s, n)) {
+      if (!s.acc[n]) HIP_TRY(h, hipMalloc(&s.acc[n], sizeof(double) * 4 * n3));
+      HIP_TRY(h, hipMemsetAsync(s.acc[n], 0, sizeof(double) * 4 * n3, h->stream));
+    }
     // hg_setup: rho = 1, m = 0, E = cs2 rho/(g-1) (q equation of state)
     std::vector<float> init(5 * n3, 0.0f);
     for (int64_t i = 0; i < n3; i++) {
@@ -918,8 +920,8 @@ int fl_density_fine(cube_handle* h, float a_mid, double* mass_added, double* mas
   return 0;
 }
 
-// The three fine-force components (Ff[d], row pitch pf[d]) into the
-// accumulators of every active fluid.
+// The three fine-force components (Ff[d], row pitch pf[d]) into every active
+// fluid, or into its accumulators where the gather does not update it itself.
 int fl_gravity_fine(cube_handle* h, const void* const Ff[3], const int64_t pf[3], float a_mid, float dt) {
   NuState& s = h->nu;
   for (int n = 0; n < 3; n++) {
@@ -962,9 +964,9 @@ static int fl_apply(cube_handle* h, float a_mid) {
   return 0;
 }
 
-// After the fine kicks: apply the fine impulses, then gather and apply the
-// coarse ones (pm.f90:374-422 runs after the fine phase).  The coarse
-// acceleration at fine-cell centres goes into the fine-force buffers
+// After the fine kicks: apply the fine impulses that accumulators hold, then
+// gather and apply the coarse ones (pm.f90:374-422 runs after the fine phase).
+// The coarse acceleration at fine-cell centres goes into the fine-force buffers
 // Ff[d] (row pitch pf[d]), which the fine phase no longer needs.
 int fl_gravity_finish(cube_handle* h, void* const Ff[3], const int64_t pf[3], float a_mid, float dt) {
   NuState& s = h->nu;
