@@ -21,9 +21,15 @@ def test_generator_meshes_are_counted(nc, np_nc):
     assert meshes + meshes // 16 <= got <= 1.07 * meshes + 16 * ng  # a sixteenth for the allocator's rounding
 
 
+def free_memory(lib):
+    """Free device memory as the library's own HIP runtime reports it."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
 @pytest.mark.gpu
 def test_generator_allocates_what_is_counted():
-    import torch
     from cube_nufluid_amd.driver import Cube
     from cube_nufluid_amd.ic import power_table, velocity_factor
     from cube_nufluid_amd.params import BoxConfig
@@ -37,13 +43,12 @@ def test_generator_allocates_what_is_counted():
     stop, least = threading.Event(), []
 
     def watch():
-        low = torch.cuda.mem_get_info()[0]
+        low = free
         while not stop.is_set():
-            low = min(low, torch.cuda.mem_get_info()[0])
+            low = min(low, free_memory(cube.lib))
         least.append(low)
 
-    torch.cuda.synchronize()
-    free = torch.cuda.mem_get_info()[0]
+    free = free_memory(cube.lib)
     t = threading.Thread(target=watch)
     t.start()
     try:

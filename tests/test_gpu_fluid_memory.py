@@ -4,21 +4,19 @@ themselves."""
 import pytest
 
 from cube_nufluid_amd.params import BoxConfig
+from test_footprint import free_memory
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("nc", [64, 128])
 def test_gpu_fluid_allocations(nc):
-    import torch
     from cube_nufluid_amd.driver import Cube
     cfg = BoxConfig(nc=nc, nnt=1, ncb=6, box=100.0, np_nc=1)
     cube = Cube.from_ic(cfg, 3, 10.0)
     try:
-        torch.cuda.synchronize()
-        free = torch.cuda.mem_get_info()[0]
+        free = free_memory(cube.lib)
         cube.nu_init(m_ev=0.1, f_neu=0.0075, z_i_nu=10.0)
-        torch.cuda.synchronize()
-        used = free - torch.cuda.mem_get_info()[0]
+        used = free - free_memory(cube.lib)
         cells = [cube.nu_info(n)["nc"] ** 3 for n in range(3)]
         need = 20 * sum(cells) + 32 * cells[2]
         print("nc", nc, "taken", used, "fields and accumulators", need, flush=True)
