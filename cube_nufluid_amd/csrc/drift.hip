@@ -36,9 +36,9 @@ __device__ __forceinline__ uint16_t pack_disp(int dx, int dy, int dz) {
 }
 
 #define DP_SL 2
-// Both per-particle passes take DR_CH source cells a workgroup: 256, or fewer
-// where that leaves CUs idle (drift_cells: at 16^3 cells 16 workgroups of 256
-// took 37 us, 128 of 32 take 17).
+// Both per-particle passes take DR_CH source cells a workgroup: 256, or 32
+// where that leaves CUs idle (up to 32^3 cells, drift_launch: at 16^3 cells 16
+// workgroups of 256 took 37 us, 128 of 32 take 17).
 template <int DR_CH>
 __global__ __launch_bounds__(DR_NT) void k_drift_pass1(Geo g, const void* __restrict__ xp, const void* __restrict__ vp,
                                                        const int64_t* __restrict__ cstart, int64_t n3c,

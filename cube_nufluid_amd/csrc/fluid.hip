@@ -256,8 +256,7 @@ __global__ __launch_bounds__(FL_NT) void k_fl_dt(const float* __restrict__ F, in
 struct FlSet {  // the three fluids of the dispersive sum
   const float* rho[3];
   int nc[3];
-  float dx[3], w[3];
-  int n;
+  float w[3];
 };
 // hg_density (CIC) of the fluid of DX fine cells per cell at the centres of
 // fine cells 4a..4a+3 of row (y, z): the cells' x taps start 0, (j 's share)
@@ -513,7 +512,6 @@ __global__ __launch_bounds__(FG_NT) void k_fl_grav_sep(const T* __restrict__ A0,
   for (int j = 0; j < SPAN; j++) w[j] = j < DX ? ((double)j + 0.5) / DX : 2.0 - ((double)j + 0.5) / DX;
   const int cell = threadIdx.x % (TXY * TXY), kw = threadIdx.x / (TXY * TXY);
   const int tx = cell % TXY, ty = cell / TXY;
-  const bool owner = threadIdx.x < 256;
   double cur[5] = {0, 0, 0, 0, 0}, prev[5] = {0, 0, 0, 0, 0};
   const int64_t n3 = (int64_t)nc * nc * nc;
   for (int pz = 0; pz < (CZ + 1) * DX; pz++) {
@@ -568,50 +566,48 @@ __global__ __launch_bounds__(FG_NT) void k_fl_grav_sep(const T* __restrict__ A0,
       X[4][e] = s2;
     }
     __syncthreads();
-    if (owner) {
-      // plane pz is position j of cell l = pz / DX's window and j + DX of
-      // cell l - 1's
-      const int j = pz % DX, l = pz / DX;
-      const double wa = ((double)j + 0.5) * (1.0 / DX), wb = 2.0 - ((double)(j + DX) + 0.5) * (1.0 / DX);  // w[j], w[j + DX]
-      // sum k of this thread's cell: all five, or k = kw (and 4 beside 3)
-      auto fold = [&](int k) {
-        double y = 0;
+    // plane pz is position j of cell l = pz / DX's window and j + DX of
+    // cell l - 1's
+    const int j = pz % DX, l = pz / DX;
+    const double wa = ((double)j + 0.5) * (1.0 / DX), wb = 2.0 - ((double)(j + DX) + 0.5) * (1.0 / DX);  // w[j], w[j + DX]
+    // sum k of this thread's cell: all five, or k = kw (and 4 beside 3)
+    auto fold = [&](int k) {
+      double y = 0;
 #pragma unroll
-        for (int jy = 0; jy < SPAN; jy++) y += (k == 4 ? w[jy] * w[jy] : w[jy]) * X[k][(ty * DX + jy) * TXY + tx];
-        return y;
-      };
-      if (KW == 1) {
+      for (int jy = 0; jy < SPAN; jy++) y += (k == 4 ? w[jy] * w[jy] : w[jy]) * X[k][(ty * DX + jy) * TXY + tx];
+      return y;
+    };
+    if (KW == 1) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const double y = fold(k);
-          cur[k] += wa * y;
-          prev[k] += wb * y;
-        }
-      } else {
-        const double y = fold(kw);
-        cur[0] += wa * y;
-        prev[0] += wb * y;
+      for (int k = 0; k < 4; k++) {
+        const double y = fold(k);
+        cur[k] += wa * y;
+        prev[k] += wb * y;
       }
-      if (KW == 1 || kw == 3) {
-        const double y = fold(4);
-        cur[4] += wa * wa * y;
-        prev[4] += wb * wb * y;
+    } else {
+      const double y = fold(kw);
+      cur[0] += wa * y;
+      prev[0] += wb * y;
+    }
+    if (KW == 1 || kw == 3) {
+      const double y = fold(4);
+      cur[4] += wa * wa * y;
+      prev[4] += wb * wb * y;
+    }
+    if (j == DX - 1) {
+      if (l >= 1) {
+        const int64_t i = ((int64_t)(c0z + l - 1) * nc + (c0y + ty)) * nc + (c0x + tx);
+        if (KW == 1) {
+          const double J[3] = {prev[0], prev[1], prev[2]};
+          fl_impulse(F, n3, i, J, prev[3] - prev[4]);
+        } else {
+          acc[kw * n3 + i] += kw == 3 ? prev[0] - prev[4] : prev[0];
+        }
       }
-      if (j == DX - 1) {
-        if (l >= 1) {
-          const int64_t i = ((int64_t)(c0z + l - 1) * nc + (c0y + ty)) * nc + (c0x + tx);
-          if (KW == 1) {
-            const double J[3] = {prev[0], prev[1], prev[2]};
-            fl_impulse(F, n3, i, J, prev[3] - prev[4]);
-          } else {
-            acc[kw * n3 + i] += kw == 3 ? prev[0] - prev[4] : prev[0];
-          }
-        }
 #pragma unroll
-        for (int k = 0; k < 5; k++) {
-          prev[k] = cur[k];
-          cur[k] = 0;
-        }
+      for (int k = 0; k < 5; k++) {
+        prev[k] = cur[k];
+        cur[k] = 0;
       }
     }
     __syncthreads();
@@ -864,11 +860,9 @@ extern "C" int cube_fluid_evolve(cube_handle* h, float dt, int dir, float a, flo
 // ---- coupling to the PM step (called from cube_pm)
 static FlSet fl_set(const NuState& s) {
   FlSet f{};
-  f.n = 3;
   for (int n = 0; n < 3; n++) {
     f.rho[n] = s.F[n];
     f.nc[n] = s.nc[n];
-    f.dx[n] = s.dx[n];
     f.w[n] = s.w[n];
   }
   return f;

@@ -24,7 +24,7 @@
 //      processing the tile's peaks one after another;
 //   6. catalogue kernels: halo_info of the physical halos in output order
 //      (:422-506), with the running sums the reference never resets
-//      (inertia, dx_mean, inert) carried by single-thread scans.
+//      (inertia, dx_mean, inert) carried in order by one lane per sum.
 // A particle's tag is a 27-bit mask, one bit per tile holding a copy of it
 // (the tile's displacement -1..1 per axis from the particle's own tile).
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
         for (int64_t i0 = tid; i0 < gcn; i0 += HNT * HGL) {
           long long v[HGL];
 #pragma unroll
-          for (int u = 0; u < HGL; u++) 
+          for (int u = 0; u < HGL; u++)
             v[u] = i0 + u * HNT < gcn ? (long long)__hip_atomic_load(ws.grid + i0 + u * HNT, __ATOMIC_RELAXED,
                                                                      __HIP_MEMORY_SCOPE_AGENT)
                                       : -1;
@@ -635,46 +635,46 @@ __global__ __launch_bounds__(HNT) void k_halo_process(Geo g, HalopCfg c, const v
         }
         __syncthreads();
       } else {
-      for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
-        ws.key[0][m] = __float_as_uint(norm3(ws.x[3 * m] - hf[0], ws.x[3 * m + 1] - hf[1], ws.x[3 * m + 2] - hf[2]));
-        ws.idx[0][m] = (uint32_t)m;
-      }
-      __syncthreads();
-      for (int bitpos = 0; bitpos < 32; bitpos += 2) {
-        // bucket totals; a pass whose digits are all equal keeps the order
-        uint32_t bc[4];
-        {
-          uint64_t c0 = 0, c1 = 0, c2 = 0;
-          for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
-            const uint32_t dgt = (ws.key[cur][m] >> bitpos) & 3u;
-            c0 += dgt == 0; c1 += dgt == 1; c2 += dgt == 2;
-          }
-          uint64_t t0, t1, t2;
-          block_scan_excl(c0, wsum, t0);
-          block_scan_excl(c1, wsum, t1);
-          block_scan_excl(c2, wsum, t2);
-          const uint64_t t3 = n_odc - t0 - t1 - t2;
-          if (t0 == n_odc || t1 == n_odc || t2 == n_odc || t3 == n_odc) continue;
-          bc[0] = 0; bc[1] = (uint32_t)t0; bc[2] = (uint32_t)(t0 + t1); bc[3] = (uint32_t)(t0 + t1 + t2);
-        }
-        uint32_t run[4] = {bc[0], bc[1], bc[2], bc[3]};
-        for (int64_t m0 = 0; m0 < (int64_t)n_odc; m0 += HNT) {
-          const int64_t m = m0 + tid;
-          uint32_t dgt = 4;
-          if (m < (int64_t)n_odc) dgt = (ws.key[cur][m] >> bitpos) & 3u;
-          const uint64_t onehot = dgt < 4 ? 1ull << (16 * dgt) : 0ull;
-          uint64_t tot;
-          const uint64_t pre = block_scan_excl(onehot, wsum, tot);
-          if (dgt < 4) {
-            const uint32_t dst = run[dgt] + (uint32_t)((pre >> (16 * dgt)) & 0xFFFFu);
-            ws.key[cur ^ 1][dst] = ws.key[cur][m];
-            ws.idx[cur ^ 1][dst] = ws.idx[cur][m];
-          }
-          for (int d = 0; d < 4; d++) run[d] += (uint32_t)((tot >> (16 * d)) & 0xFFFFu);
+        for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
+          ws.key[0][m] = __float_as_uint(norm3(ws.x[3 * m] - hf[0], ws.x[3 * m + 1] - hf[1], ws.x[3 * m + 2] - hf[2]));
+          ws.idx[0][m] = (uint32_t)m;
         }
         __syncthreads();
-        cur ^= 1;
-      }
+        for (int bitpos = 0; bitpos < 32; bitpos += 2) {
+          // bucket totals; a pass whose digits are all equal keeps the order
+          uint32_t bc[4];
+          {
+            uint64_t c0 = 0, c1 = 0, c2 = 0;
+            for (int64_t m = tid; m < (int64_t)n_odc; m += HNT) {
+              const uint32_t dgt = (ws.key[cur][m] >> bitpos) & 3u;
+              c0 += dgt == 0; c1 += dgt == 1; c2 += dgt == 2;
+            }
+            uint64_t t0, t1, t2;
+            block_scan_excl(c0, wsum, t0);
+            block_scan_excl(c1, wsum, t1);
+            block_scan_excl(c2, wsum, t2);
+            const uint64_t t3 = n_odc - t0 - t1 - t2;
+            if (t0 == n_odc || t1 == n_odc || t2 == n_odc || t3 == n_odc) continue;
+            bc[0] = 0; bc[1] = (uint32_t)t0; bc[2] = (uint32_t)(t0 + t1); bc[3] = (uint32_t)(t0 + t1 + t2);
+          }
+          uint32_t run[4] = {bc[0], bc[1], bc[2], bc[3]};
+          for (int64_t m0 = 0; m0 < (int64_t)n_odc; m0 += HNT) {
+            const int64_t m = m0 + tid;
+            uint32_t dgt = 4;
+            if (m < (int64_t)n_odc) dgt = (ws.key[cur][m] >> bitpos) & 3u;
+            const uint64_t onehot = dgt < 4 ? 1ull << (16 * dgt) : 0ull;
+            uint64_t tot;
+            const uint64_t pre = block_scan_excl(onehot, wsum, tot);
+            if (dgt < 4) {
+              const uint32_t dst = run[dgt] + (uint32_t)((pre >> (16 * dgt)) & 0xFFFFu);
+              ws.key[cur ^ 1][dst] = ws.key[cur][m];
+              ws.idx[cur ^ 1][dst] = ws.idx[cur][m];
+            }
+            for (int d = 0; d < 4; d++) run[d] += (uint32_t)((tot >> (16 * d)) & 0xFFFFu);
+          }
+          __syncthreads();
+          cur ^= 1;
+        }
       }
       // first ii >= 2 with enclosed density below den_odc
       const float kd = 0.75f / PI_F;
@@ -1070,21 +1070,20 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   const int64_t mcap = std::max<int64_t>(1 << 16, np + (np >> 2));
   // the workspaces come from the fine mesh's idle buffers as far as they fit
   Scratch A(h->fine);
-#define HTRY(call) HIP_TRY(h, call)
 #define HTAKE(T, var, n)                                                                               \
   T* var = A.take<T>(n);                                                                               \
   if (!var) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for " #var " (%lld entries)", (long long)(n))
   HTAKE(uint32_t, ctr, 16);                  // 0 ncand, 1 nvalid, 2 next, 3 errf, 4 walks longer than the table
   HTAKE(unsigned long long, uctr, 4);        // 0 members, 1 grid max, 2 largest search box
   HTAKE(int4, cand, cand_cap);
-  HTRY(hipMemsetAsync(ctr, 0, 16 * sizeof(uint32_t), st));
-  HTRY(hipMemsetAsync(uctr, 0, 4 * sizeof(unsigned long long), st));
+  HIP_TRY(h, hipMemsetAsync(ctr, 0, 16 * sizeof(uint32_t), st));
+  HIP_TRY(h, hipMemsetAsync(uctr, 0, 4 * sizeof(unsigned long long), st));
   // 2. peaks
   k_halo_peaks<<<8192, 256, 0, st>>>(rho, c, ctr + 0, cand_cap, cand);
-  HTRY(hipGetLastError());
+  HIP_TRY(h, hipGetLastError());
   uint32_t hc[5];
-  HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
-  HTRY(hipStreamSynchronize(st));
+  HIP_TRY(h, hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
+  HIP_TRY(h, hipStreamSynchronize(st));
   if ((int64_t)hc[0] > cand_cap)
     return cube_fail(h, CUBE_ERR_CAPACITY, "halo finder: %u candidate peaks exceed the table (%lld)", hc[0], (long long)cand_cap);
   const int64_t ncand = hc[0];
@@ -1113,21 +1112,21 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
         }
       Scratch B(A);
       size_t tb = 0;
-      HTRY(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int)ngen, 0, 41, st));
+      HIP_TRY(h, hipcub::DeviceRadixSort::SortKeys(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int)ngen, 0, 41, st));
       uint64_t* tabk = B.take<uint64_t>(ngen);
       uint64_t* tabs = B.take<uint64_t>(ngen);
       void* tmp = B.take<char>(tb);
       if (!tabk || !tabs || !tmp) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for the offset table");
       k_hoff_gen<<<(unsigned)std::min<int64_t>((ngen + 255) / 256, 4096), 256, 0, st>>>(R, tabk);
-      HTRY(hipcub::DeviceRadixSort::SortKeys(tmp, tb, tabk, tabs, (int)ngen, 0, 41, st));
+      HIP_TRY(h, hipcub::DeviceRadixSort::SortKeys(tmp, tb, tabk, tabs, (int)ngen, 0, 41, st));
       k_halo_walk<<<(unsigned)((ncand + 127) / 128), 128, 0, st>>>(rho, c, cand, ncand, tabs, ntab, R, ctr + 1, vidx, cden,
                                                                     cmesh, chpos, cloop, R < rmax ? ctr + 4 : nullptr);
-      HTRY(hipGetLastError());
-      HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
-      HTRY(hipStreamSynchronize(st));
+      HIP_TRY(h, hipGetLastError());
+      HIP_TRY(h, hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
+      HIP_TRY(h, hipStreamSynchronize(st));
       if (hc[4] == 0) break;
-      HTRY(hipMemsetAsync(ctr + 1, 0, sizeof(uint32_t), st));  // walked again with the whole table
-      HTRY(hipMemsetAsync(ctr + 4, 0, sizeof(uint32_t), st));
+      HIP_TRY(h, hipMemsetAsync(ctr + 1, 0, sizeof(uint32_t), st));  // walked again with the whole table
+      HIP_TRY(h, hipMemsetAsync(ctr + 4, 0, sizeof(uint32_t), st));
     }
   }
   const int64_t npk = hc[1];
@@ -1140,7 +1139,7 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   // 4. order: stable by loop index, then by (tile order, density descending)
   {
     size_t tb = 0;
-    HTRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int32_t*)nullptr,
+    HIP_TRY(h, hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int32_t*)nullptr,
                                             (int32_t*)nullptr, (int)npk, 0, 43, st));
     Scratch B(A);
     int32_t* perm1 = B.take<int32_t>(npk);
@@ -1150,11 +1149,11 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
     if (!perm1 || !k0 || !k1 || !tmp) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for the peak order");
     k_halo_key_lo<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, cloop, k0, perm0);
     size_t tu = tb;
-    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm0, perm1, (int)npk, 0, 32, st));
+    HIP_TRY(h, hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm0, perm1, (int)npk, 0, 32, st));
     const int32_t ntiles = c.nnt * c.nnt * c.nnt;
     k_halo_key_hi<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, perm1, vidx, cand, cden, ntiles, k0);
     tu = tb;
-    HTRY(hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm1, perm0, (int)npk, 0, 43, st));
+    HIP_TRY(h, hipcub::DeviceRadixSort::SortPairs(tmp, tu, k0, k1, perm1, perm0, (int)npk, 0, 43, st));
   }
   // perm0[s] = valid slot of the s-th peak in processing order
   const float gs = std::max(2.0f * (float)(c.ncb - 1) * (float)CUBE_NCELL, 1.0f);
@@ -1175,24 +1174,24 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   HTAKE(int32_t, mq, mcap);
   HTAKE(int32_t, mrk, mcap);
   HTAKE(uint32_t, mbit, mcap);
-  HTRY(hipMemsetAsync(tag, 0, (size_t)np * 4, st));
-  HTRY(hipMemsetAsync(done, 0, sizeof(int32_t) * npk, st));
-  HTRY(hipMemsetAsync(bincnt, 0, sizeof(uint32_t) * (nbins + 1), st));
-  HTRY(hipMemsetAsync(binfill, 0, sizeof(uint32_t) * (nbins + 1), st));
+  HIP_TRY(h, hipMemsetAsync(tag, 0, (size_t)np * 4, st));
+  HIP_TRY(h, hipMemsetAsync(done, 0, sizeof(int32_t) * npk, st));
+  HIP_TRY(h, hipMemsetAsync(bincnt, 0, sizeof(uint32_t) * (nbins + 1), st));
+  HIP_TRY(h, hipMemsetAsync(binfill, 0, sizeof(uint32_t) * (nbins + 1), st));
   k_halo_prep<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, perm0, vidx, cand, cmesh, chpos, c, gs, nbin, pk, bincnt,
                                                              ctr + 3, uctr + 1);
-  HTRY(hipGetLastError());
+  HIP_TRY(h, hipGetLastError());
   {
     const int r2 = scan_counts(h, (const int32_t*)bincnt, nbins, binoff);
     if (r2) return r2;
   }
   k_halo_bin_fill<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, pk, binoff, binfill, binlist);
   k_halo_box_count<<<(unsigned)((npk + HNT / 64 - 1) / (HNT / 64)), HNT, 0, st>>>(g, c, npk, pk, h->cstart, uctr + 2);
-  HTRY(hipGetLastError());
+  HIP_TRY(h, hipGetLastError());
   unsigned long long um[2] = {0, 0};  // largest refined grid, largest search box
-  HTRY(hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
-  HTRY(hipMemcpyAsync(um, uctr + 1, sizeof(um), hipMemcpyDeviceToHost, st));
-  HTRY(hipStreamSynchronize(st));
+  HIP_TRY(h, hipMemcpyAsync(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st));
+  HIP_TRY(h, hipMemcpyAsync(um, uctr + 1, sizeof(um), hipMemcpyDeviceToHost, st));
+  HIP_TRY(h, hipStreamSynchronize(st));
   if (hc[3] & 1u) return cube_fail(h, CUBE_ERR_CHECK, "halo search box beyond the tile buffer (halofind.f90:245-252)");
   if (hc[3] & 2u) return cube_fail(h, CUBE_ERR_CHECK, "newbox>newbox_max (halofind.f90:259)");
   if (hc[3] & 4u) return cube_fail(h, CUBE_ERR_CAPACITY, "halo search box holds more than %d cells", HMAXCELLS);
@@ -1236,9 +1235,9 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
   k_halo_flags<<<(unsigned)((npk + 255) / 256), 256, 0, st>>>(npk, res, c.min_np, is_halo, wcount);
   if ((rc = scan_counts(h, is_halo, npk, hidx)) || (rc = scan_counts(h, wcount, npk, woff))) return rc;
   int64_t nh = 0, nw = 0;
-  HTRY(hipMemcpyAsync(&nh, hidx + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HTRY(hipMemcpyAsync(&nw, woff + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HTRY(hipStreamSynchronize(st));
+  HIP_TRY(h, hipMemcpyAsync(&nh, hidx + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  HIP_TRY(h, hipMemcpyAsync(&nw, woff + npk, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  HIP_TRY(h, hipStreamSynchronize(st));
   if (nh > out->max_halos || nw > out->max_pid_words)
     return cube_fail(h, CUBE_ERR_CAPACITY, "halo catalogue: %lld halos / %lld pid words exceed the buffers", (long long)nh,
                      (long long)nw);
@@ -1254,7 +1253,7 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
     if (out->hid && out->nhid > 0) {
       hidd = A.take<int16_t>(out->nhid);
       if (!hidd) return cube_fail(h, CUBE_ERR_HIP, "halo finder: no memory for hid");
-      HTRY(hipMemsetAsync(hidd, 0, sizeof(int16_t) * out->nhid, st));
+      HIP_TRY(h, hipMemsetAsync(hidd, 0, sizeof(int16_t) * out->nhid, st));
     }
     const unsigned nb1 = (unsigned)std::min<int64_t>(npk, 65535);
     k_halo_cat1<<<nb1, HNT, 0, st>>>(g, c, npk, pk, res, is_halo, hidx, woff, mq, mrk, mbit, h->xp, h->vp, h->vfield, vdt,
@@ -1263,15 +1262,14 @@ extern "C" int cube_halofind(cube_handle* h, const cube_halo_params* hp, cube_ha
     k_halo_seq1<<<1, HNT, 0, st>>>(nh, sums, c.N, rec, qmean);
     k_halo_cat2<<<nb1, HNT, 0, st>>>(c, npk, res, is_halo, hidx, mq, h->pid, qmean, iq);
     k_halo_seq2<<<1, HNT, 0, st>>>(nh, iq, rec);
-    HTRY(hipGetLastError());
-    HTRY(hipMemcpyAsync(out->halos, rec, sizeof(float) * 42 * nh, hipMemcpyDeviceToHost, st));
-    HTRY(hipMemcpyAsync(out->pid_words, words, sizeof(int32_t) * nw, hipMemcpyDeviceToHost, st));
-    if (hidd) HTRY(hipMemcpyAsync(out->hid, hidd, sizeof(int16_t) * out->nhid, hipMemcpyDeviceToHost, st));
-    HTRY(hipStreamSynchronize(st));
+    HIP_TRY(h, hipGetLastError());
+    HIP_TRY(h, hipMemcpyAsync(out->halos, rec, sizeof(float) * 42 * nh, hipMemcpyDeviceToHost, st));
+    HIP_TRY(h, hipMemcpyAsync(out->pid_words, words, sizeof(int32_t) * nw, hipMemcpyDeviceToHost, st));
+    if (hidd) HIP_TRY(h, hipMemcpyAsync(out->hid, hidd, sizeof(int16_t) * out->nhid, hipMemcpyDeviceToHost, st));
+    HIP_TRY(h, hipStreamSynchronize(st));
   } else if (out->hid && out->nhid > 0) {
     memset(out->hid, 0, sizeof(int16_t) * out->nhid);
   }
   return 0;
-#undef HTRY
 #undef HTAKE
 }

@@ -127,7 +127,7 @@ __global__ void k_pk_zero(double* p, int n) {
 
 // Shared body of both entry points: argument checks, CIC density, R2C,
 // binning into `bins` (3 doubles per bin 0..nbin, cleared here by a fill
-// kernel), and the strided copies of bins 1..nbin into the caller's arrays.
+// kernel), and bins 1..nbin into the caller's arrays.
 static int pk_run(cube_handle* h, int nbin, double* modes, double* ksum, double* d2sum, double* bins) {
   const int64_t N = h->fine.N;
   const int want = (int)lrint((double)(N / 2) * sqrt(3.0));
