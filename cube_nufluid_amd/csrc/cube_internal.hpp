@@ -30,7 +30,9 @@ __host__ __device__ inline cpx<T> cmul(cpx<T> a, cpx<T> b) {
 // Three-component z convolution with N, N+1, N+2, N+4, N+8 lines a plane:
 // 0.935, 0.824, 0.807, 0.946, 0.812 ms at 512^3, 8.78, 7.46, 7.13, 7.43,
 // 8.28 ms at 1024^3, 80.1, 69.7, 70.5, 72.1, 69.6 ms at 2048^3; the y and x
-// passes move by less than 8 % either way.  At 2048^3 the z pass's HBM traffic
+// passes move by less than 8 % either way (with N+2 at 2048^3 the three y
+// inversions 52.0 -> 54.4 ms, y forward 17.4 -> 18.1, R2C 17.3 -> 17.9, against
+// 10 ms won in z).  At 2048^3 the z pass's HBM traffic
 // falls from 210 to 166 GB, against 150 it cannot do without.
 __host__ __device__ constexpr int64_t t_pitch(int64_t N) { return N + 2; }
 

@@ -98,9 +98,12 @@ __device__ __forceinline__ void fl_side(const float b[5], float y, float g, floa
 // lines, then their interface fluxes; rows are `pitch` apart, 64/W banks from
 // a whole number of rows for the strided sweeps, whose lanes run over the
 // lines first.
-//   Bound by VALU issue: 30 divisions of some 14 issue slots each per cell
-// were over half of it.  256^3 cells take 0.24, 0.26 and 0.33 ms along x, y and
-// z; with a division each and strips of 4 lines 0.32, 0.36 and 0.48.
+//   Bound by VALU issue (1.09, 0.97 and 0.78 instructions per SIMD and four
+// cycles along x, y and z at 256^3 cells; at 512^3, with strips of 4 lines, 1.15,
+// 0.72 and 0.59, where 16-byte pieces of rows wait for memory): 30 divisions of
+// some 14 issue slots each per cell were over half of it.  256^3 cells take
+// 0.24, 0.27 and 0.33 ms; with a division each and strips of 4 lines 0.32, 0.36
+// and 0.48.
 template <int AX, int W>
 __global__ __launch_bounds__(FL_SNT) void k_fl_sweep(float* F, int nc, int lnc, int pitch, float g, float yg, float dt, float ydx) {
   extern __shared__ float sm[];

@@ -529,10 +529,12 @@ struct PFcfg<4> { static constexpr int NT = 512, K = 4, CAP = 2048, OWN = 4096; 
 template <>
 struct PFcfg<2> { static constexpr int NT = 128, K = 4, CAP = 1024, OWN = 2048; };
 
-// One workgroup per PB^3 coarse cells.  The kernel is bound by VALU issue
-// (98% of the SIMDs' issue slots at 1024^3 particles), so it is written for
-// instruction count; the reach PR and the code width ZX are template
-// parameters.
+// One workgroup per PB^3 coarse cells.  VALU issue is what it runs into first
+// (0.88 instructions per SIMD and four cycles at 1024^3 particles, where 1 is
+// one full-rate instruction after another; 4.9 wavefronts a SIMD, which wait
+// for LDS and memory 60% of their time), so it is written for instruction
+// count, 2780 a wavefront instead of 3499; the reach PR and the code width ZX
+// are template parameters.
 //   1. region particles are binned by window fine cell in LDS (16-bit counts,
 //      scanned two to a word); a particle's region cell comes from a byte
 //      table filled by a max-scan of the cells' first particles, whose cost
