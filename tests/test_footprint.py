@@ -21,6 +21,25 @@ def test_generator_meshes_are_counted(nc, np_nc):
     assert meshes + meshes // 16 <= got <= 1.07 * meshes + 16 * ng  # a sixteenth for the allocator's rounding
 
 
+@pytest.mark.parametrize("nc,izipx,precision,per_cell,most", [
+    (16, 2, 4, 8, (78817541, 79114021)), (16, 1, 8, 1, (84444014, 84740494)),
+    (32, 2, 4, 8, (131452873, 133751817)), (32, 1, 8, 1, (168739381, 171038325)),
+    (64, 2, 4, 8, (529871057, 547977553)), (64, 1, 8, 1, (796102213, 814208709)),
+    (128, 2, 4, 8, (3623690798, 3767415598)), (256, 1, 8, 1, (43497518422, 44642834262)),
+    (512, 2, 4, 8, (221405811458, 230550460162)), (512, 1, 8, 1, (343412781114, 352557429818))])
+def test_no_box_asks_for_more_than_before(nc, izipx, precision, per_cell, most):
+    """`most`: the footprints without and with the generator before the fine
+    mesh's spectrum planes were padded.  A memory budget that a caller set by
+    them still admits the box."""
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    lib.cube_footprint.restype, lib.cube_footprint.argtypes = _lib.SIGNATURES["cube_footprint"]
+    p = _lib.CubeParams()
+    p.nc, p.nnt, p.ncb, p.izipx, p.izipv, p.np_max, p.precision = nc, 2, 6, izipx, 2, per_cell * nc ** 3, precision
+    for ic, m in zip((0, 2), most):
+        got = lib.cube_footprint(ctypes.byref(p), ic)
+        assert 0.98 * m < got <= m
+
+
 def free_memory(lib):
     """Free device memory as the library's own HIP runtime reports it."""
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
